@@ -1192,100 +1192,172 @@ static void laswp(T *A, long lda, long c0, long c1, long k1, long k2, const int 
   hipLaunchKernelGGL(k_laswp<T>, dim3((unsigned)((c1 - c0 + 255) / 256)), dim3(256), 0, s, A, lda, c0, c1, k1, k2, ipiv);
 }
 
-// B[w x ncol] <- L^{-1} B for the unit-lower w x w block of the panel
-// (w <= PW): L and a 128-column tile of B staged in LDS with coalesced
-// loads; each thread then carries one column in registers
-template <typename T> struct TsmCols;
-template <> struct TsmCols<double2> { static const int v = 64; };
-template <> struct TsmCols<float2> { static const int v = 128; };
-template <> struct TsmCols<double> { static const int v = 128; };
-
-template <typename T>
-__global__ void __launch_bounds__(TsmCols<T>::v)
-k_trsm_small(const T *A, long lda, long r0, int w, T *B, long ldb, long ncol)
+// lane k's value in every lane (k wave-uniform)
+__device__ inline float readlane_f(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }
+__device__ inline double readlane_f(double v, int k)
 {
-  constexpr int TSC = TsmCols<T>::v;
-  __shared__ T L[PW][PW + 1];
-  __shared__ T Bt[PW][TSC + 1];
-  const int t = threadIdx.x;
-  const long c0 = (long)blockIdx.x * TSC;
-  {
-    // L and the B tile staged through registers in batches of 8 loads
-    constexpr int NL = PW * PW / TSC;
-    const bool full = (w == PW && c0 + TSC <= ncol);
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)(b & 0xFFFFFFFF), k), hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+__device__ inline double readlane_t(double v, int k) { return readlane_f(v, k); }
+template <typename T> __device__ inline T readlane_t(T v, int k)
+{
+  T r;
+  r.x = readlane_f(v.x, k);
+  r.y = readlane_f(v.y, k);
+  return r;
+}
+
+// r - l x with fused multiply-adds
+__device__ inline double fnma_t(double r, double l, double x) { return fma(-l, x, r); }
+__device__ inline double2 fnma_t(double2 r, double2 l, double2 x)
+{
+  return make_double2(fma(-l.x, x.x, fma(l.y, x.y, r.x)), fma(-l.x, x.y, fma(-l.y, x.x, r.y)));
+}
+__device__ inline float2 fnma_t(float2 r, float2 l, float2 x)
+{
+  return make_float2(fmaf(-l.x, x.x, fmaf(l.y, x.y, r.x)), fmaf(-l.x, x.y, fmaf(-l.y, x.x, r.y)));
+}
+
+// One panel's interchanges on the columns [c0, c1) outside the panel
+// [s0, s1) and, on the columns right of the panel, the substitution with the
+// panel block's unit-lower triangle on its w rows from r0, in one launch:
+// one wave per column.  Lane e holds plan entry e (dst <- src, all sources
+// read before any write); entries 0..w-1 are the rows r0 .. r0 + w - 1, so
+// after the interchange lanes 0..w-1 hold the panel rows of the column and
+// step q passes x_q by lane reads.  Bound: the chain of w - 1 steps (about
+// 1 us); a wave per column leaves the other columns' chains to hide it.  A
+// launch of the interchanges and one of a substitution with a column per
+// thread (L and B through LDS, one wave per 64 columns) took 8 + 54 us per
+// complex128 panel at order 3840; this one takes 11 us.
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_swap_trsm(T *A, long lda, long c0, long c1, long s0, long s1, const int *plan, int w, long r0)
+{
+  const int lane = threadIdx.x & 63;
+  const long ci = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
+  const long nleft = s0 - c0;
+  if (ci >= (c1 - c0) - (s1 - s0)) return;
+  const long c = ci < nleft ? c0 + ci : s1 + (ci - nleft);
+  const int cnt = plan[PW * 4];
+  T v = zero_v<T>();
+  long dst = -1;
+  if (lane < cnt) {
+    dst = plan[lane];
+    v = A[plan[PW * 2 + lane] + c * lda];
+  }
+  if (c >= s1) {
+    // this lane's row of L11 (a clamped row and column elsewhere), all
+    // loads in flight before the substitution
+    T lr[PW];
+    const T *Lr = A + (r0 + (lane < w ? lane : 0)) + r0 * lda;
 #pragma unroll
-    for (int u0 = 0; u0 < NL; u0 += 8) {
-      T lv[8];
+    for (int k = 0; k < PW; k++) lr[k] = Lr[(k < w ? k : 0) * lda];
 #pragma unroll
-      for (int u = 0; u < 8; u++) {
-        int e = t + (u0 + u) * TSC, r = e % PW, q = e / PW;
-        if (full || (r < w && q < w)) lv[u] = A[(r0 + r) + (r0 + q) * lda];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        int e = t + (u0 + u) * TSC, r = e % PW, q = e / PW;
-        if (full || (r < w && q < w)) L[r][q] = lv[u];
-      }
-    }
-#pragma unroll
-    for (int u0 = 0; u0 < PW; u0 += 8) {
-      T bv[8];
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        int e = t + (u0 + u) * TSC, r = e % PW, cc = e / PW;
-        if (full || (r < w && c0 + cc < ncol)) bv[u] = B[r + (c0 + cc) * ldb];
-      }
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        int e = t + (u0 + u) * TSC, r = e % PW, cc = e / PW;
-        if (full || (r < w && c0 + cc < ncol)) Bt[r][cc] = bv[u];
+    for (int k = 0; k < PW; k++) {
+      if (k < w) {
+        const T x = readlane_t(v, k);
+        if (lane > k && lane < w) v = csub(v, cmul(lr[k], x));
       }
     }
   }
-  __syncthreads();
-  T x[PW];
-#pragma unroll
-  for (int r = 0; r < PW; r++) if (r < w) x[r] = Bt[r][t];
-#pragma unroll
-  for (int q = 0; q < PW; q++) {
-    if (q < w) {
-#pragma unroll
-      for (int r = q + 1; r < PW; r++)
-        if (r < w) x[r] = csub(x[r], cmul(L[r][q], x[q]));
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < PW; r++) if (r < w) Bt[r][t] = x[r];
-  __syncthreads();
-  for (int e = t; e < PW * TSC; e += TSC) {
-    int r = e % PW, cc = e / PW;
-    if (r < w && c0 + cc < ncol) B[r + (c0 + cc) * ldb] = Bt[r][cc];
-  }
+  if (lane < cnt) A[dst + c * lda] = v;
 }
 
 template <typename T>
-static void trsm_small(const T *A, long lda, long r0, int w, T *B, long ldb, long ncol, hipStream_t s)
+static void swap_trsm(T *A, long lda, long c0, long c1, long s0, long s1, const int *plan, int w, long r0, hipStream_t s)
 {
-  if (ncol <= 0 || w <= 0) return;
-  int tok = prof_begin(s, std::is_same<T, double2>::value ? PK_TRSM_C128 : PK_TRSM_C64);
-  constexpr int TSC = TsmCols<T>::v;
-  hipLaunchKernelGGL(k_trsm_small<T>, dim3((unsigned)((ncol + TSC - 1) / TSC)), dim3(TSC), 0, s, A, lda, r0, w, B, ldb, ncol);
-  prof_end(s, tok, 4.0 * (double)w * (double)w * (double)ncol);
+  const long ncol = (c1 - c0) - (s1 - s0);
+  if (ncol <= 0) return;
+  int tok = prof_begin(s, std::is_same<T, float2>::value ? PK_TRSM_C64 : PK_TRSM_C128);
+  hipLaunchKernelGGL(k_swap_trsm<T>, dim3((unsigned)((ncol + 3) / 4)), dim3(256), 0, s, A, lda, c0, c1, s0, s1, plan, w,
+                     r0);
+  prof_end(s, tok, 4.0 * (double)w * (double)w * (double)(c1 - s1));
 }
 
-// B[nb x ncol] <- L^{-1} B with the nb x nb unit-lower block at A(r0,r0),
-// by PW-row steps: substitution on the diagonal step (trsm_small) and a
-// GEMM update of the rows below it, as a blocked LAPACK trsm does
+// B[jb x ncol] <- L^-1 B for the unit-lower jb x jb diagonal block at
+// A(r0, r0), jb <= 256, in one launch: NC columns per workgroup, thread t
+// holds row t of each.  Per 32-row panel the wave that holds its rows
+// substitutes by lane reads and passes the 32 values of every column
+// through LDS; the rows below subtract L(row, panel) x, each thread's 32
+// values of L loaded before the barrier (they do not depend on x) and used
+// for all NC columns.  NC = 1 where columns are few (the next block's 256:
+// latency counts), 4 where they fill the GPU (a quarter of the reads of L:
+// 0.5 MB per workgroup in complex128).
+template <typename T, int NC>
+__global__ void __launch_bounds__(256)
+k_trsm_sub(const T *A, long lda, long r0, int jb, T *B, long ldb, long ncol)
+{
+  __shared__ T xs[2][NC][PW];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, row = threadIdx.x;
+  const long c0 = (long)blockIdx.x * NC;
+  T b[NC];
+#pragma unroll
+  for (int u = 0; u < NC; u++) {
+    b[u] = zero_v<T>();
+    if (row < jb && c0 + u < ncol) b[u] = B[row + (c0 + u) * ldb];
+  }
+  for (int i = 0; i * PW < jb; i++) {
+    const int i0 = PW * i, w = min(PW, jb - i0), si = i / 2, l0 = PW * (i & 1);
+    const bool below = row >= i0 + w && row < jb;
+    const T *Lr = A + (r0 + (row < jb ? row : 0)) + (r0 + i0) * lda;
+    T lv[PW];
+    if (wv >= si) {
+      // (the panel's own rows: their row of the triangle; rows below:
+      // their row of L; clamped columns past w are not used)
+#pragma unroll
+      for (int k = 0; k < PW; k++) lv[k] = Lr[(k < w ? k : 0) * lda];
+    }
+    if (wv == si) {
+      const bool mine = lane >= l0 && lane < l0 + w;
+#pragma unroll
+      for (int k = 0; k < PW; k++) {
+        if (k < w) {
+#pragma unroll
+          for (int u = 0; u < NC; u++) {
+            const T x = readlane_t(b[u], l0 + k);
+            if (mine && lane - l0 > k) b[u] = csub(b[u], cmul(lv[k], x));
+          }
+        }
+      }
+      if (mine) {
+#pragma unroll
+        for (int u = 0; u < NC; u++) xs[i & 1][u][lane - l0] = b[u];
+      }
+    }
+    __syncthreads();
+    if (below) {
+      // (the product summed from zero and subtracted once, as the GEMM
+      // update does: subtracting term by term rounds against b 32 times)
+      T d[NC];
+#pragma unroll
+      for (int u = 0; u < NC; u++) d[u] = zero_v<T>();
+#pragma unroll
+      for (int k = 0; k < PW; k++)
+        if (k < w) {
+#pragma unroll
+          for (int u = 0; u < NC; u++) d[u] = fnma_t(d[u], lv[k], xs[i & 1][u][k]);
+        }
+#pragma unroll
+      for (int u = 0; u < NC; u++) b[u] = cadd(b[u], d[u]);
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NC; u++)
+    if (row < jb && c0 + u < ncol) B[row + (c0 + u) * ldb] = b[u];
+}
+
 template <typename T>
 static void trsm_block(const T *A, long lda, long r0, int nb, T *B, long ldb, long ncol, hipStream_t s)
 {
-  for (int i0 = 0; i0 < nb; i0 += PW) {
-    int w = std::min(PW, nb - i0);
-    trsm_small(A, lda, r0 + i0, w, B + i0, ldb, ncol, s);
-    if (i0 + w < nb)
-      gemm_sub((long)(nb - i0 - w), ncol, (long)w, A + (r0 + i0 + w) + (r0 + i0) * lda, lda, B + i0, ldb,
-               B + i0 + w, ldb, s);
-  }
+  if (ncol <= 0 || nb <= 0) return;
+  int tok = prof_begin(s, std::is_same<T, float2>::value ? PK_TRSM_C64 : PK_TRSM_C128);
+  if (ncol <= 512)
+    hipLaunchKernelGGL((k_trsm_sub<T, 1>), dim3((unsigned)ncol), dim3(256), 0, s, A, lda, r0, nb, B, ldb, ncol);
+  else
+    hipLaunchKernelGGL((k_trsm_sub<T, 4>), dim3((unsigned)((ncol + 3) / 4)), dim3(256), 0, s, A, lda, r0, nb, B, ldb, ncol);
+  prof_end(s, tok, 4.0 * (double)nb * (double)nb * (double)ncol);
 }
 
 // B[w x ncol] <- Linv B for a w x w (w <= PW) inverse of a unit-lower
@@ -1360,13 +1432,6 @@ static void trmm_strip(const T *Linv, int w, T *B, long ldb, long ncol, hipStrea
 // Lane e holds plan entry e (dst <- src, all sources read before any
 // write); entries 0..w-1 are the rows r0 .. r0 + w - 1, so after the
 // interchange lanes 0..w-1 hold the panel rows of the column.
-__device__ inline float readlane_f(float v, int k) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), k)); }
-__device__ inline double readlane_f(double v, int k)
-{
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_readlane((int)(b & 0xFFFFFFFF), k), hi = __builtin_amdgcn_readlane((int)(b >> 32), k);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
-}
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_swap_trmm(T *A, long lda, long c0, long c1, long s0, long s1, const int *plan, const T *Linv, int w, long r0,
@@ -1644,16 +1709,16 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
       for (int j = 0; j < w; j++) pflops += (double)(m - j - 1) * (6.0 + 8.0 * (double)(w - j - 1));
       prof_end(stream, tok, pflops);
       if (e != hipSuccess) { rc = -3; break; }
-      // this panel's interchanges on the block's other columns (fast: with
-      // the product by the panel block's inverse on the columns right of it)
+      // this panel's interchanges on the block's other columns, with the
+      // substitution (fast: the product by the panel block's inverse) on the
+      // columns right of it
       long nr = K + jb - (j0 + w);
       if (fast) {
         if constexpr (!IsReal<T>::v)
           swap_trmm(A, lda, K, K + jb, j0, j0 + w, S.plan, (const T *)S.linv + (j0 / PW) * PW * PW, w, j0, stream);
       } else
-        laswp_plans(A, lda, K, K + jb, j0, j0 + w, S.plan, 1, stream);
+        swap_trsm(A, lda, K, K + jb, j0, j0 + w, S.plan, w, j0, stream);
       if (nr > 0) {
-        if (!fast) trsm_small(A, lda, j0, w, A + j0 + (j0 + w) * lda, lda, nr, stream);
         gemm_sub(n - j0 - w, nr, (long)w, A + (j0 + w) + j0 * lda, lda, A + j0 + (j0 + w) * lda, lda,
                  A + (j0 + w) + (j0 + w) * lda, lda, stream, 0, 1, 0, g3m);
       }

@@ -1,0 +1,47 @@
+"""Sizes at which the exact LU's kernels and their dispatch can go wrong:
+edges of panels, of 256-column blocks and of the rule that chooses how many
+columns a workgroup of the block-row substitution takes."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+EPS = {"complex128": 2.0 ** -53, "float64": 2.0 ** -53, "complex64": 2.0 ** -24}
+
+
+def matrix(n, dtype, seed):
+    rng = np.random.default_rng(seed)
+    A = rng.standard_normal((n, n))
+    if dtype != "float64":
+        A = A + 1j * rng.standard_normal((n, n))
+    return A.astype(dtype)
+
+
+def backward_error(A, F, piv):
+    """|P A - L U| / |A| in the Frobenius norm"""
+    n = A.shape[0]
+    wide = np.complex128 if np.iscomplexobj(A) else np.float64
+    L = np.tril(F, -1).astype(wide) + np.eye(n)
+    U = np.triu(F).astype(wide)
+    perm = np.arange(n)
+    for i in range(n):
+        p = piv[i] - 1
+        perm[[i, p]] = perm[[p, i]]
+    assert np.abs(np.tril(F, -1)).max(initial=0.0) <= np.sqrt(2.0) * (1 + 8 * EPS[str(A.dtype)])
+    return np.linalg.norm(A.astype(wide)[perm] - L @ U) / np.linalg.norm(A)
+
+
+# 1024: 512 columns right of the next block (one per workgroup), 1025: 513
+# (four per workgroup, one in the last); 1283: ragged last block and panel
+@pytest.mark.parametrize("dtype", ["complex128", "float64", "complex64"])
+@pytest.mark.parametrize("n", [31, 33, 289, 1024, 1025, 1283])
+def test_block_rows(sx, n, dtype):
+    print(f"block rows n={n} {dtype}", flush=True)
+    A = matrix(n, dtype, 31 * n)
+    M = sx.HMatrix.from_numpy(A, dtype=dtype)
+    assert M.LUFactorize() == 0
+    # |L| |U| of a random matrix under partial pivoting grows like n^(1/2)
+    # to n^(2/3) relative to |A|, and rounding adds up as n^(1/2): 4 n eps
+    # covers both with room (seen: below n eps)
+    berr = backward_error(A, M.numpy(), M.ipiv.cpu().numpy())
+    assert berr <= 4 * max(n, 32) * EPS[dtype], berr
