@@ -2,17 +2,14 @@
 // and the refinement helpers, complex128 and complex64.
 //
 // Right-looking blocked algorithm (outer block nb, inner block 32):
-//  * a 32-column sub-panel is factored column by column by one
-//    cooperative launch: every workgroup owns a slice of rows, finds its
-//    largest |re|+|im| entry, a grid barrier picks the global pivot (first
-//    maximal row, as izamax), the two rows are exchanged through a small
-//    global buffer, and each workgroup scales and rank-1 updates its rows;
-//  * row interchanges are applied to the other columns (laswp),
+//  * a 32-column sub-panel is factored in one launch: row-by-row partial
+//    pivoting (lu_panel.inc), or tournament pivoting (k_panel_ts below) for
+//    the mixed solver's complex64 factors;
+//  * row interchanges are applied to the other columns,
 //  * U12 = L11^{-1} A12 (unit-lower triangular solve),
 //  * A22 -= A21 U12 on the matrix cores: v_mfma_f64_16x16x4f64 for
 //    complex128 and v_mfma_f32_16x16x4f32 for complex64, four real
 //    products per complex product.
-#include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -23,10 +20,9 @@
 #include <vector>
 
 #include "lu.h"
+#include "lu_dev.h"
 #include "prof.h"
 #include "ws.h"
-
-namespace cg = cooperative_groups;
 
 namespace scuffx {
 
@@ -60,78 +56,6 @@ template <> struct CT<float2> {
   __device__ static inline V4 zero() { return V4{0, 0, 0, 0}; }
   __device__ static inline int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
-
-template <typename T> __device__ inline T cmul(T a, T b) { T r; r.x = a.x * b.x - a.y * b.y; r.y = a.x * b.y + a.y * b.x; return r; }
-template <typename T> __device__ inline T csub(T a, T b) { T r; r.x = a.x - b.x; r.y = a.y - b.y; return r; }
-template <typename T> __device__ inline T cadd(T a, T b) { T r; r.x = a.x + b.x; r.y = a.y + b.y; return r; }
-template <typename T> __device__ inline T crecip(T a)
-{
-  // Smith's algorithm for 1/a
-  T r;
-  typedef decltype(a.x) R;
-  if (fabs(a.x) >= fabs(a.y)) { R t = a.y / a.x, d = a.x + a.y * t; r.x = 1 / d; r.y = -t / d; }
-  else { R t = a.x / a.y, d = a.x * t + a.y; r.x = t / d; r.y = -1 / d; }
-  return r;
-}
-// real (double) counterparts, so that the panel and the solves also
-// instantiate for real matrices (LHM_REAL, dgetrf/dgetrs semantics)
-__device__ inline double cmul(double a, double b) { return a * b; }
-__device__ inline double csub(double a, double b) { return a - b; }
-__device__ inline double cadd(double a, double b) { return a + b; }
-__device__ inline double crecip(double a) { return 1.0 / a; }
-__device__ inline double cdiv(double a, double b) { return a / b; }
-// pivot magnitude |re| + |im| (izamax / idamax)
-__device__ inline double mag1(double a) { return fabs(a); }
-template <typename T> __device__ inline auto mag1(T a) -> decltype(a.x) { return fabs(a.x) + fabs(a.y); }
-__device__ inline bool nonzero(double a) { return a != 0; }
-template <typename T> __device__ inline bool nonzero(T a) { return a.x != 0 || a.y != 0; }
-template <typename T> __device__ inline T zero_v() { T r; r.x = 0; r.y = 0; return r; }
-template <> __device__ inline double zero_v<double>() { return 0; }
-template <typename T> __device__ inline T unit_v() { T r; r.x = 1; r.y = 0; return r; }
-template <> __device__ inline double unit_v<double>() { return 1; }
-// acc += a b, real and imaginary parts each as one expression
-template <typename T> __device__ inline void mac(T &acc, T a, T b)
-{
-  acc.x += a.x * b.x - a.y * b.y;
-  acc.y += a.x * b.y + a.y * b.x;
-}
-__device__ inline void mac(double &acc, double a, double b) { acc += a * b; }
-// acc += conj(a) b (conj = identity for real)
-template <typename T> __device__ inline void macc(T &acc, T a, T b, bool cj)
-{
-  if (cj) a.y = -a.y;
-  mac(acc, a, b);
-}
-__device__ inline void macc(double &acc, double a, double b, bool) { acc += a * b; }
-template <typename T> __device__ inline T conj_if(T a, bool cj) { if (cj) a.y = -a.y; return a; }
-__device__ inline double conj_if(double a, bool) { return a; }
-template <typename T> __device__ inline double re_of(T a) { return a.x; }
-template <typename T> __device__ inline double im_of(T a) { return a.y; }
-__device__ inline double re_of(double a) { return a; }
-__device__ inline double im_of(double) { return 0; }
-template <typename T> struct IsReal { static const bool v = false; };
-template <> struct IsReal<double> { static const bool v = true; };
-
-template <typename T> __device__ inline T cdiv(T a, T b)
-{
-  typedef decltype(a.x) R;
-  T r;
-  if (fabs(b.x) >= fabs(b.y)) { R t = b.y / b.x, d = b.x + b.y * t; r.x = (a.x + a.y * t) / d; r.y = (a.y - a.x * t) / d; }
-  else { R t = b.x / b.y, d = b.x * t + b.y; r.x = (a.x * t + a.y) / d; r.y = (a.y * t - a.x) / d; }
-  return r;
-}
-
-// Strides between the instances of a batch of equal-size factorizations:
-// matrix elements (a), pivot entries (p) and bytes of each instance's
-// panel scratch (s).  A single factorization is a batch of one, strides 0;
-// batched kernels take the instance from blockIdx.y or blockIdx.z.
-struct BStride {
-  long a = 0, p = 0, s = 0;
-};
-template <typename P> __device__ inline P *bshift(P *p, long bytes)
-{
-  return p ? (P *)((char *)p + bytes) : p;
-}
 
 // ---------------------------------------------------------------------
 // C[m x n] -= A[m x k] B[k x n]  (ACC)  or  C = A B  (!ACC);
@@ -366,304 +290,38 @@ static bool mixed_gemm_3m()
   return !(e && !strcmp(e, "0"));
 }
 
-// ---------------------------------------------------------------------
-// cooperative panel factorization: rows [r0, r0+m), columns [r0, r0+w),
-// w <= PW.  Workgroup g keeps rows [r0 + g*rows, ...) of the panel in
-// LDS for the whole panel.  Per column one grid barrier: before it every
-// workgroup publishes its best |re|+|im| candidate together with that
-// candidate's row, and the owner of the diagonal row publishes that row;
-// after it every workgroup picks the global pivot (largest, first row on
-// ties, as izamax) and has both rows of the interchange at hand.  The
-// published slots alternate between two buffers so that a workgroup
-// running ahead never overwrites a slot another one still reads.
-// ---------------------------------------------------------------------
-#define PW 32
-
-template <typename T> struct PanelRows;
-template <> struct PanelRows<double2> { static const int n = 128; };
-template <> struct PanelRows<float2> { static const int n = 256; };
-template <> struct PanelRows<double> { static const int n = 256; };
-
-struct PanelScratch {
-  unsigned *bar;   // grid barrier: [0] arrivals, [32] generation, [64] timeout flag (own cache lines)
-  double *candv;   // [2][Gmax]
-  unsigned long long *ckey;   // [2][Gmax]: (local candidate row << 32) | column sequence number
-  void *candrow;   // [2][Gmax][PW] T
-  void *rowc;      // [2][PW] T
-  int *plan;       // [2*PW+1]: dst rows, src rows, count of the panel's net row permutation
-  void *linv;      // [npanels][PW][PW] T or null: inverse of each panel's unit-lower block (column-major)
-  unsigned long long *ts;   // tournament-pivoting sets and root area (k_panel_ts), or null
-  // the same scratch of the instance `bytes` further on (a batch's scratch
-  // areas are equal and contiguous)
-  __device__ inline PanelScratch shift(long bytes) const
-  {
-    PanelScratch o = *this;
-    o.bar = bshift(bar, bytes); o.candv = bshift(candv, bytes); o.ckey = bshift(ckey, bytes);
-    o.candrow = bshift((char *)candrow, bytes); o.rowc = bshift((char *)rowc, bytes);
-    o.plan = bshift(plan, bytes); o.linv = bshift((char *)linv, bytes); o.ts = bshift(ts, bytes);
-    return o;
-  }
-};
-
-
-// Cross-workgroup exchange inside the panel without grid barriers: the
-// shared words are read and written only by agent-scope relaxed atomics
-// (coherent across the XCDs' L2s), and a writer waits for its data
-// stores to complete (s_waitcnt) before it stores the sequence-tagged key
-// that readers poll.  No release/acquire fences, hence no L2 write-back or
-// invalidation while the trailing GEMM runs beside the panel.
-__device__ inline void st_coh(unsigned long long *p, unsigned long long v)
+__global__ void k_fill_u64(unsigned long long *w, unsigned long long v, long n)
 {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline unsigned long long ld_coh(const unsigned long long *p)
-{
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline void st_coh(float2 *p, float2 v)
-{
-  unsigned long long u = ((unsigned long long)__float_as_uint(v.y) << 32) | __float_as_uint(v.x);
-  st_coh((unsigned long long *)p, u);
-}
-__device__ inline float2 ld_coh(const float2 *p)
-{
-  unsigned long long u = ld_coh((const unsigned long long *)p);
-  float2 v;
-  v.x = __uint_as_float((unsigned)u);
-  v.y = __uint_as_float((unsigned)(u >> 32));
-  return v;
-}
-__device__ inline void st_coh(double2 *p, double2 v)
-{
-  st_coh((unsigned long long *)p, (unsigned long long)__double_as_longlong(v.x));
-  st_coh((unsigned long long *)p + 1, (unsigned long long)__double_as_longlong(v.y));
-}
-__device__ inline void st_coh(double *p, double v)
-{
-  st_coh((unsigned long long *)p, (unsigned long long)__double_as_longlong(v));
-}
-__device__ inline double ld_coh(const double *p)
-{
-  return __longlong_as_double((long long)ld_coh((const unsigned long long *)p));
-}
-__device__ inline double2 ld_coh(const double2 *p)
-{
-  double2 v;
-  v.x = __longlong_as_double((long long)ld_coh((const unsigned long long *)p));
-  v.y = __longlong_as_double((long long)ld_coh((const unsigned long long *)p + 1));
-  return v;
-}
-// polls before a wait gives up (about a second); the kernel then
-// finishes and the host reports the time-out
-#define GBAR_SPIN (1u << 20)
-// keys one lane of the polling wave holds: up to 64 * 8 workgroups
-#define KEYS_PER_LANE 8
-
-// every memory operation this thread issued has completed; the signal
-// fences keep the compiler from moving memory operations across it
-__device__ inline void drain()
-{
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
-  __builtin_amdgcn_s_waitcnt(0);
-  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) w[i] = v;
 }
 
+// inverse of a panel's unit-lower w x w block (identity outside it), column
+// t of it by substitution: for the block rows of the mixed solver's
+// factorization with row-by-row pivoting
 template <typename T>
-__global__ void __launch_bounds__(PanelRows<T>::n)
-k_panel(T *A, long lda, long r0, long m, int w, int *ipiv, int *info, PanelScratch S, int Gmax, unsigned seq0)
+__global__ void __launch_bounds__(64) k_unit_inv(const T *A, long lda, long r0, int w, T *linv)
 {
-  typedef typename CT<T>::R R;
-  constexpr int NR = PanelRows<T>::n;
-  constexpr bool kPackKey = std::is_same<T, float2>::value;
-  __shared__ T slab[PW][NR];           // column-major: slab[q][t] = A(lo + t, r0 + q)
-  __shared__ R wv[NR / 64];
-  __shared__ int wi[NR / 64];
-  __shared__ T spiv[PW], sold[PW];
-  __shared__ long spv[PW];
-  __shared__ int s_p;
-  __shared__ R s_bv;
-  __builtin_amdgcn_s_setprio(3);   // critical path beside the trailing GEMM
-  const int t = threadIdx.x, G = gridDim.x, g = blockIdx.x, lane = t & 63, wave = t >> 6;
-  const long lo = r0 + (long)g * NR;
-  const int nrow = (int)std::min<long>(NR, r0 + m - lo);
-  const long i = lo + t;                 // this thread's row
-  T *candrow = (T *)S.candrow, *rowc = (T *)S.rowc;
-  unsigned *err = S.bar + 64;
-  __shared__ int s_gw;
-  if (t < nrow) {
-    T v[PW];
-    if (w == PW) {
-#pragma unroll
-      for (int q = 0; q < PW; q++) v[q] = A[i + (r0 + q) * lda];
-#pragma unroll
-      for (int q = 0; q < PW; q++) slab[q][t] = v[q];
-    } else {
-      for (int q = 0; q < w; q++) slab[q][t] = A[i + (r0 + q) * lda];
-    }
+  __shared__ T L[PW][PW + 1];
+  const int t = threadIdx.x;
+  for (int e = t; e < PW * PW; e += 64) {
+    const int rr = e % PW, q = e / PW;
+    L[rr][q] = (rr < w && q < w) ? A[(r0 + rr) + (r0 + q) * lda] : zero_v<T>();
   }
   __syncthreads();
-  for (int j = 0; j < w; j++) {
-    const long c = r0 + j;
-    const int buf = j & 1;
-    const unsigned seq = seq0 + (unsigned)j;
-    // local candidate: largest |re|+|im| among own rows >= c, first on ties
-    R best = -1; int bi = -1;
-    if (t < nrow && i >= c) { T v = slab[j][t]; best = mag1(v); bi = t; }
-    for (int off = 32; off > 0; off >>= 1) {
-      R ob = __shfl_xor(best, off);
-      int oi = __shfl_xor(bi, off);
-      if (ob > best || (ob == best && oi >= 0 && (bi < 0 || oi < bi))) { best = ob; bi = oi; }
-    }
-    if (lane == 0) { wv[wave] = best; wi[wave] = bi; }
-    __syncthreads();
-    R b0 = wv[0]; int bb = wi[0];
-    for (int q = 1; q < NR / 64; q++)
-      if (wv[q] > b0 || (wv[q] == b0 && wi[q] >= 0 && (bb < 0 || wi[q] < bb))) { b0 = wv[q]; bb = wi[q]; }
-    // publish: candidate row (and row c, by its owner), then value, then key
-    if (t < w) {
-      if (bb >= 0) st_coh(candrow + ((long)buf * Gmax + g) * PW + t, slab[t][bb]);
-      if (c >= lo && c < lo + nrow) st_coh(rowc + buf * PW + t, slab[t][c - lo]);
-    }
-    // complex64: the value travels in the key itself (value bits << 32 |
-    // local row << 23 | 23-bit sequence number, row 511 = no candidate), so
-    // the winner is known from the polled keys alone; complex128 needs all
-    // 64 bits of its value and publishes it beside the key
-    if (!kPackKey && t == 0)
-      st_coh((unsigned long long *)S.candv + buf * Gmax + g, (unsigned long long)__double_as_longlong((double)b0));
-    drain();
-    __syncthreads();
-    if (t == 0) {
-      unsigned long long key;
-      if (kPackKey)
-        key = ((unsigned long long)__float_as_uint((float)b0) << 32) |
-              ((unsigned long long)(bb >= 0 ? bb : 511) << 23) | (seq & 0x7FFFFFu);
-      else
-        key = ((unsigned long long)(unsigned)(bb >= 0 ? bb : -1) << 32) | seq;
-      st_coh(S.ckey + buf * Gmax + g, key);
-    }
-    // global pivot: wave 0 waits for every workgroup's key of this column
-    if (t < 64) {
-      // bounded: past GBAR_SPIN polls the error word is set, and once it
-      // is set no workgroup waits again (the panel then finishes with
-      // meaningless values and the host reports the time-out)
-      // the keys of the last poll stay in registers (G <= 64 * KEYS_PER_LANE)
-      unsigned long long kk[KEYS_PER_LANE];
-      const unsigned smask = kPackKey ? 0x7FFFFFu : 0xFFFFFFFFu;
-      unsigned spins = 0;
-      for (;;) {
-        bool ok = true;
+  if (t >= PW) return;
+  T x[PW];
 #pragma unroll
-        for (int u = 0; u < KEYS_PER_LANE; u++) {
-          const int q = lane + 64 * u;
-          if (q < G) {
-            kk[u] = ld_coh(S.ckey + buf * Gmax + q);
-            if (((unsigned)kk[u] & smask) != (seq & smask)) ok = false;
-          }
-        }
-        if (__ballot(!ok) == 0) break;
-        if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
-        if (++spins > GBAR_SPIN) { __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      __atomic_signal_fence(__ATOMIC_SEQ_CST);
-      R b = -1; long p = -1; int gw = -1;
+  for (int r = 0; r < PW; r++) {
+    T v = (r == t) ? unit_v<T>() : zero_v<T>();
+    if (r < w && t < w) {
 #pragma unroll
-      for (int u = 0; u < KEYS_PER_LANE; u++) {
-        const int q = lane + 64 * u;
-        if (q >= G) continue;
-        const unsigned long long k = kk[u];
-        int li;
-        R v;
-        if (kPackKey) {
-          li = (int)((k >> 23) & 511u);
-          if (li == 511) continue;
-          v = (R)__uint_as_float((unsigned)(k >> 32));
-        } else {
-          li = (int)(unsigned)(k >> 32);
-          if (li < 0) continue;
-          v = (R)__longlong_as_double((long long)ld_coh((const unsigned long long *)S.candv + buf * Gmax + q));
-        }
-        long ii = r0 + (long)q * NR + li;
-        if (v > b || (v == b && ii < p)) { b = v; p = ii; gw = q; }
-      }
-      for (int off = 32; off > 0; off >>= 1) {
-        R ob = __shfl_xor(b, off);
-        long op = __shfl_xor(p, off);
-        int og = __shfl_xor(gw, off);
-        if (op >= 0 && (ob > b || (ob == b && (p < 0 || op < p)))) { b = ob; p = op; gw = og; }
-      }
-      if (t == 0) { s_p = p < 0 ? (int)c : (int)p; s_gw = gw; s_bv = b; }
+      for (int k = 0; k < r; k++) v = csub(v, cmul(L[r][k], x[k]));
     }
-    __syncthreads();
-    const long p = s_p;
-    if (t < w) {
-      sold[t] = ld_coh(rowc + buf * PW + t);
-      spiv[t] = s_gw >= 0 ? ld_coh(candrow + ((long)buf * Gmax + s_gw) * PW + t) : sold[t];
-    }
-    if (t == 0) spv[j] = p;
-    if (g == 0 && t == 0) {
-      ipiv[c] = (int)(p + 1);
-      if (s_bv == 0 && *info == 0) *info = (int)(c + 1);
-    }
-    __syncthreads();
-    if (t < w) {
-      if (c >= lo && c < lo + nrow) slab[t][c - lo] = spiv[t];
-      if (p != c && p >= lo && p < lo + nrow) slab[t][p - lo] = sold[t];
-    }
-    __syncthreads();
-    T piv = spiv[j];
-    const bool nz = nonzero(piv);
-    if (t < nrow && i > c) {
-      T l = slab[j][t];
-      if (nz) { l = cmul(l, crecip(piv)); slab[j][t] = l; }
-      for (int q = j + 1; q < w; q++) slab[q][t] = csub(slab[q][t], cmul(l, spiv[q]));
-    }
-    __syncthreads();
+    x[r] = v;
   }
-  for (int q = 0; q < w; q++)
-    if (t < nrow) A[i + (r0 + q) * lda] = slab[q][t];
-  // the inverse of the panel's unit-lower w x w block (workgroup 0 holds
-  // its rows), column t by substitution, identity outside w x w
-  if (S.linv && g == 0 && t < PW) {
-    T x[PW];
 #pragma unroll
-    for (int r = 0; r < PW; r++) {
-      T v = (r == t) ? unit_v<T>() : zero_v<T>();
-      if (r < w && t < w) {
-#pragma unroll
-        for (int k = 0; k < r; k++) v = csub(v, cmul(slab[k][r], x[k]));
-      }
-      x[r] = v;
-    }
-    T *li = (T *)S.linv + (r0 / PW) * PW * PW + (long)t * PW;
-#pragma unroll
-    for (int r = 0; r < PW; r++) li[r] = x[r];
-  }
-  // net permutation of the panel's w interchanges on the rows they touch,
-  // one row per lane of wave 0: lanes 0..w-1 are rows r0.., pivot rows
-  // from below are appended.  After the interchanges row dst[q] holds
-  // what row src[q] held before.
-  if (g == 0 && t < 64) {
-    long row = (t < w) ? r0 + t : -1;
-    int content = t, cnt = w;
-    for (int j = 0; j < w; j++) {
-      const long pj = spv[j];
-      if (pj == r0 + j) continue;
-      int ip;
-      if (pj < r0 + w) ip = (int)(pj - r0);
-      else {
-        unsigned long long hit = __ballot(row == pj);
-        if (hit) ip = __ffsll(hit) - 1;
-        else { ip = cnt; if (t == cnt) { row = pj; content = cnt; } cnt++; }
-      }
-      int cj = __shfl(content, j), cp = __shfl(content, ip);
-      if (t == j) content = cp;
-      if (t == ip) content = cj;
-    }
-    long srow = __shfl(row, content);
-    if (t < cnt) { S.plan[t] = (int)row; S.plan[PW * 2 + t] = (int)srow; }
-    if (t == 0) S.plan[PW * 4] = cnt;
-  }
+  for (int r = 0; r < PW; r++) linv[(long)t * PW + r] = x[r];
 }
 
 // ---------------------------------------------------------------------
@@ -679,7 +337,7 @@ k_panel(T *A, long lda, long r0, long m, int w, int *ipiv, int *info, PanelScrat
 // Pivot choices differ from row-by-row partial pivoting (the complex128
 // path keeps that); the mixed solver's refinement in complex128 takes the
 // factors as a preconditioner.  Cross-workgroup data moves only through
-// agent-scope relaxed atomics with drain-then-flag, as in k_panel: three
+// agent-scope relaxed atomics, data drained before a flag: three
 // waits per panel (two at most 64 workgroups) instead of one per column.
 // ---------------------------------------------------------------------
 #define TS_FAN 8
@@ -728,20 +386,6 @@ __device__ inline float2 cfms(float2 r, float2 l, float2 c)
   o.x = fmaf(-l.x, c.x, fmaf(l.y, c.y, r.x));
   o.y = fmaf(-l.x, c.y, fmaf(-l.y, c.x, r.y));
   return o;
-}
-
-// maximum of a 32-bit key over the wave, in every lane: within each row
-// of 16 lanes by DPP (quad swaps, half-row and row mirrors), then over the
-// four rows by lane reads (the result is wave-uniform).  All lanes active.
-__device__ inline unsigned wave_max_key(unsigned k)
-{
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp(0, (int)k, 0xB1, 0xF, 0xF, false));    // quad_perm 1,0,3,2
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp(0, (int)k, 0x4E, 0xF, 0xF, false));    // quad_perm 2,3,0,1
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp(0, (int)k, 0x141, 0xF, 0xF, false));   // row_half_mirror
-  k = max(k, (unsigned)__builtin_amdgcn_update_dpp(0, (int)k, 0x140, 0xF, 0xF, false));   // row_mirror
-  const unsigned a = __builtin_amdgcn_readlane(k, 0), b = __builtin_amdgcn_readlane(k, 16);
-  const unsigned c = __builtin_amdgcn_readlane(k, 32), d = __builtin_amdgcn_readlane(k, 48);
-  return max(max(a, b), max(c, d));
 }
 
 // partial-pivoting LU (largest |re|+|im|, lowest row on ties) of the rows
@@ -810,8 +454,8 @@ __device__ inline int ts_count(long g, long span, long m, int w)
   return (int)min((long)w, rows);
 }
 
-// wave 0 waits until the n <= 64 words f[k * stride] hold seq (bounded as
-// in k_panel), then the workgroup synchronizes
+// wave 0 waits until the n <= 64 words f[k * stride] hold seq (bounded),
+// then the workgroup synchronizes
 __device__ void ts_wait(const unsigned long long *f, long stride, int n, unsigned long long seq, unsigned *err)
 {
   if (threadIdx.x < 64) {
@@ -831,7 +475,7 @@ __device__ void ts_wait(const unsigned long long *f, long stride, int n, unsigne
 }
 
 // panel rows [r0, r0 + m) x columns [r0, r0 + w), w <= PW; grid: one
-// workgroup per 256 rows, all co-resident; outputs as k_panel (factors in
+// workgroup per 256 rows, all co-resident; outputs as k_panel_x (factors in
 // place, ipiv, info, the net row permutation in S.plan, the inverse of the
 // unit-lower diagonal block in S.linv)
 // (at most 168 VGPRs, so that a workgroup fits on SIMDs that run three
@@ -1230,7 +874,7 @@ __device__ inline float2 fnma_t(float2 r, float2 l, float2 x)
 // 1 us); a wave per column leaves the other columns' chains to hide it.  A
 // launch of the interchanges and one of a substitution with a column per
 // thread (L and B through LDS, one wave per 64 columns) took 8 + 54 us per
-// complex128 panel at order 3840; this one takes 11 us.
+// complex128 panel at order 3840; this one takes 7 us.
 template <typename T>
 __global__ void __launch_bounds__(256)
 k_swap_trsm(T *A, long lda, long c0, long c1, long s0, long s1, const int *plan, int w, long r0)
@@ -1284,7 +928,9 @@ static void swap_trsm(T *A, long lda, long c0, long c1, long s0, long s1, const 
 // values of L loaded before the barrier (they do not depend on x) and used
 // for all NC columns.  NC = 1 where columns are few (the next block's 256:
 // latency counts), 4 where they fill the GPU (a quarter of the reads of L:
-// 0.5 MB per workgroup in complex128).
+// 0.5 MB per workgroup in complex128).  At order 3840: 40 us for the next
+// block, 150 us beside it for the rest, where 32-row substitutions and
+// updates in 15 launches took 540 us for each.
 template <typename T, int NC>
 __global__ void __launch_bounds__(256)
 k_trsm_sub(const T *A, long lda, long r0, int jb, T *B, long ldb, long ncol)
@@ -1616,7 +1262,7 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   if (nb > 256) nb = 256;
   if (nb % PW) nb = 256;
   const int ib = PW;
-  constexpr int NR = PanelRows<T>::n;
+  constexpr int NR = 256;
   const long Gmax = (n + NR - 1) / NR;
   // the mixed solver's complex64 factorization pivots by tournament
   // (SCUFFX_MIXED_PIVOTING=partial, read at every factorization: row by
@@ -1626,7 +1272,8 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   if (IsReal<T>::v) fast = 0;     // the explicit-inverse block rows are a complex64 option
   const bool tourn = fast && std::is_same<T, float2>::value && !partial_env;
   const bool g3m = tourn && mixed_gemm_3m();
-  const void *panel_fn = tourn ? (const void *)k_panel_ts : (const void *)k_panel<T>;
+  const void *panel_one = panel_x_kernel<T>(true), *panel_two = panel_x_kernel<T>(false);
+  const void *panel_fn = tourn ? (const void *)k_panel_ts : Gmax <= PX_ONE ? panel_one : panel_two;
   int dev = 0, ncu = 0, perCU = 0;
   hipGetDevice(&dev);
   hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -1635,30 +1282,24 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   if ((long)std::max(1, ncu) * std::max(1, perCU) < Gmax + (tourn ? 1 : 0)) return -5;   // not co-resident
   if (Gmax > 64 * KEYS_PER_LANE) return -5;                           // more workgroups than polled keys
   const long npanels = (n + PW - 1) / PW;
-  // panel scratch, carved from one workspace: barrier words (3 cache
-  // lines), info, all panel plans, candidate values / indices / rows,
-  // diagonal rows
+  // panel scratch, carved from one workspace: time-out word (its own cache
+  // lines), info, all panel plans, the panels' inverses, the tournament's or
+  // the exact panel's exchange area
   PanelScratch S;
   size_t off_info = 96 * sizeof(unsigned), off_plan = off_info + 64;
-  size_t off_cv = off_plan + 256 * ((sizeof(int) * PLAN_LEN * npanels + 255) / 256);
-  size_t off_ci = off_cv + 256 * ((sizeof(double) * 2 * Gmax + 255) / 256);
-  size_t off_cr = off_ci + 256 * ((sizeof(unsigned long long) * 2 * Gmax + 255) / 256);
-  size_t off_rc = off_cr + 256 * ((sizeof(T) * 2 * Gmax * PW + 255) / 256);
-  size_t off_li = off_rc + 256 * ((sizeof(T) * 2 * PW + 255) / 256);
+  size_t off_li = off_plan + 256 * ((sizeof(int) * PLAN_LEN * npanels + 255) / 256);
   size_t off_ts = off_li + 256 * (((fast ? sizeof(T) * PW * PW * npanels : 0) + 255) / 256);
   const size_t ts_words = tourn ? (size_t)ts_root_off(ts_levels(Gmax), Gmax) + TS_ROOT : 0;
-  size_t total = off_ts + sizeof(unsigned long long) * ts_words;
+  const size_t x_words = tourn ? 0 : 2 * (size_t)PW * Gmax * PXW<T>::n;
+  size_t total = off_ts + sizeof(unsigned long long) * (ts_words + x_words);
   char *wsb = (char *)ws_get(WS_PANEL, total);
   if (!wsb) return -2;
   S.linv = fast ? (void *)(wsb + off_li) : nullptr;
   S.ts = tourn ? (unsigned long long *)(wsb + off_ts) : nullptr;
+  S.xch = tourn ? nullptr : (unsigned long long *)(wsb + off_ts);
   S.bar = (unsigned *)wsb;
   int *dinfo = (int *)(wsb + off_info);
   int *plans = (int *)(wsb + off_plan);
-  S.candv = (double *)(wsb + off_cv);
-  S.ckey = (unsigned long long *)(wsb + off_ci);
-  S.candrow = (void *)(wsb + off_cr);
-  S.rowc = (void *)(wsb + off_rc);
   // The trailing update runs beside the next panels on a second stream,
   // unless the panel needs more than half of the resident workgroup slots
   // of its kernel: then the GEMM's workgroups, dispatched without pause
@@ -1672,10 +1313,12 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   hipEventCreateWithFlags(&evR, hipEventDisableTiming);
   hipMemsetAsync(dinfo, 0, sizeof(int), stream);
   hipMemsetAsync(S.bar, 0, sizeof(unsigned) * 96, stream);
-  // candidate keys start at sequence 0, which no column uses
-  hipMemsetAsync(S.ckey, 0, sizeof(unsigned long long) * 2 * Gmax, stream);
-  // tournament sets and flags likewise
+  // tournament sets and flags start at sequence 0, which no panel uses; the
+  // exact panel's slots with the sentinel
   if (tourn) hipMemsetAsync(S.ts, 0, sizeof(unsigned long long) * ts_words, stream);
+  else
+    hipLaunchKernelGGL(k_fill_u64, dim3((unsigned)((x_words + 255) / 256)), dim3(256), 0, stream, S.xch,
+                       (unsigned long long)PX_SENT, (long)x_words);
   // the side stream starts after the caller's stream has the matrix ready
   hipEventRecord(evR, stream);
   hipStreamWaitEvent(side, evR, 0);
@@ -1697,18 +1340,22 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
                       (void *)&dinfo, (void *)&S, (void *)&gmaxi, (void *)&seq0, (void *)&one};
       int tok = prof_begin(stream, IsReal<T>::v ? PK_PANEL_F64
                                    : std::is_same<T, double2>::value ? PK_PANEL_C128 : PK_PANEL_C64);
-      // the tournament panel has no grid barrier, only bounded waits along
-      // its merge tree: an ordinary launch keeps it on the stream's own
-      // hardware queue (a cooperative launch goes through a queue of its
-      // own, with a cross-queue handoff before and after every panel)
+      // neither panel has a grid barrier, only bounded waits for workgroups
+      // that become resident as the trailing update's retire: an ordinary
+      // launch keeps it on the stream's own hardware queue (a cooperative
+      // launch goes through a queue of its own, with a cross-queue handoff
+      // before and after every panel)
       hipError_t e = tourn ? hipLaunchKernel(panel_fn, dim3((unsigned)G + 1), dim3(NR), args, 0, stream)
-                           : hipLaunchCooperativeKernel(panel_fn, dim3((unsigned)G), dim3(NR), args, 0, stream);
+                           : hipLaunchKernel(G <= PX_ONE ? panel_one : panel_two, dim3((unsigned)G), dim3(NR), args, 0,
+                                             stream);
       // algorithmic flops of the m x w panel: per column, one complex
       // reciprocal-multiply per row below it and a complex rank-1 update
       double pflops = 0;
       for (int j = 0; j < w; j++) pflops += (double)(m - j - 1) * (6.0 + 8.0 * (double)(w - j - 1));
       prof_end(stream, tok, pflops);
       if (e != hipSuccess) { rc = -3; break; }
+      if (S.linv && !tourn)
+        hipLaunchKernelGGL(k_unit_inv<T>, dim3(1), dim3(64), 0, stream, A, lda, r0, w, (T *)S.linv + (j0 / PW) * PW * PW);
       // this panel's interchanges on the block's other columns, with the
       // substitution (fast: the product by the panel block's inverse) on the
       // columns right of it
@@ -2673,7 +2320,6 @@ double absmax_c128(const double2 *x, long n, double *work, hipStream_t stream)
 struct BatchLayout {
   size_t off_info, off_plan, off_li, off_ts, total;
   long Gmax, npanels;
-  size_t off_cv, off_ci, off_cr, off_rc;
 };
 
 static BatchLayout batch_layout(long n)
@@ -2684,11 +2330,7 @@ static BatchLayout batch_layout(long n)
   L.npanels = (n + PW - 1) / PW;
   L.off_info = 96 * sizeof(unsigned);
   L.off_plan = L.off_info + 64;
-  L.off_cv = L.off_plan + r256(sizeof(int) * PLAN_LEN * L.npanels);
-  L.off_ci = L.off_cv + r256(sizeof(double) * 2 * L.Gmax);
-  L.off_cr = L.off_ci + r256(sizeof(unsigned long long) * 2 * L.Gmax);
-  L.off_rc = L.off_cr + r256(sizeof(float2) * 2 * L.Gmax * PW);
-  L.off_li = L.off_rc + r256(sizeof(float2) * 2 * PW);
+  L.off_li = L.off_plan + r256(sizeof(int) * PLAN_LEN * L.npanels);
   L.off_ts = L.off_li + r256(sizeof(float2) * PW * PW * L.npanels);
   const size_t ts_words = (size_t)ts_root_off(ts_levels(L.Gmax), L.Gmax) + TS_ROOT;
   L.total = r256(L.off_ts + sizeof(unsigned long long) * ts_words);
@@ -2733,10 +2375,7 @@ int lu_factor_batch(float2 *A, long n, long lda, int nbat, long sa, int *ipiv, l
   S.bar = (unsigned *)base;
   int *dinfo = (int *)(base + L.off_info);
   int *plans = (int *)(base + L.off_plan);
-  S.candv = (double *)(base + L.off_cv);
-  S.ckey = (unsigned long long *)(base + L.off_ci);
-  S.candrow = (void *)(base + L.off_cr);
-  S.rowc = (void *)(base + L.off_rc);
+  S.xch = nullptr;
   S.linv = (void *)(base + L.off_li);
   S.ts = (unsigned long long *)(base + L.off_ts);
   const float2 *linv = (const float2 *)S.linv;

@@ -1,0 +1,6 @@
+// the exact LU's panel for real matrices
+#include "lu_panel.inc"
+
+namespace scuffx {
+template const void *panel_x_kernel<double>(bool);
+}

@@ -45,3 +45,39 @@ def test_block_rows(sx, n, dtype):
     # covers both with room (seen: below n eps)
     berr = backward_error(A, M.numpy(), M.ipiv.cpu().numpy())
     assert berr <= 4 * max(n, 32) * EPS[dtype], berr
+
+
+# order 2^k Hadamard matrices: every entry of every remaining column ties with
+# the largest (+-2^j), and elimination is exact, so the interchanges are
+# LAPACK's only if each tie goes to the first row by its current position,
+# within a workgroup and across workgroups (256 rows each)
+@pytest.mark.parametrize("dtype", ["complex128", "float64", "complex64"])
+@pytest.mark.parametrize("n", [64, 512, 1024])
+def test_pivot_ties(sx, n, dtype):
+    import scipy.linalg as sl
+    print(f"pivot ties n={n} {dtype}", flush=True)
+    H = sl.hadamard(n).astype("float64")
+    rng = np.random.default_rng(n)
+    H = H[rng.permutation(n)]
+    LU, piv = sl.lu_factor(H)
+    A = H.astype(dtype)
+    M = sx.HMatrix.from_numpy(A, dtype=dtype)
+    assert M.LUFactorize() == 0
+    assert np.array_equal(M.ipiv.cpu().numpy(), piv + 1)
+    assert np.array_equal(M.numpy(), LU.astype(dtype))
+
+
+# past 15 workgroups (3840 rows) the panel polls keys first and reads the
+# winner's row after them; the last panels of the same matrix read all
+# candidates at once
+def test_panel_both_exchanges(sx):
+    import scipy.linalg as sl
+    n = 4100
+    print(f"both panel exchanges n={n}", flush=True)
+    A = matrix(n, "float64", 5)
+    M = sx.HMatrix.from_numpy(A)
+    assert M.LUFactorize() == 0
+    LU, piv = sl.lu_factor(A)
+    assert np.array_equal(M.ipiv.cpu().numpy(), piv + 1)
+    # same pivots: the factors differ by rounding carried through n steps
+    assert np.max(np.abs(M.numpy() - LU)) <= 4 * n * EPS["float64"] * np.max(np.abs(LU)) * 10
