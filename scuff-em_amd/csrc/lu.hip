@@ -1439,68 +1439,11 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
 }
 
 // ---------------------------------------------------------------------
-// triangular solves.  Blocked for trans='N': a diagonal block is solved
-// by one workgroup per right-hand side, the rest updated by the GEMM.
+// triangular solves, in one launch per triangle: one right-hand side down
+// the 64-row blocks with the inverses of the diagonal blocks (k_trsv_chain),
+// several right-hand sides and transposed systems as a chain of block
+// products on the matrix cores with substitution (k_trsm_chain).
 // ---------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(256)
-k_trsv_block(const T *A, long lda, long r0, int bs, T *B, long ldb, int lower, int unit)
-{
-  __shared__ T x[256];
-  T *b = B + (long)blockIdx.x * ldb + r0;
-  const int tid = threadIdx.x;
-  if (tid < bs) x[tid] = b[tid];
-  __syncthreads();
-  if (lower) {
-    for (int i = 0; i < bs; i++) {
-      if (!unit && tid == 0) x[i] = cdiv(x[i], A[(r0 + i) + (r0 + i) * lda]);
-      __syncthreads();
-      T xi = x[i];
-      if (tid > i && tid < bs) x[tid] = csub(x[tid], cmul(A[(r0 + tid) + (r0 + i) * lda], xi));
-      __syncthreads();
-    }
-  } else {
-    for (int i = bs - 1; i >= 0; i--) {
-      if (!unit && tid == 0) x[i] = cdiv(x[i], A[(r0 + i) + (r0 + i) * lda]);
-      __syncthreads();
-      T xi = x[i];
-      if (tid < i) x[tid] = csub(x[tid], cmul(A[(r0 + tid) + (r0 + i) * lda], xi));
-      __syncthreads();
-    }
-  }
-  if (tid < bs) b[tid] = x[tid];
-}
-
-// transposed / conjugate-transposed solves, one workgroup per column
-template <typename T>
-__global__ void __launch_bounds__(256)
-k_trsv_trans(const T *A, long lda, long n, T *B, long ldb, int upper_first, int conj_)
-{
-  T *b = B + (long)blockIdx.x * ldb;
-  __shared__ T red[256];
-  const int tid = threadIdx.x;
-  // solve U^T y = b (forward), then L^T x = y (backward)
-  for (int pass = 0; pass < 2; pass++) {
-    bool up = (pass == 0);
-    for (long s = 0; s < n; s++) {
-      long i = up ? s : n - 1 - s;
-      T acc = zero_v<T>();
-      if (up) { for (long r = tid; r < i; r += 256) { T a = conj_if(A[r + i * lda], conj_); mac(acc, a, b[r]); } }
-      else { for (long r = i + 1 + tid; r < n; r += 256) { T a = conj_if(A[r + i * lda], conj_); mac(acc, a, b[r]); } }
-      red[tid] = acc;
-      __syncthreads();
-      for (int q = 128; q > 0; q >>= 1) { if (tid < q) red[tid] = cadd(red[tid], red[tid + q]); __syncthreads(); }
-      if (tid == 0) {
-        T v = csub(b[i], red[0]);
-        if (up) { T d = conj_if(A[i + i * lda], conj_); v = cdiv(v, d); }
-        b[i] = v;
-      }
-      __syncthreads();
-    }
-  }
-  (void)upper_first;
-}
-
 template <typename T>
 __global__ void k_laswp_rev(T *B, long ldb, long n, long nrhs, const int *ipiv)
 {
@@ -1569,52 +1512,84 @@ template <typename T>
 static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, bool fwd, T *tmp, hipStream_t s,
                            int *perm_buf = nullptr, bool perm_ready = false);
 
-// Triangular solves with few right-hand sides, in 64-row block steps.
-// The diagonal 64x64 blocks of L (unit lower) and U (upper) are inverted
-// first, all blocks at once (k_diag_inv), so every block step is a small
-// matrix-vector product instead of a 64-step serial substitution.
+// Inverses of the diagonal 64x64 blocks of L (unit lower, blockIdx.y = 0)
+// and U (blockIdx.y = 1, as the transpose of a lower triangle), identity
+// past row n: every block step of a one-right-hand-side solve is then a
+// product.  One workgroup a block, a wave for 16 columns of the inverse, a
+// lane for a row; step k passes x_k of every column by lane reads.  Bound:
+// issue of the 64 x 16 lane reads and updates.  A column per thread of one
+// wave, its sums from LDS, took 100 us for each triangle, this takes 59 us
+// for both in complex128 (order 2501; the first 16 (q + 1)
+// columns only in steps 16 q ..: 78 us with every column in every step).
 #define TB 64
-template <typename T, bool LOWER>
-__global__ void __launch_bounds__(TB)
-k_diag_inv(const T *LU, long lda, long n, T *inv, long sa, long sinv)
+template <typename T>
+__global__ void __launch_bounds__(256)
+k_tri_inv(const T *LU, long lda, long n, T *invL, T *invU, long sa, long sinv)
 {
-  {
-    const long z = blockIdx.z;   // instance of a batch
-    LU += z * sa; inv += z * sinv;
-  }
   __shared__ T D[TB][TB + 1];
-  __shared__ T X[TB][TB + 1];       // X[r][j]: column j of the inverse
-  const int t = threadIdx.x;
-  const long kb = (long)blockIdx.x * TB;
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  const bool up = blockIdx.y != 0;
+  const long z = blockIdx.z, kb = (long)blockIdx.x * TB;   // instance z of a batch
   const int bs = (int)std::min<long>(TB, n - kb);
-  for (int q = 0; q < TB; q++) {
-    T v;
-    if (t < bs && q < bs) v = LU[(kb + t) + (kb + q) * lda];
-    else v = (t == q) ? unit_v<T>() : zero_v<T>();
-    D[t][q] = v;
+  LU += z * sa + kb + kb * lda;
+  {
+    T v[16];
+#pragma unroll
+    for (int u = 0; u < 16; u++)      // (past the edge a valid element, replaced by the identity)
+      v[u] = LU[min(lane, bs - 1) + min(wave + 4 * u, bs - 1) * lda];
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int c = wave + 4 * u;
+      if (lane >= bs || c >= bs) v[u] = lane == c ? unit_v<T>() : zero_v<T>();
+      if (up) D[c][lane] = v[u]; else D[lane][c] = v[u];
+    }
   }
   __syncthreads();
-  const int j = t;
-  if (LOWER) {
-    for (int r = 0; r < j; r++) { X[r][j] = zero_v<T>(); }
-    X[j][j] = unit_v<T>();
-    for (int r = j + 1; r < TB; r++) {
-      T acc = zero_v<T>();
-      for (int k = j; k < r; k++) acc = csub(acc, cmul(D[r][k], X[k][j]));
-      X[r][j] = acc;
+  const T rd = up ? crecip(D[lane][lane]) : unit_v<T>();
+  T y[16];
+#pragma unroll
+  for (int u = 0; u < 16; u++) y[u] = lane == wave + 4 * u ? unit_v<T>() : zero_v<T>();
+  // steps 16 q .. 16 q + 15 concern the first 16 (q + 1) columns
+  auto steps = [&](auto qc) __attribute__((always_inline)) {
+    constexpr int q = decltype(qc)::value;
+#pragma unroll 2
+    for (int k = 16 * q; k < 16 * q + 16; k++) {
+      const T d = D[lane][k], rk = readlane_t(rd, k);
+#pragma unroll
+      for (int u = 0; u < 4 * q + 4; u++) {
+        T x = readlane_t(y[u], k);
+        if (up) {
+          x = cmul(x, rk);
+          if (lane == k) y[u] = x;
+        }
+        if (lane > k) y[u] = fnma_t(y[u], d, x);
+      }
     }
+  };
+  steps(std::integral_constant<int, 0>{});
+  steps(std::integral_constant<int, 1>{});
+  steps(std::integral_constant<int, 2>{});
+  steps(std::integral_constant<int, 3>{});
+  T *o = (up ? invU : invL) + z * sinv + (long)blockIdx.x * TB * TB;
+  if (up) {
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; u++) D[wave + 4 * u][lane] = y[u];
+    __syncthreads();
+    for (int u = 0; u < 16; u++) o[lane + (wave + 4 * u) * TB] = D[lane][wave + 4 * u];
   } else {
-    for (int r = j + 1; r < TB; r++) { X[r][j] = zero_v<T>(); }
-    X[j][j] = crecip(D[j][j]);
-    for (int r = j - 1; r >= 0; r--) {
-      T acc = zero_v<T>();
-      for (int k = r + 1; k <= j; k++) acc = csub(acc, cmul(D[r][k], X[k][j]));
-      X[r][j] = cdiv(acc, D[r][r]);
-    }
+#pragma unroll
+    for (int u = 0; u < 16; u++) o[lane + (wave + 4 * u) * TB] = y[u];
   }
-  __syncthreads();
-  T *o = inv + (long)blockIdx.x * TB * TB;
-  for (int q = 0; q < TB; q++) o[t + q * TB] = X[t][q];
+}
+
+template <typename T>
+static void tri_inv(const T *LU, long lda, long n, T *invL, T *invU, hipStream_t s, int nbat = 1, long sa = 0,
+                    long sinv = 0)
+{
+  const long nblk = (n + TB - 1) / TB;
+  hipLaunchKernelGGL(k_tri_inv<T>, dim3((unsigned)nblk, 2, (unsigned)nbat), dim3(256), 0, s, LU, lda, n, invL, invU, sa,
+                     sinv);
 }
 
 // one block step: x_b = inv(D_b) r_b (every workgroup, from L2), the
@@ -1822,30 +1797,228 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
   }
 }
 
+// Several right-hand sides, or transposed systems, in one launch per
+// triangle: workgroup (block g of 64 rows, tile of 16 columns) subtracts the
+// products with every earlier solution block on the matrix cores as that
+// block is published, then substitutes through its diagonal block and
+// publishes its own 64 x 16 values.  FWD: blocks in ascending order.  The
+// matrix is L (FWD) or U, TRANS: U^T (FWD) or L^T, whose blocks are read as
+// they lie (a lane then owns a row segment of 16 words).  Published values
+// lie packed, [tile][row][16], filled with the sentinel first, as in
+// k_trsv_chain: one memory round trip per block step, no barrier until the
+// last (each wave holds 16 rows and polls the words it multiplies).
+// Workgroups take their place in solve order from a ticket, so a wait is
+// only ever for a workgroup that has started: any grid makes progress.
+// Every wait is bounded all the same.
+// The diagonal block is substituted, a wave for four columns, a lane for a
+// row: products with its explicit inverse are 2 us a step cheaper, but where
+// the block is badly scaled (eps = 10 spheres at imaginary frequency 0.001)
+// they lose every digit.  Its entries come in four sets of 16 columns, the
+// first loaded before the wait, the others while the one before is used.
+// bin: column-major right-hand sides, row r taken from pin[r] if given, or
+// null: packed in win.  bout: column-major results or null, row r to pout[r]
+// if given.  cj: 1 conjugates the right-hand sides, 2 the results in bout.
+// Bound: the chain of block steps up to a few hundred columns (a round trip,
+// 16 complex 16x16x4 products and 64 substitution steps per wave), the
+// matrix units past that.  N=3840 complex128: 17 us a step; 181 columns 2.8
+// ms, where substitution in 256-row blocks by one workgroup a column and GEMM
+// updates took 6.0; one transposed system 2.4 ms, where a single workgroup
+// with a reduction per row took 24; 1920 columns 7.2 ms (31 TFLOP/s).
+template <typename T> struct ChainArgs {
+  const T *A; long lda; long n;
+  const T *bin; long ldb; const int *pin; const T *win;
+  T *w; T *bout; long ldo; const int *pout;
+  long nrhs; int cj; unsigned *err, *ticket;
+};
+
+// acc += a x for 16 k-steps of the matrix instruction
+template <typename T>
+__device__ inline void chain_mac(const T (&a)[16], const T (&x)[16], typename CT<T>::V4 &re, typename CT<T>::V4 &im)
+{
+#pragma unroll
+  for (int s = 0; s < 16; s++) {
+    if constexpr (IsReal<T>::v) re = CT<T>::mfma(a[s], x[s], re);
+    else {
+      re = CT<T>::mfma(a[s].x, x[s].x, re);
+      im = CT<T>::mfma(a[s].x, x[s].y, im);
+      re = CT<T>::mfma(-a[s].y, x[s].y, re);
+      im = CT<T>::mfma(a[s].y, x[s].x, im);
+    }
+  }
+}
+template <typename T> __device__ inline T chain_elem(typename CT<T>::V4 re, typename CT<T>::V4 im, int r)
+{
+  if constexpr (IsReal<T>::v) return re[r];
+  else { T v; v.x = re[r]; v.y = im[r]; return v; }
+}
+
+template <typename T, bool FWD, bool TRANS>
+__global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
+{
+  typedef typename CT<T>::V4 V4;
+  constexpr int NC = 16;
+  constexpr bool UNIT = FWD != TRANS;
+  __shared__ T sb[TB][NC + 1];
+  __shared__ unsigned s_tk;
+  const int t = threadIdx.x, lane = t & 63, i = lane & 15, kq = lane >> 4, w0 = (t >> 6) * 16;
+  if (t == 0) s_tk = __hip_atomic_fetch_add(p.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const long n = p.n, lda = p.lda, nblk = (n + TB - 1) / TB, ntile = (p.nrhs + NC - 1) / NC;
+  const long nk = s_tk / ntile, tile = s_tk % ntile;      // blocks before this one in solve order
+  if (nk >= nblk) return;
+  auto blk = [&](long q) { return FWD ? q : nblk - 1 - q; };
+  const long g = blk(nk);
+  const int bs = (int)std::min<long>(TB, n - g * TB);
+  T *wt = p.w + tile * nblk * TB * NC;
+  // this lane's 16 values of block (g, k): matrix row 16 kq + s of the
+  // k-step, row w0 + i of the block
+  auto load = [&](long k, T (&a)[16]) {
+    const long row = g * TB + w0 + i, col = k * TB + 16 * kq;
+    if (std::max(g, k) * TB + TB <= n) {
+      const T *q = TRANS ? p.A + col + row * lda : p.A + row + col * lda;
+#pragma unroll
+      for (int s = 0; s < 16; s++) a[s] = TRANS ? q[s] : q[s * lda];
+    } else {
+      const long rc = min(row, n - 1);
+#pragma unroll
+      for (int s = 0; s < 16; s++) {
+        const long cc = min(col + s, n - 1);
+        a[s] = TRANS ? p.A[cc + rc * lda] : p.A[rc + cc * lda];
+        if (row >= n || col + s >= n) a[s] = zero_v<T>();
+      }
+    }
+  };
+  // set u of the diagonal block in solve order: this lane's row of columns
+  // 16 u .. (FWD) or 63 - 16 u, .. (clamped past the edge, where nothing
+  // uses the values)
+  const T *Ad = p.A + g * TB * (lda + 1);
+  auto dload = [&](int u, T (&d)[16]) {
+    const int r = min(lane, bs - 1);
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      const int k = min(FWD ? 16 * u + s : TB - 1 - 16 * u - s, bs - 1);
+      d[s] = TRANS ? Ad[k + r * lda] : Ad[r + k * lda];
+    }
+  };
+  // the first set, the diagonal's reciprocal and the right-hand side,
+  // loaded ahead
+  T m[16], b[4], rd = unit_v<T>();
+  dload(0, m);
+  if (!UNIT && lane < bs) rd = crecip(Ad[lane * (lda + 1)]);
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int br = w0 + CT<T>::row(lane, r);
+    const long row = g * TB + br, c = tile * NC + i;
+    b[r] = zero_v<T>();
+    if (p.bin) {
+      if (br < bs && c < p.nrhs) b[r] = conj_if(p.bin[(p.pin ? p.pin[row] : row) + c * p.ldb], p.cj & 1);
+    } else if (br < bs) b[r] = p.win[(tile * nblk * TB + row) * NC + i];
+  }
+  V4 re = CT<T>::zero(), im = CT<T>::zero();
+  T a[16], x[16];
+  if (nk > 0) load(blk(0), a);
+  for (long q = 0; q < nk; q++) {
+    const T *xs = wt + (blk(q) * TB + 16 * kq) * NC + i;
+    unsigned spins = 0;
+    for (;;) {
+      bool ready = true;
+#pragma unroll
+      for (int s = 0; s < 16; s++) x[s] = ld_coh(xs + s * NC);
+#pragma unroll
+      for (int s = 0; s < 16; s++) ready = ready && chain_val_set(x[s]);
+      if (ready) break;
+      if (__hip_atomic_load(p.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) break;
+      if (++spins > GBAR_SPIN) { __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
+      __builtin_amdgcn_s_sleep(1);
+    }
+    chain_mac<T>(a, x, re, im);
+    if (q + 1 < nk) load(blk(q + 1), a);
+    if ((q & 3) == 3) {
+      // sums of 256 products each, subtracted one by one: a sum over the
+      // whole row would round against its own size (error 1.6 times as large)
+#pragma unroll
+      for (int r = 0; r < 4; r++) b[r] = csub(b[r], chain_elem<T>(re, im, r));
+      re = CT<T>::zero();
+      im = CT<T>::zero();
+    }
+  }
+  dload(1, x);
+  dload(2, a);
+#pragma unroll
+  for (int r = 0; r < 4; r++) sb[w0 + CT<T>::row(lane, r)][i] = csub(b[r], chain_elem<T>(re, im, r));
+  __syncthreads();
+  const int c4 = w0 / 4;                 // this wave's four columns
+  if (tile * NC + c4 < p.nrhs) {
+    T y[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) y[c] = sb[lane][c4 + c];
+    auto steps = [&](int u, const T (&d)[16]) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < 16; s++) {
+        const int k = FWD ? 16 * u + s : TB - 1 - 16 * u - s;
+        if (k < bs) {
+          const T rk = readlane_t(rd, k);
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            T v = readlane_t(y[c], k);
+            if (!UNIT) {
+              v = cmul(v, rk);
+              if (lane == k) y[c] = v;
+            }
+            if (FWD ? lane > k : lane < k) y[c] = fnma_t(y[c], d[s], v);
+          }
+        }
+      }
+    };
+    steps(0, m);
+    dload(3, m);
+    steps(1, x);
+    steps(2, a);
+    steps(3, m);
+#pragma unroll
+    for (int c = 0; c < 4; c++) sb[lane][c4 + c] = lane < bs ? y[c] : zero_v<T>();
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    const int br = w0 + kq + 4 * r;
+    const long row = g * TB + br, c = tile * NC + i;
+    const T v = sb[br][i];
+    st_coh(wt + row * NC + i, v);
+    if (p.bout && br < bs && c < p.nrhs) p.bout[(p.pout ? p.pout[row] : row) + c * p.ldo] = conj_if(v, (p.cj & 2) != 0);
+  }
+}
+
 __global__ void k_zero_u64(unsigned long long *w, long n)
 {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) w[i] = 0ull;
 }
 
+// whether a grid of one workgroup per 64 rows is resident (cooperative launch)
+template <typename T> static bool chain_resident(long n)
+{
+  static int ncu = -1, perCU = 0;
+  if (ncu < 0) {
+    int dev = 0, c = 0;
+    hipGetDevice(&dev);
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_trsv_chain<T, true>, 256, 0);
+    hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
+    ncu = c;
+  }
+  return (long)ncu * perCU >= (n + TB - 1) / TB;
+}
+
 // lower (forward) then upper (backward) solve of one right-hand side in
-// two cooperative launches; returns -1 if it cannot run (grid not
-// co-resident, workspace), -6 on a time-out
+// two cooperative launches (chain_resident(n)); returns -2 without a
+// workspace, -6 on a time-out
 template <typename T>
 static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *invU, T *B, T *W, hipStream_t s,
                       unsigned long long *words)
 {
   const long nblk = (n + TB - 1) / TB;
-  static int ncu = -1, perCU = 0;
-  if (ncu < 0) {
-    int dev = 0;
-    hipGetDevice(&dev);
-    hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_trsv_chain<T, true>, 256, 0);
-  }
-  if ((long)ncu * perCU < nblk) return -1;
   char *w = words ? (char *)words : (char *)ws_get(WS_CHAIN, sizeof(unsigned long long) * (2 * nblk + 8));
-  if (!w) return -1;
+  if (!w) return -2;
   unsigned *err = (unsigned *)w;
   // cleared and filled by kernels (not memset nodes, so that a captured
   // sequence does the same on every replay)
@@ -1886,6 +2059,66 @@ static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, b
   hipMemcpy2DAsync(B, sizeof(T) * ldb, tmp, sizeof(T) * n, sizeof(T) * n, nrhs, hipMemcpyDeviceToDevice, s);
 }
 
+// one triangle of k_trsm_chain
+template <typename T>
+static void trsm_launch(bool fwd, bool trans, const ChainArgs<T> &p, hipStream_t s)
+{
+  const long nblk = (p.n + TB - 1) / TB, ntile = (p.nrhs + 15) / 16;
+  const dim3 grid((unsigned)(nblk * ntile));
+  if (fwd && !trans) hipLaunchKernelGGL((k_trsm_chain<T, true, false>), grid, dim3(256), 0, s, p);
+  else if (!trans) hipLaunchKernelGGL((k_trsm_chain<T, false, false>), grid, dim3(256), 0, s, p);
+  else if (fwd) hipLaunchKernelGGL((k_trsm_chain<T, true, true>), grid, dim3(256), 0, s, p);
+  else hipLaunchKernelGGL((k_trsm_chain<T, false, true>), grid, dim3(256), 0, s, p);
+}
+
+// op(A) X = B for any number of right-hand sides, at most CHAIN_COLS at a
+// time: that bounds the workspace, and 64 tiles a block step fill the GPU.
+#define CHAIN_COLS 1024
+template <typename T>
+static int trsm_chain(const T *LU, long lda, long n, const int *ipiv, bool tr, bool cj, long nrhs, T *B, long ldb,
+                      hipStream_t s)
+{
+  const long nblk = (n + TB - 1) / TB, cols = std::min<long>(nrhs, CHAIN_COLS);
+  const size_t wlen = (size_t)nblk * TB * 16 * ((cols + 15) / 16);      // elements of one packed set
+  T *W1 = (T *)ws_get(WS_SOLVE_W, sizeof(T) * wlen), *W2 = (T *)ws_get(WS_PERM_TMP, sizeof(T) * wlen);
+  unsigned long long *word = (unsigned long long *)ws_get(WS_CHAIN, sizeof(unsigned long long) * (2 * nblk + 8));
+  int *perm = n > PERM_LDS_MAX ? nullptr : (int *)ws_get(WS_PERM, sizeof(int) * n);
+  if (!W1 || !W2 || !word || (n <= PERM_LDS_MAX && !perm)) return -2;
+  if (perm) hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(64), 0, s, ipiv, n, perm, 0L, 0L);
+  ChainArgs<T> p;
+  p.lda = lda;
+  p.err = (unsigned *)word;
+  auto fill = [&](T *w, long ncol) {
+    const long ne = nblk * TB * 16 * ((ncol + 15) / 16);
+    hipLaunchKernelGGL(k_chain_fill<T>, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s, w, ne);
+  };
+  // the time-out word once, the two tickets before every set of columns
+  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, word, 1L);
+  for (long c0 = 0; c0 < nrhs; c0 += CHAIN_COLS) {
+    const long nc = std::min<long>(CHAIN_COLS, nrhs - c0);
+    T *Bc = B + c0 * ldb;
+    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, word + 1, 2L);
+    p.nrhs = nc;
+    if (!perm && !tr) laswp(Bc, ldb, 0, nc, 0, n, ipiv, s);
+    fill(W1, nc);
+    fill(W2, nc);
+    p.A = LU; p.n = n; p.ldb = p.ldo = ldb;
+    p.bin = Bc; p.pin = tr ? nullptr : perm; p.win = nullptr;
+    p.w = W1; p.bout = nullptr; p.pout = nullptr; p.cj = cj ? 1 : 0; p.ticket = (unsigned *)(word + 1);
+    trsm_launch(true, tr, p, s);
+    p.bin = nullptr; p.pin = nullptr; p.win = W1;
+    p.w = W2; p.bout = Bc; p.pout = tr ? perm : nullptr; p.cj = cj ? 2 : 0; p.ticket = (unsigned *)(word + 2);
+    trsm_launch(false, tr, p, s);
+    if (!perm && tr)
+      hipLaunchKernelGGL(k_laswp_rev<T>, dim3((unsigned)((nc + 63) / 64)), dim3(64), 0, s, Bc, ldb, n, nc, ipiv);
+  }
+  unsigned tmo = 0;
+  hipMemcpyAsync(&tmo, p.err, sizeof(unsigned), hipMemcpyDeviceToHost, s);
+  hipStreamSynchronize(s);
+  if (hipGetLastError() != hipSuccess) return -3;
+  return tmo ? -6 : 0;
+}
+
 template <typename T>
 size_t solve_ws_bytes(long n)
 {
@@ -1916,9 +2149,11 @@ int lu_solve(const T *LU, long n, long lda, const int *d_ipiv, char trans, long 
   if (n < 0 || nrhs < 0 || lda < std::max(1L, n) || ldb < std::max(1L, n)) return -1;
   if (n == 0 || nrhs == 0) return 0;
   if (ws && !((trans == 'N' || trans == 'n') && nrhs == 1)) return -1;
-  if ((trans == 'N' || trans == 'n') && nrhs <= 16) {
+  const bool tr = trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', cj = trans == 'C' || trans == 'c';
+  if (!tr && trans != 'N' && trans != 'n') return -1;
+  if (!tr && nrhs == 1 && chain_resident<T>(n)) {
     const long nblk = (n + TB - 1) / TB;
-    T *W = ws ? ws->W : (T *)ws_get(WS_SOLVE_W, sizeof(T) * n * nrhs);
+    T *W = ws ? ws->W : (T *)ws_get(WS_SOLVE_W, sizeof(T) * n);
     T *invL = ws ? ws->invL : (T *)ws_get(WS_SOLVE_INVL, sizeof(T) * nblk * TB * TB);
     T *invU = ws ? ws->invU : (T *)ws_get(WS_SOLVE_INVU, sizeof(T) * nblk * TB * TB);
     if (!W || !invL || !invU) return -2;
@@ -1926,54 +2161,13 @@ int lu_solve(const T *LU, long n, long lda, const int *d_ipiv, char trans, long 
     // inverses and the composed permutation
     const bool cached = ws && ws->inv_ready;
     if (!cached) {
-      hipLaunchKernelGGL((k_diag_inv<T, true>), dim3((unsigned)nblk), dim3(TB), 0, stream, LU, lda, n, invL, 0L, 0L);
-      hipLaunchKernelGGL((k_diag_inv<T, false>), dim3((unsigned)nblk), dim3(TB), 0, stream, LU, lda, n, invU, 0L, 0L);
+      tri_inv(LU, lda, n, invL, invU, stream);
       if (ws) ws->inv_ready = true;
     }
     apply_row_perm(B, ldb, n, nrhs, d_ipiv, true, W, stream, ws ? ws->perm : nullptr, cached);
-    if (nrhs == 1) {
-      int rc = trsv_chain(LU, lda, n, invL, invU, B, W, stream, ws ? ws->chain : nullptr);
-      if (rc != -1) return rc;
-    }
-    // L y = P b: y accumulates in W, B holds the running right-hand side
-    for (long kb = 0; kb < n; kb += TB) {
-      int bs = (int)std::min<long>(TB, n - kb);
-      long rows = n - kb - bs;
-      dim3 grid((unsigned)std::max<long>(1, (rows + 255) / 256), (unsigned)nrhs);
-      hipLaunchKernelGGL((k_trsv_inv<T, true>), grid, dim3(256), 0, stream, LU, lda, n, kb, bs,
-                         invL + (kb / TB) * TB * TB, B, ldb, W, n, 0L, 0L, 0L, 0L);
-    }
-    // U x = y: W is updated in place, the solution lands in B
-    long last = ((n - 1) / TB) * TB;
-    for (long kb = last; kb >= 0; kb -= TB) {
-      int bs = (int)std::min<long>(TB, n - kb);
-      dim3 grid((unsigned)std::max<long>(1, (kb + 255) / 256), (unsigned)nrhs);
-      hipLaunchKernelGGL((k_trsv_inv<T, false>), grid, dim3(256), 0, stream, LU, lda, n, kb, bs,
-                         invU + (kb / TB) * TB * TB, W, n, B, ldb, 0L, 0L, 0L, 0L);
-    }
-    return hipGetLastError() == hipSuccess ? 0 : -3;
+    return trsv_chain(LU, lda, n, invL, invU, B, W, stream, ws ? ws->chain : nullptr);
   }
-  T *tmp = (T *)ws_get(WS_PERM_TMP, sizeof(T) * n * nrhs);
-  if (trans == 'N' || trans == 'n') {
-    apply_row_perm(B, ldb, n, nrhs, d_ipiv, true, tmp, stream);
-    const int bs = 256;
-    for (long kb = 0; kb < n; kb += bs) {
-      int w = (int)std::min<long>(bs, n - kb);
-      hipLaunchKernelGGL(k_trsv_block<T>, dim3((unsigned)nrhs), dim3(256), 0, stream, LU, lda, kb, w, B, ldb, 1, 1);
-      if (kb + w < n) gemm_sub(n - kb - w, nrhs, (long)w, LU + (kb + w) + kb * lda, lda, B + kb, ldb, B + kb + w, ldb, stream);
-    }
-    long last = ((n - 1) / bs) * bs;
-    for (long kb = last; kb >= 0; kb -= bs) {
-      int w = (int)std::min<long>(bs, n - kb);
-      hipLaunchKernelGGL(k_trsv_block<T>, dim3((unsigned)nrhs), dim3(256), 0, stream, LU, lda, kb, w, B, ldb, 0, 0);
-      if (kb > 0) gemm_sub(kb, nrhs, (long)w, LU + kb * lda, lda, B + kb, ldb, B, ldb, stream);
-    }
-  } else if (trans == 'T' || trans == 't' || trans == 'C' || trans == 'c') {
-    int cj = (trans == 'C' || trans == 'c');
-    hipLaunchKernelGGL(k_trsv_trans<T>, dim3((unsigned)nrhs), dim3(256), 0, stream, LU, lda, n, B, ldb, 1, cj);
-    apply_row_perm(B, ldb, n, nrhs, d_ipiv, false, tmp, stream);
-  } else return -1;
-  return hipGetLastError() == hipSuccess ? 0 : -3;
+  return trsm_chain(LU, lda, n, d_ipiv, tr, cj, nrhs, B, ldb, stream);
 }
 
 // log det of an LU-factored matrix: sum of log |U_ii| and of arg U_ii, plus
@@ -2451,10 +2645,7 @@ int lu_solve_batch_prepare(const float2 *LU, long n, long lda, int nbat, long sa
   const long sw = (long)L.total, nblk = (n + TB - 1) / TB;
   char *base = (char *)ws;
   hipLaunchKernelGGL(k_perm_build, dim3((unsigned)nbat), dim3(64), 0, s, ipiv, n, (int *)base, sp, sw / 4);
-  hipLaunchKernelGGL((k_diag_inv<float2, true>), dim3((unsigned)nblk, 1, (unsigned)nbat), dim3(TB), 0, s, LU, lda, n,
-                     (float2 *)(base + L.off_invL), sa, sw / 8);
-  hipLaunchKernelGGL((k_diag_inv<float2, false>), dim3((unsigned)nblk, 1, (unsigned)nbat), dim3(TB), 0, s, LU, lda, n,
-                     (float2 *)(base + L.off_invU), sa, sw / 8);
+  tri_inv(LU, lda, n, (float2 *)(base + L.off_invL), (float2 *)(base + L.off_invU), s, nbat, sa, sw / 8);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 

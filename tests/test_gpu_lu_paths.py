@@ -81,3 +81,28 @@ def test_panel_both_exchanges(sx):
     assert np.array_equal(M.ipiv.cpu().numpy(), piv + 1)
     # same pivots: the factors differ by rounding carried through n steps
     assert np.max(np.abs(M.numpy() - LU)) <= 4 * n * EPS["float64"] * np.max(np.abs(LU)) * 10
+
+
+# solves by blocks of 64 rows and tiles of 16 columns: one row, the edges of
+# a block and of a tile, one and several blocks, a ragged last block; 1100
+# columns take two sets
+@pytest.mark.parametrize("dtype", ["complex128", "float64", "complex64"])
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (1, 3), (63, 2), (64, 16), (65, 17), (300, 1), (300, 40), (1030, 5),
+                                    (300, 600), (130, 1100)])
+def test_solve_blocks(sx, n, nrhs, dtype):
+    A = matrix(n, dtype, 7 * n + nrhs)
+    B = matrix(max(n, nrhs), dtype, n + nrhs)[:n, :nrhs].copy()
+    M = sx.HMatrix.from_numpy(A, dtype=dtype)
+    assert M.LUFactorize() == 0
+    wide = np.complex128 if np.iscomplexobj(A) else np.float64
+    for trans in "NTC":
+        print(f"solve n={n} nrhs={nrhs} {trans} {dtype}", flush=True)
+        X = sx.HMatrix.from_numpy(B, dtype=dtype)
+        M.LUSolve(X, Trans=trans)
+        x = X.numpy().astype(wide)
+        op = {"N": A, "T": A.T, "C": A.conj().T}[trans].astype(wide)
+        # columnwise |b - op(A) x| against |A| |x|: the factorization's
+        # backward error (4 n eps, as above) and two triangles of inner
+        # products, with the 64-row blocks' inverses, of the same order
+        res = np.linalg.norm(B - op @ x, axis=0) / (np.linalg.norm(A) * np.linalg.norm(x, axis=0))
+        assert res.max() <= 8 * max(n, 32) * EPS[dtype], res.max()
