@@ -645,7 +645,7 @@ int Assembler::run_sw(int sa, int sb, int bi, const RegionK *rk, int nreg, const
   const Surface &Sa = G_.Surfaces[sa], &Sb = G_.Surfaces[sb];
   const NearBlock &B = blocks_[bi];
   const int same = (sa == sb);
-  std::vector<SWJob> jobs;
+  std::vector<SWJob> byKind[4];
   std::vector<char> seen(B.pairs.size(), 0);
   for (int r = 0; r < nreg; r++) {
     const double ak = std::hypot(rk[r].k.r, rk[r].k.i);
@@ -659,16 +659,22 @@ int Assembler::run_sw(int sa, int sb, int bi, const RegionK *rk, int nreg, const
         const double kR = ak * std::max(Sa.Panels[pa].Radius, Sb.Panels[pb].Radius);
         if (!(kR > M_PI)) continue;
         const int ncv = B.pairs[id].ncv;
-        if (ncv == 0) { jobs.push_back(SWJob{id, r, 0, 0}); continue; }
+        if (ncv == 0) { byKind[0].push_back(SWJob{id, r, 0, 0}); continue; }
         if (kR > 20.0) {
           err_ = "common-edge/vertex pair with |k| R_panel > 20: the reference's high-k gradient kernel "
                  "has no defined value there (TaylorDuffy.cc:812)";
           return -5;
         }
-        for (int q = 0; q < 9; q++) jobs.push_back(SWJob{id, r, q, 1});
+        for (int q = 0; q < 9; q++) byKind[ncv].push_back(SWJob{id, r, q, ncv});
       }
     // a self panel past |k| R > 20 (high-k Taylor-Duffy) always comes
     // with common-edge neighbours past 20 on a closed mesh, rejected above
+  }
+  std::vector<SWJob> jobs;
+  int njobs[4];
+  for (int kind = 0; kind < 4; kind++) {
+    njobs[kind] = (int)byKind[kind].size();
+    jobs.insert(jobs.end(), byKind[kind].begin(), byKind[kind].end());
   }
   if (jobs.empty()) return 0;
   if (jobs.size() > cap_swjobs_) {
@@ -679,11 +685,10 @@ int Assembler::run_sw(int sa, int sb, int bi, const RegionK *rk, int nreg, const
     cap_swjobs_ = jobs.size();
   }
   HIPCHK(hipMemcpy(d_swjobs_, jobs.data(), sizeof(SWJob) * jobs.size(), hipMemcpyHostToDevice));
-  // one wave per job; 4096 jobs (16 waves per CU) hold 415 MB of value caches
-  const int chunk = 4096;
-  if (ensure(&d_scratch_, &cap_scratch_, (size_t)chunk * SCUFFX_SW_SLAB)) return -2;
-  HIPCHK(launch_sw(stream, d_swjobs_, (int)jobs.size(), B.d_pairs, ds_[sa].V, ds_[sa].PVI, nreg, dreg, needH1,
-                   d_HN_, d_HS_, d_scratch_, chunk));
+  // one wave per job; 4096 of them (16 waves per CU) hold 415 MB of value caches
+  const int slabs = 4096;
+  if (ensure(&d_scratch_, &cap_scratch_, (size_t)slabs * SCUFFX_SW_SLAB)) return -2;
+  HIPCHK(launch_sw(stream, d_swjobs_, njobs, B.d_pairs, nreg, dreg, needH1, d_HN_, d_scratch_, slabs));
   stats_.nsw += (long)jobs.size();
   return 0;
 }

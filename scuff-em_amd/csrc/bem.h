@@ -94,17 +94,17 @@ hipError_t launch_stamp(hipStream_t stream, int nEa, const int *EIa, const doubl
                         MatOut M, int rowOff, int colOff);
 hipError_t launch_mirror(hipStream_t stream, MatOut M, int n);
 hipError_t launch_copy_block(hipStream_t stream, MatOut M, long from, long to, long n);
-// short-wavelength panel pairs (kern_sw.hip): kind 0 = near pair without a
-// common vertex (all 9 combinations, 78-point rules), 1 = common edge /
-// vertex near pair (Taylor-Duffy, combination q); pair = near-pair index
+// short-wavelength panel pairs (kern_sw.hip): kind = common vertices; 0: all
+// 9 combinations, 78-point rules, else Taylor-Duffy, combination q; pair =
+// near-pair index
 struct SWJob {
   int pair, region, q, kind;
 };
 // doubles of scratch per Taylor-Duffy job (its cached integrand values)
 #define SCUFFX_SW_SLAB (2112 * 6)
-hipError_t launch_sw(hipStream_t stream, const SWJob *jobs, int njobs, const NearPair *nps, const double *V,
-                     const int *PVI, int nreg, const RegionK *regs, int needH1, double *HN, double *HS,
-                     double *scratch, int chunk);
+// jobs ordered by kind, njobs[kind] of each; slabs: job slabs in scratch
+hipError_t launch_sw(hipStream_t stream, const SWJob *jobs, const int njobs[4], const NearPair *nps, int nreg,
+                     const RegionK *regs, int needH1, double *HN, double *scratch, int slabs);
 // rotation generators of up to three torque axes, Gamma[9 t + i + 3 j]
 struct GammaSet {
   int n;

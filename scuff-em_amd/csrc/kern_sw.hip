@@ -18,6 +18,7 @@
 #include <hip/hip_runtime.h>
 
 #include "bem.h"
+#include "exprel.h"
 #include "tcr20.inc"
 
 namespace scuffx {
@@ -26,6 +27,7 @@ namespace scuffx {
 #define TD_CT 3
 #define TD_CE 2
 #define TD_CV 1
+#define SW_SEP 0
 #define TD_NREG 6
 #define TD_NWP 5
 #define TD_NMON 22
@@ -45,28 +47,24 @@ enum { T1 = 0, TY1 = 1, TY12 = 2, TY2 = 3, TY1Y2 = 4, TY22 = 5, TY13 = 6,
        TY12Y2 = 7, TY1Y22 = 8, TY23 = 9, TY12Y22 = 10, TY13Y2 = 11, TY13Y22 = 12,
        TY3 = 13, TY1Y3 = 14, TY2Y3 = 15, TY12Y3 = 16, TY1Y2Y3 = 17, TY22Y3 = 18,
        TY12Y2Y3 = 19, TY1Y22Y32 = 20, TY22Y32 = 21 };
-enum { K_HELM = 0, K_GRADHELM = 1 };
 
 __constant__ double c_swx[PC_NX];
 __constant__ double c_sww[PC_NW];
 __constant__ double c_swtcr20[234];
 
 struct TDGeo {
-  int WhichCase, NumPKs;
-  int KIndex[TD_NPK];
+  int WhichCase;
   cplx k;
   double A2, B2, AP2, BP2, L2, AdB, AdAP, AdBP, AdL, BdAP, BdBP, APdBP, BPdL;
   int nMin[TD_NPK], nMax[TD_NPK];
 };
 
 // Upsilon coefficient tables (TaylorDuffy.cc:940-1262); C = {C2010, C2001,
-// C0210, C0201}, M symmetric 4x4 (upper triangle used, M[i + 4 j]), V[4], S
+// C0210, C0201}, M symmetric 4x4 (upper triangle used, M[i + 4 j]), V[4], S;
+// U comes zeroed
 __device__ void td_upsilon(int WhichCase, const double *C, const double *M, const double *V,
                            double S, double (*U)[TD_NWP][TD_NMON])
 {
-  for (int d = 0; d < TD_NREG; d++)
-    for (int n = 0; n < TD_NWP; n++)
-      for (int q = 0; q < TD_NMON; q++) U[d][n][q] = 0.0;
   double C2010 = C[0], C2001 = C[1], C0210 = C[2], C0201 = C[3];
   double M11 = M[0], M12 = M[4], M13 = M[8], M14 = M[12];
   double M22 = M[5], M23 = M[9], M24 = M[13];
@@ -319,143 +317,99 @@ __device__ inline double cv_x(const TDGeo &W, double xi1, double xi2, double eta
               - 2.0 * xi2 * (eta1 * W.BdAP + eta2 * W.BdBP)
               + 2.0 * eta1 * eta2 * W.APdBP);
 }
-__device__ void td_x(const TDGeo &W, const double *y, double *X)
+// (d is the same for every lane)
+template <int CASE> __device__ inline double td_x(const TDGeo &W, const double *y, int d)
 {
-  if (W.WhichCase == TD_CT) {
-    double t = y[0], u1, u2;
-    u1 = 1.0; u2 = t;     X[0] = sqrt(W.A2 * u1 * u1 + 2.0 * W.AdB * u1 * u2 + W.B2 * u2 * u2);
-    u1 = t; u2 = (t - 1); X[1] = sqrt(W.A2 * u1 * u1 + 2.0 * W.AdB * u1 * u2 + W.B2 * u2 * u2);
-    u1 = t; u2 = 1.0;     X[2] = sqrt(W.A2 * u1 * u1 + 2.0 * W.AdB * u1 * u2 + W.B2 * u2 * u2);
-  } else if (W.WhichCase == TD_CE) {
-    double y1 = y[0], y2 = y[1];
-    X[0] = ce_x(W, -y1, -y1 * y2, 1.0 - y1 + y1 * y2);
-    X[1] = ce_x(W, y1, y1 * y2, 1.0 - y1);
-    X[2] = ce_x(W, -y1 * y2, y1 * (1.0 - y2), 1.0 - y1);
-    X[3] = ce_x(W, y1 * y2, -y1 * (1.0 - y2), 1.0 - y1 * y2);
-    X[4] = ce_x(W, -y1 * y2, -y1, 1.0);
-    X[5] = ce_x(W, y1 * y2, y1, 1.0 - y1);
+  if constexpr (CASE == TD_CT) {
+    const double t = y[0], u1 = d == 0 ? 1.0 : t, u2 = d == 0 ? t : d == 1 ? t - 1 : 1.0;
+    return sqrt(W.A2 * u1 * u1 + 2.0 * W.AdB * u1 * u2 + W.B2 * u2 * u2);
+  } else if constexpr (CASE == TD_CE) {
+    const double y1 = y[0], y2 = y[1];
+    double u1, u2, xi2;
+    if (d == 0) { u1 = -y1; u2 = -y1 * y2; xi2 = 1.0 - y1 + y1 * y2; }
+    else if (d == 1) { u1 = y1; u2 = y1 * y2; xi2 = 1.0 - y1; }
+    else if (d == 2) { u1 = -y1 * y2; u2 = y1 * (1.0 - y2); xi2 = 1.0 - y1; }
+    else if (d == 3) { u1 = y1 * y2; u2 = -y1 * (1.0 - y2); xi2 = 1.0 - y1 * y2; }
+    else if (d == 4) { u1 = -y1 * y2; u2 = -y1; xi2 = 1.0; }
+    else { u1 = y1 * y2; u2 = y1; xi2 = 1.0 - y1; }
+    return ce_x(W, u1, u2, xi2);
   } else {
-    double y1 = y[0], y2 = y[1], y3 = y[2];
-    X[0] = cv_x(W, 1.0, y1, y2, y2 * y3);
-    X[1] = cv_x(W, y2, y2 * y3, 1.0, y1);
+    const double y1 = y[0], y2 = y[1], y3 = y[2];
+    return d == 0 ? cv_x(W, 1.0, y1, y2, y2 * y3) : cv_x(W, y2, y2 * y3, 1.0, y1);
   }
 }
 
-// script P of one polynomial at y (TaylorDuffy.cc:568-634): P[d][n][0..1]
-__device__ void td_script_p(const TDGeo &W, const double (*U)[TD_NWP][TD_NMON], int nMin, int nMax,
-                            const double *y, double (*P)[TD_NWP][2])
+// TaylorDuffySum (TaylorDuffy.cc:152-258) for P = UNITY, PMCHWG1 with the
+// Helmholtz kernel and PMCHWC with its gradient (script K, :896-935):
+// f[2 npk], f[2 npk + 1].  A region's relative exponentials of every order
+// are formed once for the three polynomials from one sine, cosine and pair
+// of exponentials: each of the tens of script-K values of a point with its
+// own, and with quotients, made the jobs of a 960-function sphere's shape
+// gradient (0.99 million) take 915 ms, 147 now.  Regions stay a rolled loop:
+// unrolled, the kernel spilled 200 registers and took twice as long.
+template <int CASE>
+__device__ inline void td_sum(const TDGeo &W, const double (*U)[TD_NREG][TD_NWP][TD_NMON], const double *y, double *f)
 {
-  if (W.WhichCase == TD_CT) {
-    for (int d = 0; d < 3; d++)
-      for (int n = nMin; n <= nMax; n++) { P[d][n][0] = U[d][n][T1]; P[d][n][1] = U[d][n][TY1]; }
-  } else if (W.WhichCase == TD_CE) {
-    double y1 = y[0], y12 = y1 * y1;
-    for (int d = 0; d < 6; d++)
-      for (int n = nMin; n <= nMax; n++) {
-        P[d][n][0] = U[d][n][T1] + U[d][n][TY1] * y1 + U[d][n][TY12] * y12;
-        P[d][n][1] = U[d][n][TY2] + U[d][n][TY1Y2] * y1 + U[d][n][TY12Y2] * y12;
+#pragma clang fp contract(fast)
+  constexpr int NR = CASE == TD_CT ? 3 : CASE == TD_CE ? 6 : 2, nOffset = CASE == TD_CT ? 1 : CASE == TD_CE ? 2 : 3;
+  const double yIn = y[nOffset - 1], Jac = CASE == TD_CT ? 1.0 : y[nOffset - 2];
+  if (Jac == 0.0) { for (int q = 0; q < SW_FDIM; q++) f[q] = 0.0; return; }
+  cplx s[TD_NPK];
+  for (int npk = 0; npk < TD_NPK; npk++) s[npk] = mk(0, 0);
+  const cplx IK = IMUL(W.k);
+  const double y1 = y[0], y12 = y1 * y1, y2 = CASE == TD_CV ? y[1] : 0.0, y22 = y2 * y2;
+  // highest order any polynomial asks for
+  const int nTop = max(max(W.nMax[0], W.nMax[1]), W.nMax[2] - 1) + nOffset;
+#pragma unroll 1
+  for (int d = 0; d < NR; d++) {
+    const double Xd = td_x<CASE>(W, y, d), iX = 1.0 / Xd;
+    const cplx IKX = IK * Xd;
+    double sn, cs;
+    sincos(IKX.i, &sn, &cs);
+    const double ep = exp(IKX.r), em = exp(-IKX.r);
+    const cplx e = mk(ep * cs, ep * sn);
+    cplx ER[TD_NER];
+    exprels(nTop, -IKX, mk(em * cs, -(em * sn)), ER);
+#pragma unroll
+    for (int npk = 0; npk < TD_NPK; npk++) {
+#pragma unroll
+      for (int n = 0; n < TD_NWP; n++) {
+        if (n < W.nMin[npk] || n > W.nMax[npk]) continue;
+        // script P (TaylorDuffy.cc:568-634)
+        const double *u = U[npk][d][n];
+        double P;
+        if constexpr (CASE == TD_CT) P = u[T1] + yIn * u[TY1];
+        else if constexpr (CASE == TD_CE)
+          P = u[T1] + u[TY1] * y1 + u[TY12] * y12 + yIn * (u[TY2] + u[TY1Y2] * y1 + u[TY12Y2] * y12);
+        else
+          P = u[T1] + u[TY1] * y1 + u[TY2] * y2 + u[TY12] * y12 + u[TY1Y2] * y1 * y2 + u[TY22] * y22 +
+              u[TY12Y2] * y12 * y2 + u[TY1Y22] * y1 * y22 +
+              yIn * (u[TY2Y3] * y2 + u[TY1Y2Y3] * y1 * y2 + u[TY22Y3] * y22 + u[TY12Y2Y3] * y12 * y2);
+        const int o = n + nOffset;
+        cplx K;
+        if (npk < 2) K = ((1.0 / o) * iX) * ER[o];
+        else if (o < 2) K = mk(0, 0);       // (common triangle: no such power)
+        else K = (iX * iX) * (cmulf(IK, (1.0 / (o - 1)) * ER[o - 1]) - (c_inv.v[o - 2] * iX) * ER[o - 2]);
+        s[npk] = cfma(P * e, K, s[npk]);
       }
-  } else {
-    double y1 = y[0], y12 = y1 * y1, y2 = y[1], y22 = y2 * y2;
-    for (int d = 0; d < 2; d++)
-      for (int n = nMin; n <= nMax; n++) {
-        P[d][n][0] = U[d][n][T1] + U[d][n][TY1] * y1 + U[d][n][TY2] * y2 + U[d][n][TY12] * y12
-                     + U[d][n][TY1Y2] * y1 * y2 + U[d][n][TY22] * y22 + U[d][n][TY12Y2] * y12 * y2
-                     + U[d][n][TY1Y22] * y1 * y22;
-        P[d][n][1] = U[d][n][TY2Y3] * y2 + U[d][n][TY1Y2Y3] * y1 * y2 + U[d][n][TY22Y3] * y22
-                     + U[d][n][TY12Y2Y3] * y12 * y2;
-      }
-  }
-}
-
-// relative exponential ExpRelV3P0 (TaylorDuffy.cc:840-893)
-__device__ cplx sw_exprel(int n, cplx Z)
-{
-  int m;
-  if (Z.i == 0.0) {
-    double X = Z.r, Term, Sum;
-    if (fabs(X) < 0.1) {
-      Sum = 1.0;
-      for (Term = 1.0, m = 1; m < 100; m++) {
-        Term *= X / ((double)(m + n));
-        Sum += Term;
-        if (fabs(Term) < 1.0e-8 * fabs(Sum)) break;
-      }
-      return mk(Sum, 0);
     }
-    Sum = exp(X);
-    for (Term = 1.0, m = 0; m < n; m++) { Sum -= Term; Term *= X / ((double)(m + 1)); }
-    return mk(Sum / Term, 0);
   }
-  cplx Term, Sum;
-  if (sqrt(norm2(Z)) < 0.1) {
-    Sum = Term = mk(1, 0);
-    for (m = 1; m < 100; m++) {
-      Term = Term * (Z / (double)(m + n));
-      Sum += Term;
-      if (norm2(Term) < 1.0e-16 * norm2(Sum)) break;
-    }
-    return Sum;
-  }
-  Sum = cexp_(Z);
-  Term = mk(1, 0);
-  for (m = 0; m < n; m++) { Sum -= Term; Term = Term * (Z / (double)(m + 1)); }
-  return Sum / Term;
-}
-
-// script K of the Helmholtz kernels (TaylorDuffy.cc:896-935)
-__device__ void td_script_k(int WhichK, cplx KParam, double X, int nMin, int nMax, cplx *K)
-{
-  cplx IK = IMUL(KParam), IKX = IK * X, e = cexp_(IKX);
-  if (WhichK == K_HELM) {
-    for (int n = nMin; n <= nMax; n++) K[n] = e * sw_exprel(n, -IKX) / (n * X);
-  } else {
-    cplx ER[10];
-    if ((nMin - 2) < 0 || (nMax - 1) >= 10) {
-      for (int n = 0; n < nMin; n++) K[n] = mk(0, 0);
-      nMin = 2;
-    }
-    for (int n = nMin - 2; n <= nMax - 1; n++) ER[n] = sw_exprel(n, -IKX);
-    for (int n = nMin; n <= nMax; n++)
-      K[n] = e * (IK * ER[n - 1] / ((double)n - 1.0) - ER[n - 2] / (((double)n - 2.0) * X)) / (X * X);
-  }
-}
-
-// TaylorDuffySum (TaylorDuffy.cc:152-258) for the once-integrable
-// (Helmholtz) kernels: f[2 npk], f[2 npk + 1]
-__device__ void td_sum(const TDGeo &W, const double (*U)[TD_NREG][TD_NWP][TD_NMON], const double *y, double *f)
-{
-  int NumRegions, nOffset;
-  double yIn, Jac;
-  if (W.WhichCase == TD_CT) { NumRegions = 3; nOffset = 1; yIn = y[0]; Jac = 1.0; }
-  else if (W.WhichCase == TD_CE) { NumRegions = 6; nOffset = 2; yIn = y[1]; Jac = y[0]; }
-  else { NumRegions = 2; nOffset = 3; yIn = y[2]; Jac = y[1]; }
-  if (Jac == 0.0) { for (int q = 0; q < 2 * W.NumPKs; q++) f[q] = 0.0; return; }
-  double X[TD_NREG];
-  td_x(W, y, X);
-  for (int npk = 0; npk < W.NumPKs; npk++) {
-    const int nMin = W.nMin[npk], nMax = W.nMax[npk];
-    double P[TD_NREG][TD_NWP][2];
-    td_script_p(W, U[npk], nMin, nMax, y, P);
-    cplx K[TD_NREG][8];
-    for (int d = 0; d < NumRegions; d++) td_script_k(W.KIndex[npk], W.k, X[d], nMin + nOffset, nMax + nOffset, K[d]);
-    cplx s = mk(0, 0);
-    for (int n = nMin; n <= nMax; n++)
-      for (int d = 0; d < NumRegions; d++) s += (P[d][n][0] + yIn * P[d][n][1]) * K[d][n + nOffset];
-    s = s * (Jac / (4.0 * M_PI));
-    f[2 * npk] = s.r; f[2 * npk + 1] = s.i;
+  for (int npk = 0; npk < TD_NPK; npk++) {
+    f[2 * npk] = s[npk].r * (Jac / (4.0 * M_PI));
+    f[2 * npk + 1] = s[npk].i * (Jac / (4.0 * M_PI));
   }
 }
 
 // ComputeGeometricParameters (TaylorDuffy.cc:1265-1528) for P = UNITY,
 // PMCHWG1, PMCHWC (the first NumPKs of them): the geometric scalars into W
-// (every lane), and, on lane npk < NumPKs, the Upsilon table of polynomial
-// npk into U[npk] and its lowest and highest nonzero power into nm[npk],
-// nm[TD_NPK + npk]
+// (every lane), the Upsilon table of polynomial npk into U[npk] (lane npk)
+// and its lowest and highest nonzero power into W.nMin, W.nMax
 __device__ void td_geometry(int WhichCase, const double *V1, const double *V2, const double *V3, const double *V2P,
                             const double *V3P, const double *Q, const double *QP, TDGeo &W,
-                            double (*U)[TD_NREG][TD_NWP][TD_NMON], int *nm)
+                            double (*U)[TD_NREG][TD_NWP][TD_NMON])
 {
+  for (int e = threadIdx.x; e < TD_NPK * TD_NREG * TD_NWP * TD_NMON; e += 64) (&U[0][0][0][0])[e] = 0.0;
+  __syncthreads();
   if (WhichCase == TD_CT) { V2P = V2; V3P = V3; }
   else if (WhichCase == TD_CE) V2P = V2;
   double A[3], B[3], AP[3], BP[3], L[3];
@@ -470,9 +424,8 @@ __device__ void td_geometry(int WhichCase, const double *V1, const double *V2, c
     W.AP2 = dot3(AP, AP); W.BP2 = dot3(BP, BP); W.AdAP = dot3(A, AP); W.AdBP = dot3(A, BP);
     W.BdAP = dot3(B, AP); W.BdBP = dot3(B, BP); W.APdBP = dot3(AP, BP);
   }
+  if (threadIdx.x < TD_NPK) {
   const int npk = threadIdx.x;
-  if (npk >= W.NumPKs) return;
-  const int NumRegions = (WhichCase == TD_CV) ? 2 : (WhichCase == TD_CE ? 6 : 3);
   double D[3], DP[3], DeltaD[3], Scr[3], Scr2[3];
   sub3(V1, Q, D); sub3(V1, QP, DP); sub3(QP, Q, DeltaD);
   double C[4] = {0, 0, 0, 0}, M[16], V[4] = {0, 0, 0, 0}, S = 0.0;
@@ -492,12 +445,23 @@ __device__ void td_geometry(int WhichCase, const double *V1, const double *V2, c
     V[0] = -dot3(A, Scr2); V[1] = -dot3(B, Scr2); V[2] = dot3(AP, Scr2); V[3] = dot3(BP, Scr2);
   }
   td_upsilon(WhichCase, C, M, V, S, U[npk]);
-  int nMin = TD_NWP - 1, nMax = -1;
-  for (int n = 0; n < TD_NWP; n++)
-    for (int nr = 0; nr < NumRegions; nr++)
-      for (int q = 0; q < TD_NMON; q++)
-        if (fabs(U[npk][nr][n][q]) > 1.0e-8) { if (n < nMin) nMin = n; if (n > nMax) nMax = n; }
-  nm[npk] = nMin; nm[TD_NPK + npk] = nMax;
+  }
+  __syncthreads();
+  // the powers with a nonzero coefficient, entries over the lanes
+  for (int npk = 0; npk < TD_NPK; npk++) {
+    int mask = 0;
+    for (int e = threadIdx.x; e < TD_NREG * TD_NWP * TD_NMON; e += 64)
+      if (fabs((&U[npk][0][0][0])[e]) > 1.0e-8) mask |= 1 << (e / TD_NMON % TD_NWP);
+    int nMin = TD_NWP - 1, nMax = -1;
+#pragma unroll
+    for (int n = 0; n < TD_NWP; n++)
+      if (__ballot((mask >> n) & 1)) {
+        nMin = min(nMin, n);
+        nMax = n;
+      }
+    W.nMin[npk] = nMin;
+    W.nMax[npk] = nMax;
+  }
 }
 
 // ---------------------------------------------------------------------
@@ -553,8 +517,8 @@ __device__ inline double wave_sum(double v)
 
 // appends the block of points of rule orders m[] whose dimension mi is at
 // its newest level: entry E[ne] (LDS, lane 0), values at vals + nval
-template <typename F>
-__device__ void pc_add(F &f, int dim, const int *m, int mi, PCEntry *E, int &ne, double *vals, int &nval)
+template <int dim, typename F>
+__device__ inline void pc_add(F &f, const int *m, int mi, PCEntry *E, int &ne, double *vals, int &nval)
 {
   if (threadIdx.x == 0) {
     PCEntry &e = E[ne];
@@ -562,12 +526,15 @@ __device__ void pc_add(F &f, int dim, const int *m, int mi, PCEntry *E, int &ne,
   }
   ne++;
   int cnt[3] = {1, 1, 1};
+#pragma unroll
   for (int d = 0; d < dim; d++) cnt[d] = pc_count(m[d], d == mi);
   const int total = cnt[0] * cnt[1] * cnt[2];
   for (int L = threadIdx.x; L < total; L += 64) {
     int l[3] = {0, 0, 0}, rem = L;
+#pragma unroll
     for (int d = dim - 1; d >= 0; d--) { l[d] = rem % cnt[d]; rem /= cnt[d]; }
     double y[3];
+#pragma unroll
     for (int d = 0; d < dim; d++) y[d] = pc_coord(m[d], d == mi, l[d]);
     f(y, vals + (long)(nval + L) * SW_FDIM);
   }
@@ -577,50 +544,54 @@ __device__ void pc_add(F &f, int dim, const int *m, int mi, PCEntry *E, int &ne,
 
 // the rule of order m over the cache, reduced in dimension md (md = dim:
 // none), for md = 0..dim at once: S[md][q], identical on every lane
-__device__ void pc_evals(int dim, const PCEntry *E, int ne, const double *vals, const int *m, double V,
-                         double (*S)[SW_FDIM])
+template <int dim>
+__device__ inline void pc_evals(const PCEntry *E, int ne, const double *vals, const int *m, double V,
+                         double (&S)[dim + 1][SW_FDIM])
 {
 #pragma unroll
-  for (int md = 0; md < 4; md++)
+  for (int md = 0; md <= dim; md++)
 #pragma unroll
     for (int q = 0; q < SW_FDIM; q++) S[md][q] = 0.0;
   for (int c = 0; c < ne; c++) {
     const PCEntry e = E[c];
     const int cm[3] = {e.m0, e.m1, e.m2};
-    bool inc[4];
+    bool inc[dim + 1], any = false;
 #pragma unroll
-    for (int md = 0; md < 4; md++)
-      inc[md] = md <= dim && (e.mi >= dim || cm[e.mi] + (e.mi == md) <= m[e.mi]);
-    if (!(inc[0] || inc[1] || inc[2] || inc[3])) continue;
+    for (int md = 0; md <= dim; md++)
+    {
+      inc[md] = e.mi >= dim || (e.mi == 0 ? cm[0] + (md == 0) <= m[0] : e.mi == 1 ? cm[1] + (md == 1) <= m[1] : cm[2] + (md == 2) <= m[2]);
+      any = any || inc[md];
+    }
+    if (!any) continue;
     int cnt[3] = {1, 1, 1};
+#pragma unroll
     for (int d = 0; d < dim; d++) cnt[d] = pc_count(cm[d], d == e.mi);
     const int total = cnt[0] * cnt[1] * cnt[2];
     for (int L = threadIdx.x; L < total; L += 64) {
       int l[3] = {0, 0, 0}, rem = L;
+#pragma unroll
       for (int d = dim - 1; d >= 0; d--) { l[d] = rem % cnt[d]; rem /= cnt[d]; }
       double wf[3] = {1, 1, 1}, wr[3] = {1, 1, 1};
 #pragma unroll
-      for (int d = 0; d < 3; d++)
-        if (d < dim) {
-          wf[d] = pc_weight(cm[d], d == e.mi, m[d], false, l[d]);
-          wr[d] = pc_weight(cm[d], d == e.mi, m[d], true, l[d]);
-        }
+      for (int d = 0; d < dim; d++) {
+        wf[d] = pc_weight(cm[d], d == e.mi, m[d], false, l[d]);
+        wr[d] = pc_weight(cm[d], d == e.mi, m[d], true, l[d]);
+      }
       const double *v = vals + (long)(e.off + L) * SW_FDIM;
       double vv[SW_FDIM];
 #pragma unroll
       for (int q = 0; q < SW_FDIM; q++) vv[q] = v[q];
 #pragma unroll
-      for (int md = 0; md < 4; md++) {
+      for (int md = 0; md <= dim; md++) {
         if (!inc[md]) continue;
         double wt = V;
         bool use = true;
 #pragma unroll
-        for (int d = 0; d < 3; d++)
-          if (d < dim) {
-            const double w = d == md ? wr[d] : wf[d];
-            if (w < 0) use = false;
-            else wt *= w;
-          }
+        for (int d = 0; d < dim; d++) {
+          const double w = d == md ? wr[d] : wf[d];
+          if (w < 0) use = false;
+          else wt *= w;
+        }
         if (!use) continue;
 #pragma unroll
         for (int q = 0; q < SW_FDIM; q++) S[md][q] += vv[q] * wt;
@@ -628,37 +599,35 @@ __device__ void pc_evals(int dim, const PCEntry *E, int ne, const double *vals, 
     }
   }
 #pragma unroll
-  for (int md = 0; md < 4; md++)
-    if (md <= dim)
+  for (int md = 0; md <= dim; md++)
 #pragma unroll
-      for (int q = 0; q < SW_FDIM; q++) S[md][q] = wave_sum(S[md][q]);
+    for (int q = 0; q < SW_FDIM; q++) S[md][q] = wave_sum(S[md][q]);
 }
 
 // the integral into val[SW_FDIM] (every lane); vals: the job's value
 // cache in scratch memory, E: its entries in LDS
-template <typename F>
-__device__ void pcubature_wave(F &f, int dim, double *vals, PCEntry *E, double *val)
+template <int dim, typename F>
+__device__ inline void pcubature_wave(F &f, double *vals, PCEntry *E, double *val)
 {
   int m[3] = {0, 0, 0};
   double V = 1.0;
   for (int d = 0; d < dim; d++) V *= 0.5;
   int ne = 0, nval = 0;
   long numEval = 0;
-  pc_add(f, dim, m, dim, E, ne, vals, nval);
+  pc_add<dim>(f, m, dim, E, ne, vals, nval);
   for (;;) {
-    double S[4][SW_FDIM];
-    pc_evals(dim, E, ne, vals, m, V, S);
+    double S[dim + 1][SW_FDIM];
+    pc_evals<dim>(E, ne, vals, m, V, S);
     double err[SW_FDIM];
 #pragma unroll
     for (int q = 0; q < SW_FDIM; q++) {
-      val[q] = dim == 1 ? S[1][q] : (dim == 2 ? S[2][q] : S[3][q]);
+      val[q] = S[dim][q];
       err[q] = 0.0;
     }
     int mi = 0;
     double maxerr = 0.0;
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
-      if (i >= dim) continue;
+    for (int i = 0; i < dim; i++) {
       double emax = 0.0;
 #pragma unroll
       for (int q = 0; q < SW_FDIM; q++) {
@@ -673,12 +642,15 @@ __device__ void pcubature_wave(F &f, int dim, double *vals, PCEntry *E, double *
     for (int q = 0; q < SW_FDIM; q++)
       if (err[q] > 0.0 && err[q] > fabs(val[q]) * TD_RELTOL) conv = false;
     if (conv || numEval > TD_MAXEVAL) break;
-    m[mi] += 1;
-    if (m[mi] >= PC_M) break;     // not reached within TD_MAXEVAL points
     int nb = 1;
-    for (int d = 0; d < dim; d++) nb *= pc_count(m[d], d == mi);
-    if (ne >= PC_MAXENT || nval + nb > PC_MAXVAL) { m[mi] -= 1; break; }
-    pc_add(f, dim, m, mi, E, ne, vals, nval);
+    bool top = false;
+#pragma unroll
+    for (int d = 0; d < dim; d++) {
+      if (d == mi) { m[d] += 1; top = m[d] >= PC_M; }   // (top: not reached within TD_MAXEVAL points)
+      nb *= pc_count(m[d], d == mi);
+    }
+    if (top || ne >= PC_MAXENT || nval + nb > PC_MAXVAL) break;
+    pc_add<dim>(f, m, mi, E, ne, vals, nval);
     numEval += nb;
   }
 }
@@ -758,68 +730,80 @@ __device__ void sw_hocub(const NearPair &P, cplx k, int needH1, cplx *H0, cplx *
 
 static_assert(SW_SLAB == SCUFFX_SW_SLAB, "scratch slab size");
 
-struct TDFun {
+template <int CASE> struct TDFun {
   const TDGeo *W;
   const double (*U)[TD_NREG][TD_NWP][TD_NMON];
-  __device__ void operator()(const double *y, double *out) const { td_sum(*W, U, y, out); }
+  __device__ void operator()(const double *y, double *out) const { td_sum<CASE>(*W, U, y, out); }
 };
 
-// one wave (block of 64) per job; kind 0: no-common-vertex near pair (all
-// 9 combinations), 1: common-edge/vertex near pair, one (Qa, Qb).  A
+// one wave (block of 64) per job, as many waves as are resident, each taking
+// every gridDim-th job (a launch per 4096 jobs waited 240 times for its last
+// one).  KIND SW_SEP: no-common-vertex near pairs (all 9 combinations),
+// TD_CV, TD_CE, TD_CT: pairs with one, two or three common vertices, one
+// (Qa, Qb) a job; a kernel each, since their registers and tables differ.  A
 // Taylor-Duffy job keeps its Upsilon tables and cache entries in LDS and
 // its cached integrand values in a slab of scratch memory.
-__global__ void __launch_bounds__(64)
-k_sw(const SWJob *jobs, int job0, int njobs, const NearPair *nps, const double *V, const int *PVI, int nreg,
-     const RegionK *regs, int needH1, double *HN, double *HS, double *scratch)
+template <int KIND>
+__global__ void __launch_bounds__(64, 2)
+k_sw(const SWJob *jobs, int njobs, const NearPair *nps, int nreg, const RegionK *regs, int needH1, double *HN,
+     double *scratch)
 {
-  __shared__ double sU[TD_NPK][TD_NREG][TD_NWP][TD_NMON];
-  __shared__ PCEntry sE[PC_MAXENT];
-  __shared__ int sNm[2 * TD_NPK];
-  const int t = blockIdx.x;
-  if (t >= njobs) return;
-  const SWJob J = jobs[job0 + t];
-  const cplx k = regs[J.region].k;
-  const int stride = needH1 ? 4 : 2;
-  const int lane = threadIdx.x;
-  if (J.kind == 0) {
-    cplx H0[9], H1[9];
-    sw_hocub(nps[J.pair], k, needH1, H0, H1);
+  const int stride = needH1 ? 4 : 2, lane = threadIdx.x;
+  for (int t = blockIdx.x; t < njobs; t += gridDim.x) {
+    const SWJob J = jobs[t];
+    const cplx k = regs[J.region].k;
+    const NearPair &P = nps[J.pair];
     double *o = HN + ((long long)J.pair * nreg + J.region) * 9 * stride;
-    if (lane == 0)
-      for (int q = 0; q < 9; q++) {
-        o[q * stride] = H0[q].r; o[q * stride + 1] = H0[q].i;
-        if (needH1) { o[q * stride + 2] = H1[q].r; o[q * stride + 3] = H1[q].i; }
+    if constexpr (KIND == SW_SEP) {
+      cplx H0[9], H1[9];
+      sw_hocub(P, k, needH1, H0, H1);
+      if (lane == 0)
+        for (int q = 0; q < 9; q++) {
+          o[q * stride] = H0[q].r; o[q * stride + 1] = H0[q].i;
+          if (needH1) { o[q * stride + 2] = H1[q].r; o[q * stride + 3] = H1[q].i; }
+        }
+    } else {
+      __shared__ double sU[TD_NPK][TD_NREG][TD_NWP][TD_NMON];
+      __shared__ PCEntry sE[PC_MAXENT];
+      TDGeo W;
+      W.k = k;
+      W.WhichCase = KIND;
+      const int a = J.q / 3, b = J.q % 3;
+      td_geometry(KIND, P.Va, P.Va + 3, P.Va + 6, P.Vb + 3, P.Vb + 6, P.Qa + 3 * a, P.Qb + 3 * b, W, sU);
+      double R[SW_FDIM];
+      TDFun<KIND> f{&W, sU};
+      pcubature_wave<4 - KIND>(f, scratch + (long long)blockIdx.x * SW_SLAB, sE, R);
+      if (lane == 0) {
+        cplx H0 = mk(R[2], R[3]) - 4.0 * mk(R[0], R[1]) / (k * k), H1 = mk(R[4], R[5]);
+        o += J.q * stride;
+        o[0] = H0.r; o[1] = H0.i;
+        if (needH1) { o[2] = H1.r; o[3] = H1.i; }
       }
-    return;
+      __syncthreads();   // the next job's tables overwrite this one's
+    }
   }
-  double *vals = scratch + (long long)t * SW_SLAB;
-  TDGeo W;
-  W.k = k;
-  const int a = J.q / 3, b = J.q % 3;
-  const NearPair &P = nps[J.pair];
-  W.WhichCase = P.ncv; W.NumPKs = 3;
-  W.KIndex[0] = K_HELM; W.KIndex[1] = K_HELM; W.KIndex[2] = K_GRADHELM;
-  td_geometry(P.ncv, P.Va, P.Va + 3, P.Va + 6, P.Vb + 3, P.Vb + 6, P.Qa + 3 * a, P.Qb + 3 * b, W, sU, sNm);
-  __syncthreads();
-  for (int npk = 0; npk < TD_NPK; npk++) { W.nMin[npk] = sNm[npk]; W.nMax[npk] = sNm[TD_NPK + npk]; }
-  TDFun f{&W, sU};
-  double R[SW_FDIM];
-  pcubature_wave(f, 4 - P.ncv, vals, sE, R);
-  if (lane == 0) {
-    cplx H0 = mk(R[2], R[3]) - 4.0 * mk(R[0], R[1]) / (k * k), H1 = mk(R[4], R[5]);
-    double *o = HN + ((long long)J.pair * nreg + J.region) * 9 * stride + J.q * stride;
-    o[0] = H0.r; o[1] = H0.i;
-    if (needH1) { o[2] = H1.r; o[3] = H1.i; }
-  }
+}
+
+template <int KIND>
+static hipError_t sw_kind(hipStream_t stream, const SWJob *jobs, int njobs, const NearPair *nps, int nreg,
+                          const RegionK *regs, int needH1, double *HN, double *scratch, int slabs)
+{
+  if (njobs <= 0) return hipSuccess;
+  int dev = 0, ncu = 0, perCU = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_sw<KIND>, 64, 0);
+  if (e != hipSuccess) return e;
+  const int grid = std::min(std::min(njobs, slabs), std::max(1, ncu * perCU));
+  hipLaunchKernelGGL(k_sw<KIND>, dim3(grid), dim3(64), 0, stream, jobs, njobs, nps, nreg, regs, needH1, HN, scratch);
+  return hipGetLastError();
 }
 
 static bool g_sw_ready[64] = {false};
 
-hipError_t launch_sw(hipStream_t stream, const SWJob *jobs, int njobs, const NearPair *nps, const double *V,
-                     const int *PVI, int nreg, const RegionK *regs, int needH1, double *HN, double *HS,
-                     double *scratch, int chunk)
+hipError_t launch_sw(hipStream_t stream, const SWJob *jobs, const int njobs[4], const NearPair *nps, int nreg,
+                     const RegionK *regs, int needH1, double *HN, double *scratch, int slabs)
 {
-  if (njobs <= 0) return hipSuccess;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return hipErrorInvalidDevice;
   if (!g_sw_ready[dev & 63]) {
@@ -857,14 +841,12 @@ hipError_t launch_sw(hipStream_t stream, const SWJob *jobs, int njobs, const Nea
     if (e != hipSuccess) return e;
     g_sw_ready[dev & 63] = true;
   }
-  for (int j0 = 0; j0 < njobs; j0 += chunk) {
-    int n = std::min(chunk, njobs - j0);
-    hipLaunchKernelGGL(k_sw, dim3(n), dim3(64), 0, stream, jobs, j0, n, nps, V, PVI, nreg, regs, needH1,
-                       HN, HS, scratch);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const SWJob *j1 = jobs + njobs[0], *j2 = j1 + njobs[1], *j3 = j2 + njobs[2];
+  hipError_t e = sw_kind<SW_SEP>(stream, jobs, njobs[0], nps, nreg, regs, needH1, HN, scratch, slabs);
+  if (e == hipSuccess) e = sw_kind<TD_CV>(stream, j1, njobs[1], nps, nreg, regs, needH1, HN, scratch, slabs);
+  if (e == hipSuccess) e = sw_kind<TD_CE>(stream, j2, njobs[2], nps, nreg, regs, needH1, HN, scratch, slabs);
+  if (e == hipSuccess) e = sw_kind<TD_CT>(stream, j3, njobs[3], nps, nreg, regs, needH1, HN, scratch, slabs);
+  return e;
 }
 
 }  // namespace scuffx

@@ -264,25 +264,30 @@ int Assembler::vertex_gradient(cdouble omega, const double2 *M, long ldm, const 
   double *dHN = sc.alloc<double>(hnTotal), *dHS = sc.alloc<double>(hsTotal);
   if (!dHN || !dHS) return bad(-2, "device allocation failed");
   {
-    // Taylor-Duffy jobs, one launch per surface
-    const int chunk = 4096;
+    // Taylor-Duffy jobs, one set of launches per surface
+    const int slabs = 4096;
     double *scr = nullptr;
     bool needSW = false;
     for (int s = 0; s < NS; s++) needSW = needSW || !sj[s].np.empty();
-    if (needSW && !(scr = sc.alloc<double>((size_t)chunk * SCUFFX_SW_SLAB))) return bad(-2, "device allocation failed");
+    if (needSW && !(scr = sc.alloc<double>((size_t)slabs * SCUFFX_SW_SLAB))) return bad(-2, "device allocation failed");
     for (int s = 0; s < NS; s++) {
       if (sj[s].np.empty()) continue;
       const int b = bidx(s, s), nr = nreg[b];
       std::vector<SWJob> jobs;
       jobs.reserve(sj[s].np.size() * nr * 9);
-      for (int n = 0; n < (int)sj[s].np.size(); n++)
-        for (int r = 0; r < nr; r++)
-          for (int q = 0; q < 9; q++) jobs.push_back(SWJob{n, r, q, 1});
+      int njobs[4] = {0, 0, 0, 0};
+      for (int kind = 1; kind < 4; kind++) {
+        const size_t j0 = jobs.size();
+        for (int n = 0; n < (int)sj[s].np.size(); n++)
+          if (sj[s].np[n].ncv == kind)
+            for (int r = 0; r < nr; r++)
+              for (int q = 0; q < 9; q++) jobs.push_back(SWJob{n, r, q, kind});
+        njobs[kind] = (int)(jobs.size() - j0);
+      }
       NearPair *dnp = sc.put(sj[s].np);
       SWJob *djobs = sc.put(jobs);
       if (!dnp || !djobs) return bad(-2, "device allocation failed");
-      if (launch_sw(stream, djobs, (int)jobs.size(), dnp, nullptr, nullptr, nr, drk + 2 * b, stride == 4,
-                    dHN + sj[s].base, nullptr, scr, chunk) != hipSuccess)
+      if (launch_sw(stream, djobs, njobs, dnp, nr, drk + 2 * b, stride == 4, dHN + sj[s].base, scr, slabs) != hipSuccess)
         return bad(-3, "Taylor-Duffy kernel failed");
     }
   }
