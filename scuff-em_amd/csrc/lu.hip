@@ -1513,14 +1513,16 @@ static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, b
                            int *perm_buf = nullptr, bool perm_ready = false);
 
 // Inverses of the diagonal 64x64 blocks of L (unit lower, blockIdx.y = 0)
-// and U (blockIdx.y = 1, as the transpose of a lower triangle), identity
-// past row n: every block step of a one-right-hand-side solve is then a
-// product.  One workgroup a block, a wave for 16 columns of the inverse, a
-// lane for a row; step k passes x_k of every column by lane reads.  Bound:
-// issue of the 64 x 16 lane reads and updates.  A column per thread of one
-// wave, its sums from LDS, took 100 us for each triangle, this takes 59 us
-// for both in complex128 (order 2501; the first 16 (q + 1)
-// columns only in steps 16 q ..: 78 us with every column in every step).
+// and U (blockIdx.y = 1), identity past row n: every block step of a
+// one-right-hand-side solve is then a product.  Columns of the inverse by
+// substitution, so that L X and U X, not X L and X U, are the identity to
+// rounding (the transpose of U^T's inverse converged ten times slower in the
+// refinement).  One workgroup a block, a wave for 16 columns of the inverse, a
+// lane for a row; a step passes one row's values of every column by lane
+// reads.  Bound: issue of the lane reads and updates.  A column per thread of
+// one wave, its sums from LDS, took 100 us for each triangle, this takes 59 us
+// for both in complex128 (order 2501; the first 16 (q + 1) columns only in
+// steps 16 q ..: 78 us with every column in every step).
 #define TB 64
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -1532,6 +1534,7 @@ k_tri_inv(const T *LU, long lda, long n, T *invL, T *invU, long sa, long sinv)
   const long z = blockIdx.z, kb = (long)blockIdx.x * TB;   // instance z of a batch
   const int bs = (int)std::min<long>(TB, n - kb);
   LU += z * sa + kb + kb * lda;
+  // the rows and columns of U in reverse: a lower triangle as well
   {
     T v[16];
 #pragma unroll
@@ -1541,7 +1544,7 @@ k_tri_inv(const T *LU, long lda, long n, T *invL, T *invU, long sa, long sinv)
     for (int u = 0; u < 16; u++) {
       const int c = wave + 4 * u;
       if (lane >= bs || c >= bs) v[u] = lane == c ? unit_v<T>() : zero_v<T>();
-      if (up) D[c][lane] = v[u]; else D[lane][c] = v[u];
+      if (up) D[TB - 1 - lane][TB - 1 - c] = v[u]; else D[lane][c] = v[u];
     }
   }
   __syncthreads();
@@ -1571,16 +1574,9 @@ k_tri_inv(const T *LU, long lda, long n, T *invL, T *invU, long sa, long sinv)
   steps(std::integral_constant<int, 2>{});
   steps(std::integral_constant<int, 3>{});
   T *o = (up ? invU : invL) + z * sinv + (long)blockIdx.x * TB * TB;
-  if (up) {
-    __syncthreads();
+  const int r = up ? TB - 1 - lane : lane;
 #pragma unroll
-    for (int u = 0; u < 16; u++) D[wave + 4 * u][lane] = y[u];
-    __syncthreads();
-    for (int u = 0; u < 16; u++) o[lane + (wave + 4 * u) * TB] = D[lane][wave + 4 * u];
-  } else {
-#pragma unroll
-    for (int u = 0; u < 16; u++) o[lane + (wave + 4 * u) * TB] = y[u];
-  }
+  for (int u = 0; u < 16; u++) o[r + (up ? TB - 1 - wave - 4 * u : wave + 4 * u) * TB] = y[u];
 }
 
 template <typename T>
