@@ -525,53 +525,33 @@ int Assembler::build_fippi(hipStream_t stream)
   }
   const int nt = (int)todo.size();
   if (nt > 0) {
-    int *d_counter = nullptr, *d_ovf = nullptr;
-    HIPCHK(hipMalloc(&d_counter, sizeof(int)));
-    HIPCHK(hipMalloc(&d_ovf, sizeof(int) * nj));
+    // separated pairs first: some of them split regions thousands of times,
+    // and whatever starts last ends last
+    std::stable_partition(todo.begin(), todo.end(), [&](int j) { return jobs_[j].ncv == 0; });
+    // heaps large enough for the whole evaluation budget (1e6 points, 66 per
+    // split), one per resident workgroup (four per CU, 9.5 MB each), fewer if
+    // there is no memory for them
+    const int cap = 15360;
+    int slots = std::min(1024, nt);
+    Scratch sc;
+    int *d_counter = sc.alloc<int>(1), *d_ovf = sc.alloc<int>(nj), *d_todo = sc.put(todo);
+    double *hd = nullptr;
+    while (!(hd = sc.alloc<double>((size_t)cap * 76 * slots)) && slots > 1) {
+      hipGetLastError();
+      slots = (slots + 1) / 2;
+    }
+    double *hk = sc.alloc<double>((size_t)cap * slots);
+    int *hs = sc.alloc<int>((size_t)cap * slots);
+    if (!d_counter || !d_ovf || !d_todo || !hd || !hk || !hs) { err_ = "device allocation failed"; return -2; }
     HIPCHK(hipMemsetAsync(d_ovf, 0, sizeof(int) * nj, stream));
     HIPCHK(hipMemsetAsync(d_counter, 0, sizeof(int), stream));
-    // pass 1: small heaps (4096 regions) for every job to compute, 2048 waves
-    int cap1 = 4096, slots1 = std::min(2048, std::max(1, nt));
-    double *hd = nullptr, *hk = nullptr;
-    int *hs = nullptr, *d_todo = nullptr;
-    if (nt < nj) {
-      HIPCHK(hipMalloc(&d_todo, sizeof(int) * nt));
-      HIPCHK(hipMemcpy(d_todo, todo.data(), sizeof(int) * nt, hipMemcpyHostToDevice));
-    }
-    HIPCHK(hipMalloc(&hd, sizeof(double) * (size_t)cap1 * 76 * slots1));
-    HIPCHK(hipMalloc(&hk, sizeof(double) * (size_t)cap1 * slots1));
-    HIPCHK(hipMalloc(&hs, sizeof(int) * (size_t)cap1 * slots1));
     int tok = prof_begin(stream, PK_FIPPI);
-    HIPCHK(launch_fippi(stream, d_jobs_, nt, d_records_, hd, hs, hk, cap1, slots1, d_counter, d_ovf, d_todo));
+    HIPCHK(launch_fippi(stream, d_jobs_, nt, d_records_, hd, hs, hk, cap, slots, d_counter, d_ovf, d_todo));
     prof_end(stream, tok, 0.0);
     std::vector<int> ovf(nj);
     HIPCHK(hipMemcpyAsync(ovf.data(), d_ovf, sizeof(int) * nj, hipMemcpyDeviceToHost, stream));
     HIPCHK(hipStreamSynchronize(stream));
-    hipFree(hd); hipFree(hk); hipFree(hs); hipFree(d_todo);
-    std::vector<int> redo;
-    for (int j = 0; j < nj; j++) if (ovf[j]) redo.push_back(j);
-    if (!redo.empty()) {
-      // pass 2: the jobs that outgrew the small heap, heaps large enough for
-      // the whole evaluation budget (1e6 points / 66 per split), up to 1024
-      // waves (about 20 MB of heap each)
-      int cap2 = 32768, slots2 = std::min<int>(1024, (int)redo.size());
-      int *d_list = nullptr;
-      HIPCHK(hipMalloc(&d_list, sizeof(int) * redo.size()));
-      HIPCHK(hipMemcpyAsync(d_list, redo.data(), sizeof(int) * redo.size(), hipMemcpyHostToDevice, stream));
-      HIPCHK(hipMemsetAsync(d_counter, 0, sizeof(int), stream));
-      HIPCHK(hipMemsetAsync(d_ovf, 0, sizeof(int) * nj, stream));
-      HIPCHK(hipMalloc(&hd, sizeof(double) * (size_t)cap2 * 76 * slots2));
-      HIPCHK(hipMalloc(&hk, sizeof(double) * (size_t)cap2 * slots2));
-      HIPCHK(hipMalloc(&hs, sizeof(int) * (size_t)cap2 * slots2));
-      tok = prof_begin(stream, PK_FIPPI);
-      HIPCHK(launch_fippi(stream, d_jobs_, (int)redo.size(), d_records_, hd, hs, hk, cap2, slots2, d_counter, d_ovf, d_list));
-      prof_end(stream, tok, 0.0);
-      HIPCHK(hipMemcpyAsync(ovf.data(), d_ovf, sizeof(int) * nj, hipMemcpyDeviceToHost, stream));
-      HIPCHK(hipStreamSynchronize(stream));
-      hipFree(hd); hipFree(hk); hipFree(hs); hipFree(d_list);
-      for (int j = 0; j < nj; j++) if (ovf[j]) { err_ = "FIPPI cubature exceeded its region budget"; hipFree(d_counter); hipFree(d_ovf); return -4; }
-    }
-    hipFree(d_counter); hipFree(d_ovf);
+    for (int j = 0; j < nj; j++) if (ovf[j]) { err_ = "FIPPI cubature exceeded its region budget"; return -4; }
     if (prof_enabled()) prof_collect();
     // the new records join the process-wide cache (StoreCache writes them)
     HIPCHK(hipMemcpy(rec.data(), d_records_, sizeof(double) * SCUFFX_QIF_LEN * nj, hipMemcpyDeviceToHost));

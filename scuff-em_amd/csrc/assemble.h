@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -10,8 +11,35 @@
 #include "fippi_cache.h"
 #include "geometry.h"
 #include "vgrad.h"
+#include "ws.h"
 
 namespace scuffx {
+
+// device buffers of one call, freed on every way out
+struct Scratch {
+  std::vector<void *> ptrs;
+  ~Scratch()
+  {
+    if (hip_down()) return;
+    for (void *p : ptrs) hipFree(p);
+  }
+  template <typename T>
+  T *alloc(size_t n)
+  {
+    void *p = nullptr;
+    if (hipMalloc(&p, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) return nullptr;
+    ptrs.push_back(p);
+    return (T *)p;
+  }
+  template <typename T>
+  T *put(const std::vector<T> &h)
+  {
+    T *d = alloc<T>(h.size());
+    if (d && !h.empty() && hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice) != hipSuccess)
+      return nullptr;
+    return d;
+  }
+};
 
 struct DevSurface {
   double *V = nullptr;

@@ -1,5 +1,5 @@
 // kern_fippi.hip -- frequency-independent panel-panel integrals (FIPPIs)
-// by h-adaptive cubature, one wavefront per unique panel-pair job.
+// by h-adaptive cubature, one workgroup per unique panel-pair job.
 //
 // Restates the serial h-adaptive scheme of libs/libSGJC/hcubature.c
 // (:455-615 Genz-Malik 7/5 rule for 2-D/3-D, :619-758 Gauss-Kronrod 15
@@ -10,11 +10,12 @@
 //   ncv > 0: the 1-D (common edge) / 2-D (common vertex) Taylor-Duffy
 //            integrand of QIFIPPITaylorDuffyV2P0.cc:91-221, :329-900
 //            (ABSTOL 0, RELTOL 1e-5, MAXFEVALS 1e4)
-// Per iteration the lanes evaluate the 2 x (15|17|33) rule points of
-// the two halves of the split region in parallel into LDS; lanes 0..32
-// then form each function's rule sums, lane 0 keeps the heap (in HBM,
-// one slab per wave slot).  Heap order, running totals and the final
-// re-summation follow the reference exactly.
+// Two waves a job: per iteration each evaluates the 15, 17 or 33 rule points
+// of one half of the split region in parallel into LDS, its lanes 0..32
+// then form each function's rule sums, and one lane keeps the heap, whose
+// upper levels lie in LDS (the rest and the region records in HBM, one slab
+// per workgroup).  Heap order, running totals and the final re-summation
+// follow the reference exactly.
 #include <hip/hip_runtime.h>
 
 #include "bem.h"
@@ -27,6 +28,7 @@ namespace scuffx {
 struct FipW {
   // ncv = 0
   double V0[3], A[3], B[3], V0P[3], AP[3], BP[3];
+  double a, a2, a3;              // |BP| and its powers
   // ncv > 0
   double tA[3], tB[3], tAP[3], tBP[3];
   double V0xAP[3], V0xBP[3], AxV0[3], BxV0[3], AxAP[3], AxBP[3], BxAP[3], BxBP[3];
@@ -38,16 +40,15 @@ struct FipW {
 __device__ void cfd3(const FipW &W, const double *x, double *fval)
 {
   double u = x[0], v = u * x[1], up = x[2];
-  double X[3], Y[3], Z[3], BPdY = 0, Y2 = 0, a2 = 0;
+  double X[3], Y[3], Z[3], BPdY = 0, Y2 = 0;
   for (int m = 0; m < 3; m++) {
     X[m] = W.V0[m] + u * W.A[m] + v * W.B[m];
     Z[m] = W.V0P[m] + up * W.AP[m];
     Y[m] = X[m] - Z[m];
-    a2 += W.BP[m] * W.BP[m];
     BPdY += W.BP[m] * Y[m];
     Y2 += Y[m] * Y[m];
   }
-  double a = sqrt(a2), a3 = a * a2;
+  const double a = W.a, a2 = W.a2, a3 = W.a3;
   double vp0 = -BPdY / a2, vp02 = vp0 * vp0, vp03 = vp02 * vp0, vp04 = vp03 * vp0;
   double b2 = Y2 / a2 - vp02;
   double OneRM3, vpRM3, OneRM1, vpRM1, OneR1, vpR1, OneR2, vpR2;
@@ -543,38 +544,53 @@ __device__ void rule_sums(int dim, int j, const double *buf, double vol, double 
 }
 
 // ------------------------------ heap ----------------------------------
-struct HeapRef { double *key; int *slot; };
+// binary max-heap of (error, region), entries below HEAP_LDS in LDS: a level
+// of a pop is a dependent read of two keys
+#define HEAP_LDS 2000
+struct HeapRef {
+  double *lkey, *gkey;
+  unsigned short *lslot;
+  int *gslot;
+  __device__ double key(int i) const { return i < HEAP_LDS ? lkey[i] : gkey[i]; }
+  __device__ int slot(int i) const { return i < HEAP_LDS ? (int)lslot[i] : gslot[i]; }
+  __device__ void set(int i, double k, int s) const
+  {
+    if (i < HEAP_LDS) { lkey[i] = k; lslot[i] = (unsigned short)s; }
+    else { gkey[i] = k; gslot[i] = s; }
+  }
+};
 
-__device__ void heap_push(HeapRef h, int &n, double key, int slot)
+__device__ inline void heap_push(const HeapRef &h, int &n, double key, int slot)
 {
   int ins = n++;
   while (ins) {
-    int parent = (ins - 1) / 2;
-    if (key <= h.key[parent]) break;
-    h.key[ins] = h.key[parent];
-    h.slot[ins] = h.slot[parent];
+    const int parent = (ins - 1) / 2;
+    const double pk = h.key(parent);
+    if (key <= pk) break;
+    h.set(ins, pk, h.slot(parent));
     ins = parent;
   }
-  h.key[ins] = key;
-  h.slot[ins] = slot;
+  h.set(ins, key, slot);
 }
 
-__device__ int heap_pop(HeapRef h, int &n)
+__device__ inline int heap_pop(const HeapRef &h, int &n)
 {
-  int ret = h.slot[0];
-  int i = 0, nn = --n, child;
-  h.key[0] = h.key[nn];
-  h.slot[0] = h.slot[nn];
+  const int ret = h.slot(0), nn = --n;
+  const double key = h.key(nn);
+  const int slot = h.slot(nn);
+  int i = 0, child;
   while ((child = i * 2 + 1) < nn) {
-    int largest;
-    if (h.key[child] <= h.key[i]) largest = i; else largest = child;
-    if (++child < nn && h.key[largest] < h.key[child]) largest = child;
+    // (both children read at once; the second counts only below nn)
+    const double k1 = h.key(child), k2 = child + 1 < nn ? h.key(child + 1) : k1;
+    int largest = i;
+    double kl = key;
+    if (k1 > kl) { largest = child; kl = k1; }
+    if (child + 1 < nn && kl < k2) { largest = child + 1; kl = k2; }
     if (largest == i) break;
-    double tk = h.key[i]; int ts = h.slot[i];
-    h.key[i] = h.key[largest]; h.slot[i] = h.slot[largest];
-    h.key[largest] = tk; h.slot[largest] = ts;
+    h.set(i, kl, h.slot(largest));
     i = largest;
   }
+  h.set(i, key, slot);
   return ret;
 }
 
@@ -588,6 +604,10 @@ __device__ void setup_w(const FippiJob &J, FipW &W)
       W.V0[m] = a0[m]; W.A[m] = a1[m] - a0[m]; W.B[m] = a2[m] - a1[m];
       W.V0P[m] = b0[m]; W.AP[m] = b1[m] - b0[m]; W.BP[m] = b2[m] - b1[m];
     }
+    W.a2 = 0;
+    for (int m = 0; m < 3; m++) W.a2 += W.BP[m] * W.BP[m];
+    W.a = sqrt(W.a2);
+    W.a3 = W.a * W.a2;
     W.ce = 0;
     return;
   }
@@ -608,169 +628,217 @@ __device__ void setup_w(const FippiJob &J, FipW &W)
 }
 
 // ------------------------------ kernel --------------------------------
-// one 64-lane block per wave slot; jobs pulled from a counter
-__global__ void __launch_bounds__(64)
+// largest of the wave's values (at least 0), in every lane
+__device__ inline double wave_max(double v)
+{
+  for (int s = 32; s >= 1; s >>= 1) v = fmax(v, __shfl_xor(v, s, 64));
+  return v;
+}
+
+// one workgroup of two waves per slot; jobs pulled from a counter.  Bound:
+// the chain of a job's region splits (up to 15000 for nearly touching
+// panels), FIPNUM
+// LDS: 40 KB, four workgroups on a CU, as many as the registers allow.
+__global__ void __launch_bounds__(128, 2)
 k_fippi(const FippiJob *jobs, int njobs, const int *jobList, double *records,
         double *heapData, int *heapSlot, double *heapKey, int cap, int *counter, int *overflow)
 {
-  __shared__ double buf[66 * NF];
-  __shared__ double dpart[2][NF][3];
+  __shared__ double buf[2][33 * NF];
+  __shared__ double dpart[2][3][NF];
   __shared__ double sreg[2][8];     // center[3] half[3] vol split for A, B
   __shared__ double eA[2][NF], rA[2][NF];
-  __shared__ int s_job, s_pop, s_slotB;
-  __shared__ int s_stop;
+  __shared__ double hkey[HEAP_LDS];
+  __shared__ unsigned short hslot[HEAP_LDS];
+  __shared__ double s_em[2];
+  __shared__ int s_job, s_pop, s_nh;
   // the job's constants, the same for every lane: in LDS, not in each
   // lane's registers
   __shared__ FipW sW;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, rg = threadIdx.x >> 6;
   double *data = heapData + (long long)blockIdx.x * cap * REC;
-  HeapRef H;
-  H.key = heapKey + (long long)blockIdx.x * cap;
-  H.slot = heapSlot + (long long)blockIdx.x * cap;
+  const HeapRef H{hkey, heapKey + (long long)blockIdx.x * cap, hslot, heapSlot + (long long)blockIdx.x * cap};
 
   for (;;) {
-    if (lane == 0) s_job = atomicAdd(counter, 1);
+    if (threadIdx.x == 0) s_job = atomicAdd(counter, 1);
     __syncthreads();
-    int jj = s_job;
+    const int jj = s_job;
     if (jj >= njobs) break;
-    int job = jobList ? jobList[jj] : jj;
+    const int job = jobList ? jobList[jj] : jj;
     const FippiJob &J = jobs[job];
-    if (lane == 0) setup_w(J, sW);
+    if (threadIdx.x == 0) setup_w(J, sW);
     __syncthreads();
     const FipW &W = sW;
     const int dim = (J.ncv == 0) ? 3 : (W.ce ? 1 : 2);
     const int npts = (dim == 1) ? 15 : 1 + 4 * dim + 2 * dim * (dim - 1) + (1 << dim);
     const long maxEval = (J.ncv == 0) ? 1000000 : 10000;
     const double reqAbs = (J.ncv == 0) ? 1.0e-10 : 0.0, reqRel = (J.ncv == 0) ? 1.0e-6 : 1.0e-5;
-    // running totals held by lanes 0..32
+    // the rule on this wave's region sreg[rg]: values and errors into eA, rA,
+    // the largest error into s_em, the split dimension into sreg[rg][7]
+    auto rule = [&]() __attribute__((always_inline)) {
+      if (lane < npts) {
+        double x[3], f[NF];
+        rule_point(dim, lane, sreg[rg], sreg[rg] + 3, x);
+        integrand(W, x, f);
+#pragma unroll
+        for (int q = 0; q < NF; q++) buf[rg][lane * NF + q] = f[q];
+      }
+      __syncthreads();
+      double e = 0.0;
+      if (lane < NF) {
+        double v, d[3] = {0, 0, 0};
+        rule_sums(dim, lane, buf[rg], sreg[rg][6], &v, &e, d);
+        eA[rg][lane] = v;
+        rA[rg][lane] = e;
+#pragma unroll
+        for (int i = 0; i < 3; i++) dpart[rg][i][lane] = d[i];
+      }
+      const double em = wave_max(e);
+      __syncthreads();
+      // the functions' fourth differences summed in order, a lane per dimension
+      double ds = 0.0;
+      if (lane < dim) {
+#pragma unroll
+        for (int q = 0; q < NF; q++) ds += dpart[rg][lane][q];
+      }
+      const double d0 = __shfl(ds, 0), d1 = __shfl(ds, 1), d2 = __shfl(ds, 2);
+      if (lane == 0) {
+        double mx = 0;
+        int sd = 0;
+        if (d0 > mx) { mx = d0; sd = 0; }
+        if (dim > 1 && d1 > mx) { mx = d1; sd = 1; }
+        if (dim > 2 && d2 > mx) { mx = d2; sd = 2; }
+        sreg[rg][7] = dim == 1 ? 0 : sd;
+        s_em[rg] = em;
+      }
+      __syncthreads();
+    };
+    // running totals of function `lane` held by lanes 0..32 of both waves
     double totV = 0.0, totE = 0.0;
-    int n = 0, nused = 0;
+    int n = 0, nused = 0;             // (n: thread 0's)
     long numEval = 0;
     bool ovf = false;
-    // initial region
+    // initial region (both waves the same)
     if (lane == 0) {
-      for (int i = 0; i < 3; i++) { sreg[0][i] = 0.5; sreg[0][3 + i] = 0.5; }
+      for (int i = 0; i < 6; i++) sreg[rg][i] = 0.5;
       double v = 1.0;
       for (int i = 0; i < dim; i++) v *= 2 * 0.5;
-      sreg[0][6] = v; sreg[0][7] = 0;
+      sreg[rg][6] = v;
     }
     __syncthreads();
-    for (int p = lane; p < npts; p += 64) {
-      double x[3];
-      rule_point(dim, p, sreg[0], sreg[0] + 3, x);
-      double f[NF];
-      integrand(W, x, f);
-      for (int q = 0; q < NF; q++) buf[p * NF + q] = f[q];
+    rule();
+    if (rg == 0) {
+      if (lane < 8) data[lane] = sreg[0][lane];
+      if (lane < NF) { data[8 + lane] = eA[0][lane]; data[8 + NF + lane] = rA[0][lane]; }
     }
-    __syncthreads();
-    if (lane < NF) {
-      double v, e, d[3] = {0, 0, 0};
-      rule_sums(dim, lane, buf, sreg[0][6], &v, &e, d);
-      eA[0][lane] = v; rA[0][lane] = e;
-      for (int q = 0; q < 3; q++) dpart[0][lane][q] = d[q];
-    }
-    __syncthreads();
-    if (lane == 0) {
-      double dsum[3] = {0, 0, 0}, em = 0;
-      for (int q = 0; q < NF; q++) { for (int i = 0; i < dim; i++) dsum[i] += dpart[0][q][i]; if (rA[0][q] > em) em = rA[0][q]; }
-      double mx = 0; int sd = 0;
-      for (int i = 0; i < dim; i++) if (dsum[i] > mx) { mx = dsum[i]; sd = i; }
-      if (dim == 1) sd = 0;
-      double *R = data;
-      for (int i = 0; i < 6; i++) R[i] = sreg[0][i];
-      R[6] = sreg[0][6]; R[7] = sd;
-      heap_push(H, n, em, 0);
-    }
-    if (lane < NF) { data[8 + lane] = eA[0][lane]; data[8 + NF + lane] = rA[0][lane]; totV += eA[0][lane]; totE += rA[0][lane]; }
+    if (threadIdx.x == 0) heap_push(H, n, s_em[0], 0);
+    if (lane < NF) { totV += eA[0][lane]; totE += rA[0][lane]; }
     nused = 1;
     numEval = npts;
-    __syncthreads();
+    // the records that the next pop can return: the two regions of the last
+    // split (slots sa, sb; in LDS) and the heap's top before they were
+    // pushed (slot sp; read while they were evaluated).  lane < 8: geometry,
+    // lane < 33: value and error
+    int sa = 0, sb = -1, sp = -1;
+    double pg = 0, pv = 0, pe = 0;
 
     while (numEval < maxEval) {
       // convergence (converged.h ERROR_INDIVIDUAL)
-      int bad = (lane < NF) && (totE > reqAbs && totE > fabs(totV) * reqRel);
+      const int bad = (lane < NF) && (totE > reqAbs && totE > fabs(totV) * reqRel);
       if (!__any(bad)) break;
       if (nused + 1 > cap) { ovf = true; break; }
-      if (lane == 0) { s_pop = heap_pop(H, n); s_slotB = nused; }
+      int top = -1;
+      if (threadIdx.x == 0) {
+        const int s = heap_pop(H, n);
+        s_pop = s;
+        s_nh = n > 0 ? H.slot(0) : -1;
+      }
       __syncthreads();
-      int sa = s_pop, sb = s_slotB;
+      const int s = s_pop, s2 = nused;
+      top = s_nh;
       nused++;
-      double *RA = data + (long long)sa * REC, *RB = data + (long long)sb * REC;
-      if (lane < NF) { totV -= RA[8 + lane]; totE -= RA[8 + NF + lane]; }
-      if (lane == 0) {
-        // cut_region (hcubature.c:215-228)
-        int d = (int)RA[7];
-        double c[3] = {RA[0], RA[1], RA[2]}, h[3] = {RA[3], RA[4], RA[5]};
-        double vol = RA[6];
-        h[d] *= 0.5;
-        vol *= 0.5;
-        double volB = 1;
-        for (int i = 0; i < dim; i++) volB *= 2 * h[i];
-        double cA[3] = {c[0], c[1], c[2]}, cB[3] = {c[0], c[1], c[2]};
-        cA[d] -= h[d];
-        cB[d] += h[d];
-        for (int i = 0; i < 3; i++) { sreg[0][i] = cA[i]; sreg[0][3 + i] = h[i]; sreg[1][i] = cB[i]; sreg[1][3 + i] = h[i]; }
-        sreg[0][6] = vol; sreg[1][6] = volB;
+      // the popped region's record
+      double g, v, e;
+      if (s == sa || s == sb) {
+        const int w = s == sa ? 0 : 1;
+        g = sreg[w][lane & 7];
+        v = lane < NF ? eA[w][lane] : 0.0;
+        e = lane < NF ? rA[w][lane] : 0.0;
+      } else if (s == sp) { g = pg; v = pv; e = pe; }
+      else {
+        const double *R = data + (long long)s * REC;
+        g = R[lane & 7];
+        v = lane < NF ? R[8 + lane] : 0.0;
+        e = lane < NF ? R[8 + NF + lane] : 0.0;
       }
-      __syncthreads();
-      for (int g = lane; g < 2 * npts; g += 64) {
-        int rg = g / npts, p = g % npts;
-        double x[3];
-        rule_point(dim, p, sreg[rg], sreg[rg] + 3, x);
-        double f[NF];
-        integrand(W, x, f);
-        for (int q = 0; q < NF; q++) buf[g * NF + q] = f[q];
-      }
-      __syncthreads();
-      if (lane < NF) {
-        for (int rg = 0; rg < 2; rg++) {
-          double v, e, d[3] = {0, 0, 0};
-          rule_sums(dim, lane, buf + rg * npts * NF, sreg[rg][6], &v, &e, d);
-          eA[rg][lane] = v; rA[rg][lane] = e;
-          for (int q = 0; q < 3; q++) dpart[rg][lane][q] = d[q];
+      // the top that remains: from the same places, else read ahead
+      if (top >= 0 && top != sp) {
+        if (top == sa || top == sb) {
+          const int w = top == sa ? 0 : 1;
+          pg = sreg[w][lane & 7];
+          pv = lane < NF ? eA[w][lane] : 0.0;
+          pe = lane < NF ? rA[w][lane] : 0.0;
+        } else {
+          const double *R = data + (long long)top * REC;
+          pg = R[lane & 7];
+          pv = lane < NF ? R[8 + lane] : 0.0;
+          pe = lane < NF ? R[8 + NF + lane] : 0.0;
         }
       }
+      sp = top;
+      sa = s;
+      sb = s2;
+      totV -= v;
+      totE -= e;
+      // cut_region (hcubature.c:215-228): lane i < 3 center i, 3 + i half i
+      const int d = (int)__shfl(g, 7);
+      const double vol = __shfl(g, 6) * 0.5, hd = __shfl(g, 3 + d) * 0.5;
+      if (lane == 3 + d) g = hd;
+      double volB = 1;
+      for (int i = 0; i < dim; i++) volB *= 2 * __shfl(g, 3 + i);
+      if (lane == d) g = rg == 0 ? g - hd : g + hd;
+      if (lane == 6) g = rg == 0 ? vol : volB;
+      __syncthreads();                // (both waves have read sreg, eA, rA)
+      if (lane < 7) sreg[rg][lane] = g;
       __syncthreads();
+      rule();
+      {
+        double *R = data + (long long)(rg == 0 ? sa : sb) * REC;
+        if (lane < 8) R[lane] = sreg[rg][lane];
+        if (lane < NF) { R[8 + lane] = eA[rg][lane]; R[8 + NF + lane] = rA[rg][lane]; }
+      }
       if (lane < NF) {
-        RA[8 + lane] = eA[0][lane]; RA[8 + NF + lane] = rA[0][lane];
-        RB[8 + lane] = eA[1][lane]; RB[8 + NF + lane] = rA[1][lane];
         totV += eA[0][lane]; totE += rA[0][lane];
         totV += eA[1][lane]; totE += rA[1][lane];
       }
-      if (lane == 0) {
-        double em[2];
-        int sdim[2];
-        for (int rg = 0; rg < 2; rg++) {
-          double dsum[3] = {0, 0, 0}, m = 0;
-          for (int q = 0; q < NF; q++) { for (int i = 0; i < dim; i++) dsum[i] += dpart[rg][q][i]; if (rA[rg][q] > m) m = rA[rg][q]; }
-          double mx = 0; int sd = 0;
-          for (int i = 0; i < dim; i++) if (dsum[i] > mx) { mx = dsum[i]; sd = i; }
-          em[rg] = m; sdim[rg] = sd;
-        }
-        for (int i = 0; i < 6; i++) { RA[i] = sreg[0][i]; RB[i] = sreg[1][i]; }
-        RA[6] = sreg[0][6]; RB[6] = sreg[1][6];
-        RA[7] = sdim[0]; RB[7] = sdim[1];
-        heap_push(H, n, em[0], sa);
-        heap_push(H, n, em[1], sb);
+      if (threadIdx.x == 0) {
+        heap_push(H, n, s_em[0], sa);
+        heap_push(H, n, s_em[1], sb);
       }
       numEval += 2 * npts;
-      __syncthreads();
     }
-    // broadcast the heap size held by lane 0
-    if (lane == 0) s_stop = n;
+    // broadcast the heap size held by thread 0
+    if (threadIdx.x == 0) s_nh = n;
     __syncthreads();
-    int nh = s_stop;
+    const int nh = s_nh;
     if (ovf) {
-      if (lane == 0) overflow[job] = 1;
-    } else if (lane < NF) {
-      double v = 0;
-      for (int i = 0; i < nh; i++) v += data[(long long)H.slot[i] * REC + 8 + lane];
+      if (threadIdx.x == 0) overflow[job] = 1;
+    } else if (rg == 0) {
       double *out = records + (long long)job * SCUFFX_QIF_LEN;
-      out[lane] = v;
-    }
-    if (!ovf && lane < 3) {
-      double *out = records + (long long)job * SCUFFX_QIF_LEN;
-      out[33 + lane] = (J.OVa[lane] + J.OVa[3 + lane] + J.OVa[6 + lane]) / 3.0;
+      if (lane < NF) {
+        // the regions' values in heap order, 16 loads in flight
+        double v = 0;
+        int i = 0;
+        for (; i + 16 <= nh; i += 16) {
+          double r[16];
+#pragma unroll
+          for (int u = 0; u < 16; u++) r[u] = data[(long long)H.slot(i + u) * REC + 8 + lane];
+#pragma unroll
+          for (int u = 0; u < 16; u++) v += r[u];
+        }
+        for (; i < nh; i++) v += data[(long long)H.slot(i) * REC + 8 + lane];
+        out[lane] = v;
+      }
+      if (lane < 3) out[33 + lane] = (J.OVa[lane] + J.OVa[3 + lane] + J.OVa[6 + lane]) / 3.0;
     }
     __syncthreads();
   }
@@ -781,7 +849,8 @@ hipError_t launch_fippi(hipStream_t stream, const FippiJob *jobs, int njobs, dou
                         int *counter, int *overflow, const int *jobList)
 {
   if (njobs <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fippi, dim3(nslots), dim3(64), 0, stream, jobs, njobs, jobList, records,
+  if (cap > 65536) return hipErrorInvalidValue;   // regions are 16-bit numbers in the heap
+  hipLaunchKernelGGL(k_fippi, dim3(nslots), dim3(128), 0, stream, jobs, njobs, jobList, records,
                      heapData, heapSlot, heapKey, cap, counter, overflow);
   return hipGetLastError();
 }

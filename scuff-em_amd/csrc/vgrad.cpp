@@ -24,32 +24,6 @@ namespace scuffx {
 
 namespace {
 
-// device buffers of one call, freed on return
-struct Scratch {
-  std::vector<void *> ptrs;
-  ~Scratch()
-  {
-    if (hip_down()) return;
-    for (void *p : ptrs) hipFree(p);
-  }
-  template <typename T>
-  T *alloc(size_t n)
-  {
-    void *p = nullptr;
-    if (hipMalloc(&p, sizeof(T) * std::max<size_t>(n, 1)) != hipSuccess) return nullptr;
-    ptrs.push_back(p);
-    return (T *)p;
-  }
-  template <typename T>
-  T *put(const std::vector<T> &h)
-  {
-    T *d = alloc<T>(h.size());
-    if (d && !h.empty() && hipMemcpy(d, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice) != hipSuccess)
-      return nullptr;
-    return d;
-  }
-};
-
 // relative step of the central differences, in units of the larger
 // panel radius of the pair
 constexpr double kFDStep = 1.0e-4;
