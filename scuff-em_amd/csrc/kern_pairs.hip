@@ -136,50 +136,106 @@ __device__ inline void tcr4_point(const double *p, int i, double *x)
   for (int c = 0; c < 3; c++) x[c] = p[c] + s * p[3 + c] + u * p[6 + c];
 }
 
-// pair_moments<0> with the points formed on the fly and the 6 x 6 point
-// loop kept rolled: the same sums in the same order, in about half the
-// registers of the unrolled form (two waves per SIMD instead of one)
-__device__ inline void pair_moments_far(const double *pa, const double *pb, const double *D, cplx k, int needH1,
-                                        Moments &m)
+// 1/sqrt(x) and sqrt(x) of a normal x > 0: the hardware's estimate, one
+// third-order step, then each corrected by its own residual (half an ulp, as
+// the square root and the quotient it replaces)
+__device__ inline void rsqrt_sqrt(double x, double *ir, double *r)
+{
+  double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  y = fma(y * e, fma(0.375, e, 0.5), y);
+  const double q = x * y;
+  *r = fma(fma(-q, q, x), 0.5 * y, q);
+  *ir = fma(fma(-*r, y, 1.0), y, y);
+}
+
+// Phi sums over the six points y of the second panel for one point x of the
+// first: p0 = sum Phi, p = sum y Phi, q0 = sum Psi, q = sum y Psi (the
+// weights of y in Phi)
+struct RowSums {
+  cplx p0, p[3], q0, q[3];
+};
+
+// The moments of pair_moments<0>, from the row sums: with R = D + x - y
+// every moment is linear in them, e.g. u = sum (R x x) Psi = (D x x) q0 +
+// x x q and s = sum ((x x y).R) Psi = (x x q).D, so a point pair costs its
+// kernel and 16 multiply-adds where the moments themselves took 40 and the
+// vector products 27 operations more.  sy: the points of the second panel
+// (one panel for the whole workgroup); sp: per thread the first panel as {V0 -
+// centroid, V1 - V0, V2 - V0} and D, in LDS, so that the point loop, rolled,
+// keeps to 256 registers (two waves per SIMD).  Bound: FP64 vector rate; FARNUM
+__device__ inline void pair_moments_far(const double (*sp)[256], const double (*sy)[3], cplx k, int needH1, Moments &m)
 {
 #pragma clang fp contract(fast)
   m.S1 = mk(0, 0); m.Sxy = mk(0, 0); m.s = mk(0, 0);
   for (int c = 0; c < 3; c++) { m.Sx[c] = mk(0, 0); m.Sy[c] = mk(0, 0); m.u[c] = mk(0, 0); m.v[c] = mk(0, 0); m.w[c] = mk(0, 0); }
-  cplx ik = IMUL(k);
 #pragma unroll 1
   for (int i = 0; i < 6; i++) {
-    const double wi = c_tcr4[3 * i + 2];
-    double x[3];
-    tcr4_point(pa, i, x);
+    const double wi = c_tcr4[3 * i + 2] * SCUFFX_INV4PI;
+    const int tid = threadIdx.x;
+    double Dx[3];
+    asm volatile("" ::: "memory");   // (or the values stay in registers after all)
+    {
+      const double s = c_tcr4[3 * i], u = c_tcr4[3 * i + 1];
+      for (int c = 0; c < 3; c++) Dx[c] = sp[9 + c][tid] + ((sp[c][tid] + s * sp[3 + c][tid]) + u * sp[6 + c][tid]);
+    }
+    RowSums t;
+    t.p0 = mk(0, 0); t.q0 = mk(0, 0);
+    for (int c = 0; c < 3; c++) { t.p[c] = mk(0, 0); t.q[c] = mk(0, 0); }
 #pragma unroll 1
     for (int j = 0; j < 6; j++) {
-      const double wj = c_tcr4[3 * j + 2];
-      double y[3];
-      tcr4_point(pb, j, y);
-      double R[3] = {D[0] + x[0] - y[0], D[1] + x[1] - y[1], D[2] + x[2] - y[2]};
-      double r2 = R[0] * R[0] + R[1] * R[1] + R[2] * R[2];
-      double r = sqrt(r2);
-      double ir = 1.0 / r;
+      const double y[3] = {sy[j][0], sy[j][1], sy[j][2]};
+      const double R[3] = {Dx[0] - y[0], Dx[1] - y[1], Dx[2] - y[2]};
+      double r, ir, sn = 0.0, cs = 1.0;
+      rsqrt_sqrt(R[0] * R[0] + R[1] * R[1] + R[2] * R[2], &ir, &r);
       // (a real wavenumber, as in a lossless region at real frequency,
-      // skips the exponential: exp(-0) is 1 exactly)
-      double e = 1.0, sn, cs;
-      if (k.i != 0) e = exp(-k.i * r);
-      sincos(k.r * r, &sn, &cs);
-      cplx Phi = mk(e * cs, e * sn) * (SCUFFX_INV4PI * ir);
-      Phi = Phi * (wi * wj);
-      m.S1 += Phi;
-      for (int c = 0; c < 3; c++) { m.Sx[c] += x[c] * Phi; m.Sy[c] += y[c] * Phi; }
-      m.Sxy += (x[0] * y[0] + x[1] * y[1] + x[2] * y[2]) * Phi;
+      // skips the exponential, an imaginary one, as at imaginary frequency,
+      // the sine and cosine: both are exact there)
+      double e = c_tcr4[3 * j + 2] * ir;
+      if (k.i != 0) e *= exp(-k.i * r);
+      if (k.r != 0) sincos(k.r * r, &sn, &cs);
+      const double fr = e * cs, fi = e * sn;
+      t.p0.r += fr; t.p0.i += fi;
+      for (int c = 0; c < 3; c++) { t.p[c].r += y[c] * fr; t.p[c].i += y[c] * fi; }
       if (needH1) {
-        cplx Psi = Phi * (ik - mk(ir, 0)) * ir;
-        double xy[3], Rx[3], yR[3];
-        cross3(x, y, xy);
-        cross3(R, x, Rx);
-        cross3(y, R, yR);
-        m.s += (xy[0] * R[0] + xy[1] * R[1] + xy[2] * R[2]) * Psi;
-        for (int c = 0; c < 3; c++) { m.u[c] += Rx[c] * Psi; m.v[c] += yR[c] * Psi; m.w[c] += R[c] * Psi; }
+        // Psi = Phi (ik - 1/r) / r
+        const double a = -(k.i + ir) * ir, b = k.r * ir;
+        const double gr = fr * a - fi * b, gi = fr * b + fi * a;
+        t.q0.r += gr; t.q0.i += gi;
+        for (int c = 0; c < 3; c++) { t.q[c].r += y[c] * gr; t.q[c].i += y[c] * gi; }
       }
     }
+    // x and D again (held in LDS through the point loop)
+    double x[3], D[3];
+    asm volatile("" ::: "memory");
+    {
+      const double s = c_tcr4[3 * i], u = c_tcr4[3 * i + 1];
+      for (int c = 0; c < 3; c++) {
+        D[c] = sp[9 + c][tid];
+        x[c] = (sp[c][tid] + s * sp[3 + c][tid]) + u * sp[6 + c][tid];
+      }
+    }
+    auto part = [&](auto get, auto put) __attribute__((always_inline)) {
+      const double p0 = wi * get(t.p0), p[3] = {wi * get(t.p[0]), wi * get(t.p[1]), wi * get(t.p[2])};
+      put(m.S1, p0);
+      for (int c = 0; c < 3; c++) { put(m.Sx[c], x[c] * p0); put(m.Sy[c], p[c]); }
+      put(m.Sxy, x[0] * p[0] + x[1] * p[1] + x[2] * p[2]);
+      if (needH1) {
+        const double q0 = wi * get(t.q0), q[3] = {wi * get(t.q[0]), wi * get(t.q[1]), wi * get(t.q[2])};
+        double xq[3], Dxx[3], qD[3];
+        cross3(x, q, xq);
+        cross3(D, x, Dxx);
+        cross3(q, Dx, qD);
+        put(m.s, xq[0] * D[0] + xq[1] * D[1] + xq[2] * D[2]);
+        for (int c = 0; c < 3; c++) {
+          put(m.u[c], Dxx[c] * q0 + xq[c]);
+          put(m.v[c], qD[c]);
+          put(m.w[c], Dx[c] * q0 - q[c]);
+        }
+      }
+    };
+    part([](cplx z) { return z.r; }, [](cplx &z, double v) { z.r += v; });
+    part([](cplx z) { return z.i; }, [](cplx &z, double v) { z.i += v; });
   }
 }
 
@@ -192,39 +248,46 @@ __device__ inline void pair_moments_far(const double *pa, const double *pb, cons
 // (Qa, Qb) combinations 3 qa + qb of {H0[, H1]}.
 // grid.x over row panels, grid.y = slot.
 // ---------------------------------------------------------------------
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, 2)
 k_far(const double *Va, const int *PVIa, const double *PCa, int rowLimit,
       const double *Vb, const int *PVIb, const double *PCb, const int *slotPanels, int same,
       const int *nearRowPtr, const int *nearCol, int nreg, const RegionK *regs,
       int needH1, double *HB, long rowsCap)
 {
+  __shared__ double sy[6][3], sp[12][256];
   const int slot = blockIdx.y;
   const int pa = blockIdx.x * blockDim.x + threadIdx.x;
-  if (pa >= rowLimit) return;
   const int pb = slotPanels[slot];
+  const double *cb = PCb + 4 * pb;
+  const double *B0 = Vb + 3 * PVIb[3 * pb], *B1 = Vb + 3 * PVIb[3 * pb + 1], *B2 = Vb + 3 * PVIb[3 * pb + 2];
+  if (threadIdx.x < 6) {
+    double PB[9];
+    for (int c = 0; c < 3; c++) { PB[c] = B0[c] - cb[c]; PB[3 + c] = B1[c] - B0[c]; PB[6 + c] = B2[c] - B0[c]; }
+    tcr4_point(PB, threadIdx.x, sy[threadIdx.x]);
+  }
+  __syncthreads();
+  if (pa >= rowLimit) return;
   if (same && pb == pa) return;
   if (near_find(nearRowPtr, nearCol, pa, pb) >= 0) {
     const int stride = needH1 ? 4 : 2;
     HB[((long)slot * rowsCap + pa) * (long)(nreg * 9 * stride)] = __longlong_as_double((long long)SCUFFX_NEAR_MARK);
     return;
   }
-  double ca[3] = {PCa[4 * pa], PCa[4 * pa + 1], PCa[4 * pa + 2]};
-  double cb[3] = {PCb[4 * pb], PCb[4 * pb + 1], PCb[4 * pb + 2]};
+  const double *ca = PCa + 4 * pa;
   const double *A0 = Va + 3 * PVIa[3 * pa], *A1 = Va + 3 * PVIa[3 * pa + 1], *A2 = Va + 3 * PVIa[3 * pa + 2];
-  const double *B0 = Vb + 3 * PVIb[3 * pb], *B1 = Vb + 3 * PVIb[3 * pb + 1], *B2 = Vb + 3 * PVIb[3 * pb + 2];
-  // panels as {V0 - centroid, V1 - V0, V2 - V0}; D = centroid difference
-  double PA[9], PB[9], D[3];
+  // (each thread reads only what it wrote: no barrier)
   for (int c = 0; c < 3; c++) {
-    PA[c] = A0[c] - ca[c]; PA[3 + c] = A1[c] - A0[c]; PA[6 + c] = A2[c] - A0[c];
-    PB[c] = B0[c] - cb[c]; PB[3 + c] = B1[c] - B0[c]; PB[6 + c] = B2[c] - B0[c];
-    D[c] = ca[c] - cb[c];
+    sp[c][threadIdx.x] = A0[c] - ca[c];
+    sp[3 + c][threadIdx.x] = A1[c] - A0[c];
+    sp[6 + c][threadIdx.x] = A2[c] - A0[c];
+    sp[9 + c][threadIdx.x] = ca[c] - cb[c];
   }
   const int stride = needH1 ? 4 : 2;
   double *out = HB + ((long)slot * rowsCap + pa) * (long)(nreg * 9 * stride);
   for (int r = 0; r < nreg; r++) {
     Moments m;
     cplx k = regs[r].k;
-    pair_moments_far(PA, PB, D, k, needH1, m);
+    pair_moments_far(sp, sy, k, needH1, m);
     // source vertices relative to the centroids
     double Qa[9], Qb[9];
     for (int c = 0; c < 3; c++) {
