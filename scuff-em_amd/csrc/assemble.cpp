@@ -715,11 +715,10 @@ int Assembler::assemble(cdouble omega, void *Mp, long ldm, int kind, hipStream_t
       if (ensure(&d_HN_, &cap_HN_, (size_t)B.pairs.size() * nreg * 9 * stride)) return -2;
       if (same) {
         if (ensure(&d_HS_, &cap_HS_, (size_t)Da.nP * nreg * 18)) return -2;
-        int chunk = 16384;
-        if (ensure(&d_scratch_, &cap_scratch_, (size_t)chunk * 1025 * 4)) return -2;
+        if (ensure(&d_scratch_, &cap_scratch_, (size_t)SCUFFX_SELF_SLABS * SCUFFX_SELF_SLAB)) return -2;
         hipEventRecord(ev[0], stream);
         int tok = prof_begin(stream, PK_SELF);
-        if (nreg > 0) HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, dreg, d_HS_, d_scratch_, chunk));
+        if (nreg > 0) HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, dreg, d_HS_, d_scratch_));
         prof_end(stream, tok, 0.0);
         hipEventRecord(ev[1], stream);
         stats_.nself += (long)Da.nP * 9 * nreg;
@@ -810,7 +809,7 @@ int Assembler::prepare_graph(const std::vector<cdouble> &omegas, hipStream_t str
       }
   }
   if (ensure(&d_HN_, &cap_HN_, need_hn) || ensure(&d_HS_, &cap_HS_, need_hs) || ensure(&d_HP_, &cap_HP_, need_hb) ||
-      ensure(&d_scratch_, &cap_scratch_, (size_t)16384 * 1025 * 4))
+      ensure(&d_scratch_, &cap_scratch_, (size_t)SCUFFX_SELF_SLABS * SCUFFX_SELF_SLAB))
     return -2;
   const size_t bytes = sizeof(RegionK) * tab.size();
   if (bytes > cap_regtab_) {
@@ -847,7 +846,7 @@ int Assembler::assemble_graph(int f, void *Mp, long ldm, hipStream_t stream)
       const RegionK *dreg = d_regtab_ + ((size_t)f * nblk + bi) * 2;
       const int needH1 = !(Sa.IsPEC && Sb.IsPEC);
       if (same && nreg > 0)
-        HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, dreg, d_HS_, d_scratch_, 16384));
+        HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, dreg, d_HS_, d_scratch_));
       if (nreg > 0 && !B.pairs.empty())
         HIPCHK(launch_near(stream, B.d_pairs, (int)B.pairs.size(), d_records_, nreg, dreg, needH1, d_HN_));
       int rc = far_and_stamp(B, Da, Db, Sa, Sb, nreg, dreg, needH1, M, G_.BFIndexOffset[sa], G_.BFIndexOffset[sb],
@@ -916,10 +915,9 @@ int Assembler::assemble_block(int sa, int sb, cdouble omega, double2 *B, long ld
   HIPCHK(hipMemcpyAsync(d_regs_, rk, sizeof(RegionK) * std::max(nreg, 1), hipMemcpyHostToDevice, stream));
   if (ensure(&d_HN_, &cap_HN_, (size_t)NB.pairs.size() * nreg * 9 * stride)) return -2;
   if (same && nreg > 0) {
-    const int chunk = 16384;
     if (ensure(&d_HS_, &cap_HS_, (size_t)Da.nP * nreg * 18)) return -2;
-    if (ensure(&d_scratch_, &cap_scratch_, (size_t)chunk * 1025 * 4)) return -2;
-    HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, d_regs_, d_HS_, d_scratch_, chunk));
+    if (ensure(&d_scratch_, &cap_scratch_, (size_t)SCUFFX_SELF_SLABS * SCUFFX_SELF_SLAB)) return -2;
+    HIPCHK(launch_self(stream, Da.V, Da.PVI, Da.nP, nreg, d_regs_, d_HS_, d_scratch_));
   }
   // the block in (lo, hi) orientation, directly into B or into a
   // staging copy that is transposed into B

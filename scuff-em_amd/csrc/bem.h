@@ -80,7 +80,11 @@ hipError_t launch_far(hipStream_t stream, const double *Va, const int *PVIa, con
 hipError_t launch_near(hipStream_t stream, const NearPair *np, int nnear, const double *records,
                        int nreg, const RegionK *regs, int needH1, double *HN);
 hipError_t launch_self(hipStream_t stream, const double *V, const int *PVI, int nP, int nreg,
-                       const RegionK *regs, double *HS, double *scratch, int chunk);
+                       const RegionK *regs, double *HS, double *scratch);
+// doubles of scratch per wave of the self-term kernel (nodes past order 5) and
+// its waves (ten on a CU)
+#define SCUFFX_SELF_SLAB (960 * 20)
+#define SCUFFX_SELF_SLABS 2560
 hipError_t launch_fippi(hipStream_t stream, const FippiJob *jobs, int njobs, double *records,
                         double *heapData, int *heapSlot, double *heapKey, int cap, int nslots,
                         int *counter, int *overflow, const int *jobList);

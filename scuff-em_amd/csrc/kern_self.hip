@@ -7,61 +7,29 @@
 // remaining 1-D integral is done by p-adaptive Clenshaw-Curtis
 // quadrature, relative tolerance 1e-10, at most 1000 new points
 // (TaylorDuffy.cc:152-367, libs/libSGJC/pcubature.c:323-385).
-// One wave per (panel, Qa, Qb, region) job; the function values of a job
-// live in a scratch slab so every refinement level reuses them.
+// One wave per (panel, region) job: the kernel values at a node serve all
+// nine (Qa, Qb).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "bem.h"
+#include "exprel.h"
 
 namespace scuffx {
 
 #define TD_NWP 5
 #define TD_MAXM 9            // 2^(9+1)+1 = 1025 nodes reached by MaxEval=1000
-#define TD_NODES 1025
 #define TD_NPRE 64           // cache entries computed up front, one per lane
 
 __constant__ double c_ccx[512];            // nodes x_i, layout as the oracle
 __constant__ double c_ccw[TD_MAXM + 1 + (1 << (TD_MAXM + 1))];
 
-// relative exponential ExpRelV3P0 (TaylorDuffy.cc:840-893)
-__device__ cplx exprel_v3(int n, cplx Z)
-{
-  int m;
-  if (Z.i == 0.0) {
-    double X = Z.r, Term, Sum;
-    if (fabs(X) < 0.1) {
-      Sum = 1.0;
-      for (Term = 1.0, m = 1; m < 100; m++) {
-        Term *= X / ((double)(m + n));
-        Sum += Term;
-        if (fabs(Term) < 1.0e-8 * fabs(Sum)) break;
-      }
-      return mk(Sum, 0);
-    }
-    Sum = exp(X);
-    for (Term = 1.0, m = 0; m < n; m++) { Sum -= Term; Term *= X / ((double)(m + 1)); }
-    return mk(Sum / Term, 0);
-  }
-  cplx Term, Sum;
-  if (sqrt(Z.r * Z.r + Z.i * Z.i) < 0.1) {
-    Sum = Term = mk(1, 0);
-    for (m = 1; m < 100; m++) {
-      Term = Term * (Z / (double)(m + n));
-      Sum += Term;
-      if (norm2(Term) < 1.0e-16 * norm2(Sum)) break;
-    }
-    return Sum;
-  }
-  Sum = cexp_(Z);
-  Term = mk(1, 0);
-  for (m = 0; m < n; m++) { Sum -= Term; Term = Term * (Z / (double)(m + 1)); }
-  return Sum / Term;
-}
-
 // common-triangle Upsilon coefficients (TaylorDuffy.cc:966-1057):
 // U[d][n][0..2] = coefficients of 1, y, y^2; only M13,M14,M23,M24,V,S
-// are non-zero for P in {1, PMCHWG1}.
-struct CTPoly { double U[3][TD_NWP][3]; int nMin, nMax; };
+// are non-zero for P in {1, PMCHWG1}.  Powers n outside the range that the
+// sums take (below) are left zero.
+struct CTPoly { double U[3][TD_NWP][3]; };
 
 __device__ void ct_upsilon(double M13, double M14, double M23, double M24, double V1, double V2,
                            double V3, double V4, double S, CTPoly &P)
@@ -122,40 +90,52 @@ __device__ void ct_upsilon(double M13, double M14, double M23, double M24, doubl
     for (int d = 0; d < 3; d++)
       for (int j = 0; j < 3; j++)
         if (fabs(U[d][n][j]) > 1.0e-8) { if (n < nMin) nMin = n; if (n > nMax) nMax = n; }
-  P.nMin = nMin; P.nMax = nMax;
+  for (int n = 0; n < TD_NWP; n++)
+    if (n < nMin || n > nMax)
+      for (int d = 0; d < 3; d++)
+        for (int j = 0; j < 3; j++) U[d][n][j] = 0.0;
 }
 
-struct CTJob { double A2, AdB, B2; CTPoly P[2]; cplx k; };
+// polynomial 0: P = 1, 1 + 3 qa + qb: PMCHWG1 of (Qa, Qb)
+#define CT_NP 10
+#define CT_NV (2 * CT_NP)                // real values of a node
+struct CTJob { double A2, AdB, B2; CTPoly P[CT_NP]; cplx k; };
 
-// integrand at y: two complex values (P=1, P=PMCHWG1) as 4 doubles.  The
-// job (J, in LDS) is shared by the wave; the kernel values K_n(X_d) =
-// e^{ikX} ExpRel_n(-ikX) / (n X) are formed where the sum uses them (the
-// same operations as tabulating them first, without an array indexed by
-// the run-time power range, which would live in scratch memory), and
-// e^{ikX_d} once for both polynomials.
-__device__ void ct_integrand(const CTJob &J, double y, double *f)
+// integrand at y for all ten polynomials.  The job (J, in LDS) is shared by
+// the wave; the kernel values K_n(X_d) = e^{ikX} ExpRel_n(-ikX) / (n X) of
+// every power are formed once, from one sine, cosine and pair of
+// exponentials a distance
+__device__ inline void ct_integrand(const CTJob &J, double y, double *f)
 {
-  double X[3], u1, u2;
-  u1 = 1.0; u2 = y;       X[0] = sqrt(J.A2 * u1 * u1 + 2.0 * J.AdB * u1 * u2 + J.B2 * u2 * u2);
-  u1 = y;   u2 = (y - 1); X[1] = sqrt(J.A2 * u1 * u1 + 2.0 * J.AdB * u1 * u2 + J.B2 * u2 * u2);
-  u1 = y;   u2 = 1.0;     X[2] = sqrt(J.A2 * u1 * u1 + 2.0 * J.AdB * u1 * u2 + J.B2 * u2 * u2);
+#pragma clang fp contract(fast)
+#pragma unroll
+  for (int v = 0; v < CT_NV; v++) f[v] = 0.0;
   const cplx IK = IMUL(J.k);
-  cplx IKX[3], E[3];
+#pragma unroll 1
   for (int d = 0; d < 3; d++) {
-    IKX[d] = IK * X[d];
-    E[d] = cexp_(IKX[d]);
-  }
-  for (int pk = 0; pk < 2; pk++) {
-    const CTPoly &P = J.P[pk];
-    cplx s = mk(0, 0);
-    for (int n = P.nMin; n <= P.nMax; n++)
-      for (int d = 0; d < 3; d++) {
-        const cplx K = E[d] * exprel_v3(n + 1, -IKX[d]) / ((n + 1) * X[d]);
-        s += (P.U[d][n][0] + y * P.U[d][n][1]) * K;
+    const double u1 = d == 0 ? 1.0 : y, u2 = d == 0 ? y : d == 1 ? y - 1 : 1.0;
+    const double X = sqrt(J.A2 * u1 * u1 + 2.0 * J.AdB * u1 * u2 + J.B2 * u2 * u2), iX = 1.0 / X;
+    const cplx IKX = IK * X;
+    double sn, cs;
+    sincos(IKX.i, &sn, &cs);
+    const double ep = exp(IKX.r), em = exp(-IKX.r);
+    cplx ER[TD_NER];
+    exprels(TD_NWP, -IKX, mk(em * cs, -(em * sn)), ER);
+    const cplx e = mk(ep * cs * iX, ep * sn * iX);
+    cplx K[TD_NWP];
+#pragma unroll
+    for (int n = 0; n < TD_NWP; n++) K[n] = (1.0 / (n + 1)) * cmulf(e, ER[n + 1]);
+#pragma unroll
+    for (int p = 0; p < CT_NP; p++)
+#pragma unroll
+      for (int n = 0; n < TD_NWP; n++) {
+        const double c = J.P[p].U[d][n][0] + y * J.P[p].U[d][n][1];
+        f[2 * p] += c * K[n].r;
+        f[2 * p + 1] += c * K[n].i;
       }
-    s = s * (1.0 / (4.0 * M_PI));
-    f[2 * pk] = s.r; f[2 * pk + 1] = s.i;
   }
+#pragma unroll
+  for (int v = 0; v < CT_NV; v++) f[v] *= 1.0 / (4.0 * M_PI);
 }
 
 // weight of cache entry e in the Clenshaw-Curtis rule of the given order
@@ -173,97 +153,144 @@ __device__ inline double cc_weight(int e, int order)
   return w[1 + nl + ((e - (1 << l) - 1) >> 1)];
 }
 
-// One wave per (panel, Qa, Qb, region) job: each refinement level's new
-// points are evaluated across the 64 lanes, and the two rule estimates
-// are lane-strided partial sums reduced over the wave (the same stopping
-// rule as the reference's p-adaptive cubature: relative 1e-10 per
-// component, at most 1000 new points).
+// node of cache entry e (entries as in cc_weight)
+__device__ inline double cc_node(int e)
+{
+  if (e == 0) return 0.5;
+  const int l = e < 3 ? 0 : 31 - __clz(e - 1), k = e < 3 ? e - 1 : e - (1 << l) - 1;
+  const double x = c_ccx[(e < 3 ? 0 : 1 << (l - 1)) + (k >> 1)];
+  return (k & 1) ? 0.5 - 0.5 * x : 0.5 + 0.5 * x;
+}
+
+// One wave per (panel, region) job.  The p-adaptive cubature of each (Qa,
+// Qb) stops by itself (P = 1 and its PMCHWG1 within 1e-10 of the next lower
+// order's, at most 1000 new points, as the reference does), but all nine
+// read the same nodes, whose ten integrands share the kernel values.  The
+// first TD_NPRE nodes, one per lane (orders 0 .. 4), come before the first
+// test, order 5's last one if it is asked for; their sums are taken from LDS,
+// a lane per order and value.  Later orders, if any, keep their nodes in a
+// scratch slab.  Bound: FP64 vector rate of the kernel values; SELFNUM
 __global__ void __launch_bounds__(64)
 k_self(const double *V, const int *PVI, int nP, int nreg, const RegionK *regs,
-       double *HS, double *scratch, int job0, int njobs)
+       double *HS, double *scratch, int njobs)
 {
-  const int t = blockIdx.x, lane = threadIdx.x;
-  if (t >= njobs) return;
-  const int job = job0 + t;
-  const int r = job % nreg, q = (job / nreg) % 9, p = job / (9 * nreg);
-  const int qa = q / 3, qb = q % 3;
-  const double *V1 = V + 3 * PVI[3 * p], *V2 = V + 3 * PVI[3 * p + 1], *V3 = V + 3 * PVI[3 * p + 2];
-  const double *Q = V + 3 * PVI[3 * p + qa], *QP = V + 3 * PVI[3 * p + qb];
-  double A[3], B[3], D[3], DP[3];
-  sub3(V2, V1, A); sub3(V3, V2, B); sub3(V1, Q, D); sub3(V1, QP, DP);
-  // the job's constants in LDS (read by every lane at the same address)
+  const int lane = threadIdx.x;
+  // the job's constants in LDS (read by every lane at the same address), the
+  // node values, the sums of orders -1 .. 5
   __shared__ CTJob J;
-  if (lane == 0) {
-    J.A2 = dot3(A, A); J.AdB = dot3(A, B); J.B2 = dot3(B, B);
-    J.k = regs[r].k;
-    ct_upsilon(0, 0, 0, 0, 0, 0, 0, 0, 1.0, J.P[0]);
-    ct_upsilon(dot3(A, A), dot3(A, B), dot3(B, A), dot3(B, B), dot3(A, DP), dot3(B, DP),
-               dot3(D, A), dot3(D, B), dot3(D, DP), J.P[1]);
-  }
-  __syncthreads();
-  double *vals = scratch + (long long)t * TD_NODES * 4;
-  const double c = 0.5, rr = 0.5, Vol = 0.5;
-  // The first TD_NPRE cache entries (centre, the pair at x_0, then
-  // 2^(l-1) pairs per level l: rule orders 0 .. 4 and all but the last
-  // entry of order 5) are filled at once, one per lane, before the first
-  // convergence test: the lanes a low order leaves idle evaluate the next
-  // orders' points meanwhile.  The tests below read the same values in
-  // the same order as if each order's points were computed after the
-  // previous order's test; only the number of sequential passes shrinks.
-  for (int e = lane; e < TD_NPRE; e += 64) {
-    double y;
-    if (e == 0) y = c;
-    else if (e < 3) y = e == 1 ? c + rr * c_ccx[0] : c - rr * c_ccx[0];
-    else {
-      const int l = 31 - __clz(e - 1), k = e - (1 << l) - 1, nl = 1 << (l - 1);
-      const double x = c_ccx[nl + (k >> 1)];
-      y = (k & 1) ? c - rr * x : c + rr * x;
+  __shared__ double vals[TD_NPRE + 1][CT_NV + 1];
+  __shared__ double S[7][CT_NV];
+  for (int job = blockIdx.x; job < njobs; job += gridDim.x) {
+    const int r = job % nreg, p = job / nreg;
+    const double *V1 = V + 3 * PVI[3 * p], *V2 = V + 3 * PVI[3 * p + 1], *V3 = V + 3 * PVI[3 * p + 2];
+    if (lane < CT_NP) {
+      double A[3], B[3], D[3], DP[3];
+      sub3(V2, V1, A); sub3(V3, V2, B);
+      if (lane == 0) {
+        J.A2 = dot3(A, A); J.AdB = dot3(A, B); J.B2 = dot3(B, B);
+        J.k = regs[r].k;
+        ct_upsilon(0, 0, 0, 0, 0, 0, 0, 0, 1.0, J.P[0]);
+      } else {
+        const int qa = (lane - 1) / 3, qb = (lane - 1) % 3;
+        sub3(V1, V + 3 * PVI[3 * p + qa], D); sub3(V1, V + 3 * PVI[3 * p + qb], DP);
+        ct_upsilon(dot3(A, A), dot3(A, B), dot3(B, A), dot3(B, B), dot3(A, DP), dot3(B, DP),
+                   dot3(D, A), dot3(D, B), dot3(D, DP), J.P[lane]);
+      }
     }
-    ct_integrand(J, y, vals + 4 * e);
-  }
-  __syncthreads();
-  int m = 0, nstored = 3;
-  long numEval = 0;
-  double val[4], val1[4];
-  for (;;) {
-    double a[4] = {0, 0, 0, 0}, b[4] = {0, 0, 0, 0};
-    for (int e = lane; e < nstored; e += 64) {
-      const double wa = cc_weight(e, m) * Vol, wb = cc_weight(e, m - 1) * Vol;
-      for (int cc = 0; cc < 4; cc++) { a[cc] += vals[4 * e + cc] * wa; b[cc] += vals[4 * e + cc] * wb; }
-    }
-    for (int off = 32; off > 0; off >>= 1)
-      for (int cc = 0; cc < 4; cc++) { a[cc] += __shfl_xor(a[cc], off); b[cc] += __shfl_xor(b[cc], off); }
-    bool conv = true;
-    for (int cc = 0; cc < 4; cc++) {
-      val[cc] = a[cc]; val1[cc] = b[cc];
-      const double e = fabs(val[cc] - val1[cc]);
-      if (e > 0.0 && e > fabs(val[cc]) * 1.0e-10) conv = false;
-    }
-    if (conv || numEval > 1000 || m >= TD_MAXM) break;
-    m += 1;
-    const int nl = 1 << (m - 1);
-    for (int k = lane; k < 2 * nl; k += 64) {
-      if (nstored + k < TD_NPRE) continue;   // computed up front
-      const double x = c_ccx[nl + (k >> 1)];
-      ct_integrand(J, (k & 1) ? c - rr * x : c + rr * x, vals + 4 * (nstored + k));
-    }
-    nstored += 2 * nl;
-    numEval += 2 * nl;
     __syncthreads();
-  }
-  if (lane == 0) {
-    cplx I0 = mk(val[0], val[1]), I1 = mk(val[2], val[3]);
-    cplx k = J.k;
-    cplx H0 = I1 - 4.0 * I0 / (k * k);
-    double *o = HS + ((long long)p * nreg + r) * 18 + 2 * q;
-    o[0] = H0.r; o[1] = H0.i;
+    const double Vol = 0.5;
+    double f[CT_NV];
+    ct_integrand(J, cc_node(lane), f);
+#pragma unroll
+    for (int v = 0; v < CT_NV; v++) vals[lane][v] = f[v];
+    __syncthreads();
+    // sums of the orders lane / 20 and lane / 20 + 3 (up to 4 here)
+    const int cv = lane % CT_NV, og = lane / CT_NV;
+    auto rule = [&](int o) {
+      double a = 0.0;
+      const int ne = (1 << (o + 1)) + 1;
+      for (int e = 0; e < ne; e++) a += vals[e][cv] * (cc_weight(e, o) * Vol);
+      S[o + 1][cv] = a;
+    };
+    if (og < 3) {
+      if (og == 0) S[0][cv] = vals[0][cv] * (2.0 * Vol);
+      rule(og);
+      if (og < 2) rule(og + 3);
+    }
+    __syncthreads();
+    // lanes 0 .. 8: combination q; open: not converged yet
+    const bool mine = lane < 9;
+    const int q = mine ? lane : 0;
+    bool open = mine;
+    double R[4] = {0, 0, 0, 0};
+    auto test = [&](int m) {
+      if (!open) return;
+      bool conv = true;
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int v = c < 2 ? c : 2 * q + c;
+        R[c] = S[m + 1][v];
+        const double e = fabs(R[c] - S[m][v]);
+        if (e > 0.0 && e > fabs(R[c]) * 1.0e-10) conv = false;
+      }
+      if (conv) open = false;
+    };
+    for (int m = 0; m <= 4; m++) test(m);
+    if (__ballot(open)) {
+      if (lane == 0) {
+        ct_integrand(J, cc_node(TD_NPRE), f);
+#pragma unroll
+        for (int v = 0; v < CT_NV; v++) vals[TD_NPRE][v] = f[v];
+      }
+      __syncthreads();
+      if (og == 0) rule(5);
+      __syncthreads();
+      test(5);
+      double *slab = scratch + (long long)blockIdx.x * SCUFFX_SELF_SLAB;
+      long numEval = 62;
+      for (int m = 6; m <= TD_MAXM && numEval <= 1000 && __ballot(open); m++) {
+        const int ne = (1 << (m + 1)) + 1;
+        for (int e = (1 << m) + 1 + lane; e < ne; e += 64) {
+          ct_integrand(J, cc_node(e), f);
+#pragma unroll
+          for (int v = 0; v < CT_NV; v++) slab[(long)(e - TD_NPRE - 1) * CT_NV + v] = f[v];
+        }
+        numEval += 1 << m;
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < CT_NV; v++) f[v] = 0.0;
+        for (int e = lane; e < ne; e += 64) {
+          const double w = cc_weight(e, m) * Vol;
+          const double *x = e <= TD_NPRE ? &vals[e][0] : slab + (long)(e - TD_NPRE - 1) * CT_NV;
+#pragma unroll
+          for (int v = 0; v < CT_NV; v++) f[v] += x[v] * w;
+        }
+#pragma unroll
+        for (int v = 0; v < CT_NV; v++) {
+          for (int off = 32; off > 0; off >>= 1) f[v] += __shfl_xor(f[v], off);
+          // (row 5: the order before, row 6: this one)
+          if (lane == 0) { S[5][v] = S[6][v]; S[6][v] = f[v]; }
+        }
+        __syncthreads();
+        test(5);
+      }
+    }
+    if (mine) {
+      const cplx I0 = mk(R[0], R[1]), I1 = mk(R[2], R[3]), k = J.k;
+      const cplx H0 = I1 - 4.0 * I0 / (k * k);
+      double *o = HS + ((long long)p * nreg + r) * 18 + 2 * q;
+      o[0] = H0.r; o[1] = H0.i;
+    }
+    __syncthreads();   // the next job's constants overwrite this one's
   }
 }
+
+static_assert(SCUFFX_SELF_SLAB == ((2 << TD_MAXM) - TD_NPRE) * CT_NV, "scratch slab size");
 
 static bool g_cc_ready[64] = {false};
 
 hipError_t launch_self(hipStream_t stream, const double *V, const int *PVI, int nP, int nreg,
-                       const RegionK *regs, double *HS, double *scratch, int chunk)
+                       const RegionK *regs, double *HS, double *scratch)
 {
   int dev = 0;
   hipGetDevice(&dev);
@@ -302,14 +329,11 @@ hipError_t launch_self(hipStream_t stream, const double *V, const int *PVI, int 
     if (e != hipSuccess) return e;
     g_cc_ready[dev & 63] = true;
   }
-  int njobs = nP * 9 * nreg;
-  for (int j0 = 0; j0 < njobs; j0 += chunk) {
-    int nj = njobs - j0 < chunk ? njobs - j0 : chunk;
-    hipLaunchKernelGGL(k_self, dim3(nj), dim3(64), 0, stream, V, PVI, nP, nreg, regs, HS, scratch, j0, nj);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-  }
-  return hipSuccess;
+  const int njobs = nP * nreg;
+  if (njobs <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_self, dim3(std::min(njobs, SCUFFX_SELF_SLABS)), dim3(64), 0, stream, V, PVI, nP, nreg, regs, HS,
+                     scratch, njobs);
+  return hipGetLastError();
 }
 
 }  // namespace scuffx

@@ -266,8 +266,7 @@ int Assembler::vertex_gradient(cdouble omega, const double2 *M, long ldm, const 
     }
   }
   if (!synPVI.empty()) {
-    const int chunk = 8192;
-    double *scr = sc.alloc<double>((size_t)chunk * 1025 * 4), *dV = sc.put(synV);
+    double *scr = sc.alloc<double>((size_t)SCUFFX_SELF_SLABS * SCUFFX_SELF_SLAB), *dV = sc.put(synV);
     int *dP = sc.put(synPVI);
     if (!scr || !dV || !dP) return bad(-2, "device allocation failed");
     for (int s = 0; s < NS; s++) {
@@ -275,7 +274,7 @@ int Assembler::vertex_gradient(cdouble omega, const double2 *M, long ldm, const 
       const int b = bidx(s, s), nr = nreg[b];
       long hs0 = 0;
       for (int t = 0; t < s; t++) hs0 += synCount[t] * nreg[bidx(t, t)] * 18;
-      if (launch_self(stream, dV, dP + 3 * synBase[s], (int)synCount[s], nr, drk + 2 * b, dHS + hs0, scr, chunk) !=
+      if (launch_self(stream, dV, dP + 3 * synBase[s], (int)synCount[s], nr, drk + 2 * b, dHS + hs0, scr) !=
           hipSuccess)
         return bad(-3, "self-term kernel failed");
     }
