@@ -29,8 +29,10 @@ __device__ void pw_fields(const cplx *E0, const double *nh, cplx K, cplx Z, cons
   EH[5] = (nh[0] * EH[1] - nh[1] * EH[0]) / Z;
 }
 
-__device__ void panel_ip(const double *V1, const double *V2, const double *V3, const double *Q, double pre,
-                         const cplx *E0, const double *nh, cplx K, cplx Z, double sgn, double *I)
+// the inner products of one panel's half of an RWG function with E and H,
+// point q of the rule: added to I[4]
+__device__ inline void panel_ip(const double *V1, const double *V2, const double *V3, const double *Q, double pre,
+                                const cplx *E0, const double *nh, cplx K, cplx Z, double sgn, int q, double *I)
 {
   double A[3], B[3], C, J;
   for (int i = 0; i < 3; i++) { A[i] = V2[i] - V1[i]; B[i] = V3[i] - V1[i]; }
@@ -38,43 +40,49 @@ __device__ void panel_ip(const double *V1, const double *V2, const double *V3, c
   C = A[2] * B[0] - A[0] * B[2]; J += C * C;
   C = A[0] * B[1] - A[1] * B[0]; J += C * C;
   J = sqrt(J);
-  for (int q = 0; q < 4; q++) I[q] = 0;
-  for (int q = 0; q < 78; q++) {
-    double u = c_tcr20[3 * q], v = c_tcr20[3 * q + 1], w = J * c_tcr20[3 * q + 2];
-    double X[3], f[3];
-    for (int i = 0; i < 3; i++) X[i] = V1[i] + u * A[i] + v * B[i];
-    for (int i = 0; i < 3; i++) f[i] = (X[i] - Q[i]) * pre;
-    cplx EH[6];
-    pw_fields(E0, nh, K, Z, X, EH);
-    for (int i = 0; i < 6; i++) EH[i] = sgn * EH[i];
-    cplx e = f[0] * EH[0] + f[1] * EH[1] + f[2] * EH[2];
-    cplx h = f[0] * EH[3] + f[1] * EH[4] + f[2] * EH[5];
-    I[0] += w * e.r; I[1] += w * e.i; I[2] += w * h.r; I[3] += w * h.i;
-  }
+  const double u = c_tcr20[3 * q], v = c_tcr20[3 * q + 1], w = J * c_tcr20[3 * q + 2];
+  double X[3], f[3];
+  for (int i = 0; i < 3; i++) X[i] = V1[i] + u * A[i] + v * B[i];
+  for (int i = 0; i < 3; i++) f[i] = (X[i] - Q[i]) * pre;
+  cplx EH[6];
+  pw_fields(E0, nh, K, Z, X, EH);
+  for (int i = 0; i < 6; i++) EH[i] = sgn * EH[i];
+  const cplx e = f[0] * EH[0] + f[1] * EH[1] + f[2] * EH[2];
+  const cplx h = f[0] * EH[3] + f[1] * EH[4] + f[2] * EH[5];
+  I[0] += w * e.r; I[1] += w * e.i; I[2] += w * h.r; I[3] += w * h.i;
 }
 
+// One wave per edge, its 2 x 78 points over the lanes.  Bound: latency of a
+// lane's three points (a sine, a cosine, an exponential each); an edge per
+// thread left all but a few waves of the chip idle: RHSNUM
 // kz (optional, device): K and Z as re, im, re, im in place of the values
 // passed (a recorded sequence then reads the frequency from memory)
-__global__ void k_rhs(const double *V, const int *PVI, const double *PA, const int *EV, const int *EI,
-                      const double *EL, int nE, int pec, double sgn, cplx e0x, cplx e0y, cplx e0z,
-                      double nx, double ny, double nz, cplx K, cplx Z, const double *kz, double2 *rhs)
+__global__ void __launch_bounds__(256)
+k_rhs(const double *V, const int *PVI, const double *PA, const int *EV, const int *EI,
+      const double *EL, int nE, int pec, double sgn, cplx e0x, cplx e0y, cplx e0z,
+      double nx, double ny, double nz, cplx K, cplx Z, const double *kz, double2 *rhs)
 {
-  int e = blockIdx.x * blockDim.x + threadIdx.x;
+  const int e = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (e >= nE) return;
   if (kz) { K = mk(kz[0], kz[1]); Z = mk(kz[2], kz[3]); }
   const cplx E0[3] = {e0x, e0y, e0z};
   const double nh[3] = {nx, ny, nz};
   const double *QP = V + 3 * EV[4 * e + 2], *V1 = V + 3 * EV[4 * e], *V2 = V + 3 * EV[4 * e + 1];
-  int pP = EI[4 * e], pM = EI[4 * e + 1];
-  double IP[4], IM[4] = {0, 0, 0, 0};
-  panel_ip(QP, V1, V2, QP, EL[e] / (2.0 * PA[pP]), E0, nh, K, Z, sgn, IP);
-  if (pM >= 0) {
-    const double *QM = V + 3 * EV[4 * e + 3];
-    panel_ip(V1, V2, QM, QM, EL[e] / (2.0 * PA[pM]), E0, nh, K, Z, sgn, IM);
+  const int pP = EI[4 * e], pM = EI[4 * e + 1];
+  const double *QM = pM >= 0 ? V + 3 * EV[4 * e + 3] : QP;
+  double I[4] = {0, 0, 0, 0};
+  // the plus panel (QP, V1, V2), then minus the minus panel (V1, V2, QM)
+  for (int t = lane; t < (pM >= 0 ? 156 : 78); t += 64) {
+    const bool minus = t >= 78;
+    const double *A = minus ? V1 : QP, *B = minus ? V2 : V1, *C = minus ? QM : V2, *Q = minus ? QM : QP;
+    const double pre = EL[e] / (2.0 * PA[minus ? pM : pP]);
+    panel_ip(A, B, C, Q, minus ? -pre : pre, E0, nh, K, Z, sgn, minus ? t - 78 : t, I);
   }
-  cplx EP = mk(IP[0] - IM[0], IP[1] - IM[1]), HP = mk(IP[2] - IM[2], IP[3] - IM[3]);
-  if (pec) rhs[e] = make_double2(EP.r / ZVAC_, EP.i / ZVAC_);
-  else { rhs[2 * e] = make_double2(EP.r / ZVAC_, EP.i / ZVAC_); rhs[2 * e + 1] = make_double2(HP.r, HP.i); }
+  for (int off = 32; off > 0; off >>= 1)
+    for (int q = 0; q < 4; q++) I[q] += __shfl_xor(I[q], off);
+  if (lane) return;
+  if (pec) rhs[e] = make_double2(I[0] / ZVAC_, I[1] / ZVAC_);
+  else { rhs[2 * e] = make_double2(I[0] / ZVAC_, I[1] / ZVAC_); rhs[2 * e + 1] = make_double2(I[2], I[3]); }
 }
 
 static bool g_tcr20_ready[64] = {false};
@@ -93,7 +101,7 @@ hipError_t launch_rhs(hipStream_t s, const double *V, const int *PVI, const doub
     g_tcr20_ready[dev & 63] = true;
   }
   if (nE <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rhs, dim3((nE + 63) / 64), dim3(64), 0, s, V, PVI, PA, EV, EI, EL, nE, pec, sgn,
+  hipLaunchKernelGGL(k_rhs, dim3((nE + 3) / 4), dim3(256), 0, s, V, PVI, PA, EV, EI, EL, nE, pec, sgn,
                      mk(E0[0].real(), E0[0].imag()), mk(E0[1].real(), E0[1].imag()), mk(E0[2].real(), E0[2].imag()),
                      nhat[0], nhat[1], nhat[2], mk(K.real(), K.imag()), mk(Z.real(), Z.imag()), kz, rhs);
   return hipGetLastError();
