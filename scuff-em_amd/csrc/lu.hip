@@ -1272,7 +1272,9 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   if (IsReal<T>::v) fast = 0;     // the explicit-inverse block rows are a complex64 option
   const bool tourn = fast && std::is_same<T, float2>::value && !partial_env;
   const bool g3m = tourn && mixed_gemm_3m();
+  int lrows = 0;
   const void *panel_one = panel_x_kernel<T>(true), *panel_two = panel_x_kernel<T>(false);
+  const void *panel_loc = panel_l_kernel<T>(&lrows);
   const void *panel_fn = tourn ? (const void *)k_panel_ts : Gmax <= PX_ONE ? panel_one : panel_two;
   int dev = 0, ncu = 0, perCU = 0;
   hipGetDevice(&dev);
@@ -1345,9 +1347,10 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
       // launch keeps it on the stream's own hardware queue (a cooperative
       // launch goes through a queue of its own, with a cross-queue handoff
       // before and after every panel)
-      hipError_t e = tourn ? hipLaunchKernel(panel_fn, dim3((unsigned)G + 1), dim3(NR), args, 0, stream)
-                           : hipLaunchKernel(G <= PX_ONE ? panel_one : panel_two, dim3((unsigned)G), dim3(NR), args, 0,
-                                             stream);
+      hipError_t e = tourn        ? hipLaunchKernel(panel_fn, dim3((unsigned)G + 1), dim3(NR), args, 0, stream)
+                     : m <= lrows ? hipLaunchKernel(panel_loc, dim3(1), dim3((unsigned)lrows), args, 0, stream)
+                                  : hipLaunchKernel(G <= PX_ONE ? panel_one : panel_two, dim3((unsigned)G), dim3(NR), args, 0,
+                                                    stream);
       // algorithmic flops of the m x w panel: per column, one complex
       // reciprocal-multiply per row below it and a complex rank-1 update
       double pflops = 0;

@@ -192,5 +192,8 @@ template <typename T> struct PXW { static const int n = 2 + PW * XW<T>::n; };   
 // arguments (T *A, long lda, long r0, long m, int w, int *ipiv, int *info,
 // PanelScratch S, int Gmax), one workgroup of 256 threads per 256 rows
 template <typename T> const void *panel_x_kernel(bool one);
+// the same for up to *rows rows, one workgroup of *rows threads: arguments
+// (T *A, long lda, long r0, long m, int w, int *ipiv, int *info, PanelScratch S)
+template <typename T> const void *panel_l_kernel(int *rows);
 
 }  // namespace scuffx

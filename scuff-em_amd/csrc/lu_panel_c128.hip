@@ -3,4 +3,5 @@
 
 namespace scuffx {
 template const void *panel_x_kernel<double2>(bool);
+template const void *panel_l_kernel<double2>(int *);
 }

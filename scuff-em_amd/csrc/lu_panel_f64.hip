@@ -3,4 +3,5 @@
 
 namespace scuffx {
 template const void *panel_x_kernel<double>(bool);
+template const void *panel_l_kernel<double>(int *);
 }
