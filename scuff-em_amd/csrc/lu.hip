@@ -1809,20 +1809,23 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
 // Workgroups take their place in solve order from a ticket, so a wait is
 // only ever for a workgroup that has started: any grid makes progress.
 // Every wait is bounded all the same.
-// The diagonal block is substituted, a wave for four columns, a lane for a
-// row: products with its explicit inverse are 2 us a step cheaper, but where
-// the block is badly scaled (eps = 10 spheres at imaginary frequency 0.001)
-// they lose every digit.  Its entries come in four sets of 16 columns, the
-// first loaded before the wait, the others while the one before is used.
+// The diagonal block is substituted in four sub-blocks of 16 rows: a lane
+// holds one row of one column (each wave four columns) and a step passes x_k
+// to the 16 lanes of its column by a row broadcast; the waves whose rows lie
+// further then subtract the sub-block's products on the matrix cores.  (A
+// lane for each of the 64 rows, x_k by lane reads, took 10 us a block in
+// complex128; products with the explicit inverse 2 us, but where the block is
+// badly scaled, eps = 10 spheres at imaginary frequency 0.001, they lose every
+// digit.)  The entries of the first sub-block are loaded before the wait.
 // bin: column-major right-hand sides, row r taken from pin[r] if given, or
 // null: packed in win.  bout: column-major results or null, row r to pout[r]
 // if given.  cj: 1 conjugates the right-hand sides, 2 the results in bout.
 // Bound: the chain of block steps up to a few hundred columns (a round trip,
 // 16 complex 16x16x4 products and 64 substitution steps per wave), the
-// matrix units past that.  N=3840 complex128: 17 us a step; 181 columns 2.8
+// matrix units past that.  N=3840 complex128: 12 us a step; 181 columns 2.1
 // ms, where substitution in 256-row blocks by one workgroup a column and GEMM
-// updates took 6.0; one transposed system 2.4 ms, where a single workgroup
-// with a reduction per row took 24; 1920 columns 7.2 ms (31 TFLOP/s).
+// updates took 6.0; one transposed system 1.7 ms, where a single workgroup
+// with a reduction per row took 24; 1920 columns 6.4 ms (35 TFLOP/s).
 template <typename T> struct ChainArgs {
   const T *A; long lda; long n;
   const T *bin; long ldb; const int *pin; const T *win;
@@ -1830,20 +1833,42 @@ template <typename T> struct ChainArgs {
   long nrhs; int cj; unsigned *err, *ticket;
 };
 
-// acc += a x for 16 k-steps of the matrix instruction
+// acc += a x for one and for 16 k-steps of the matrix instruction
+template <typename T>
+__device__ inline void chain_mac1(T a, T x, typename CT<T>::V4 &re, typename CT<T>::V4 &im)
+{
+  if constexpr (IsReal<T>::v) re = CT<T>::mfma(a, x, re);
+  else {
+    re = CT<T>::mfma(a.x, x.x, re);
+    im = CT<T>::mfma(a.x, x.y, im);
+    re = CT<T>::mfma(-a.y, x.y, re);
+    im = CT<T>::mfma(a.y, x.x, im);
+  }
+}
 template <typename T>
 __device__ inline void chain_mac(const T (&a)[16], const T (&x)[16], typename CT<T>::V4 &re, typename CT<T>::V4 &im)
 {
 #pragma unroll
-  for (int s = 0; s < 16; s++) {
-    if constexpr (IsReal<T>::v) re = CT<T>::mfma(a[s], x[s], re);
-    else {
-      re = CT<T>::mfma(a[s].x, x[s].x, re);
-      im = CT<T>::mfma(a[s].x, x[s].y, im);
-      re = CT<T>::mfma(-a[s].y, x[s].y, re);
-      im = CT<T>::mfma(a[s].y, x[s].x, im);
-    }
-  }
+  for (int s = 0; s < 16; s++) chain_mac1<T>(a[s], x[s], re, im);
+}
+// v of lane k of this lane's row of 16
+template <int K> __device__ inline float row_bcast(float v)
+{
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + K, 0xF, 0xF, false));
+}
+template <int K> __device__ inline double row_bcast(double v)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xFFFFFFFF), 0x150 + K, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + K, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+template <int K, typename T> __device__ inline T row_bcast(T v)
+{
+  T r;
+  r.x = row_bcast<K>(v.x);
+  r.y = row_bcast<K>(v.y);
+  return r;
 }
 template <typename T> __device__ inline T chain_elem(typename CT<T>::V4 re, typename CT<T>::V4 im, int r)
 {
@@ -1887,23 +1912,26 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
       }
     }
   };
-  // set u of the diagonal block in solve order: this lane's row of columns
-  // 16 u .. (FWD) or 63 - 16 u, .. (clamped past the edge, where nothing
-  // uses the values)
+  // sub-block u in solve order covers the rows from sub(u); its diagonal part:
+  // this lane's row i (clamped past the edge, where nothing uses the values),
+  // columns in solve order; the part left of wave row w0 for its k-steps
   const T *Ad = p.A + g * TB * (lda + 1);
+  auto sub = [&](int u) { return 16 * (FWD ? u : 3 - u); };
+  auto at = [&](int r, int k) { return TRANS ? Ad[min(k, bs - 1) + min(r, bs - 1) * lda] : Ad[min(r, bs - 1) + min(k, bs - 1) * lda]; };
   auto dload = [&](int u, T (&d)[16]) {
-    const int r = min(lane, bs - 1);
 #pragma unroll
-    for (int s = 0; s < 16; s++) {
-      const int k = min(FWD ? 16 * u + s : TB - 1 - 16 * u - s, bs - 1);
-      d[s] = TRANS ? Ad[k + r * lda] : Ad[r + k * lda];
-    }
+    for (int s = 0; s < 16; s++) d[s] = at(sub(u) + i, sub(u) + (FWD ? s : 15 - s));
   };
-  // the first set, the diagonal's reciprocal and the right-hand side,
+  auto fload = [&](int u, T (&f)[16]) {       // f[4 u ..]
+#pragma unroll
+    for (int s = 0; s < 4; s++) f[4 * u + s] = at(w0 + i, sub(u) + 4 * s + kq);
+  };
+  // the first sub-block, the diagonal's reciprocals and the right-hand side,
   // loaded ahead
-  T m[16], b[4], rd = unit_v<T>();
+  T m[16], b[4], rd[4];
   dload(0, m);
-  if (!UNIT && lane < bs) rd = crecip(Ad[lane * (lda + 1)]);
+#pragma unroll
+  for (int u = 0; u < 4; u++) rd[u] = UNIT ? unit_v<T>() : sub(u) + i < bs ? crecip(at(sub(u) + i, sub(u) + i)) : unit_v<T>();
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int br = w0 + CT<T>::row(lane, r);
@@ -1941,43 +1969,47 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
       im = CT<T>::zero();
     }
   }
-  dload(1, x);
-  dload(2, a);
+  // this wave's place in the block's solve order, its columns
+  const int me = FWD ? w0 / 16 : 3 - w0 / 16, c4 = w0 / 4;
+  dload(1, a);
 #pragma unroll
-  for (int r = 0; r < 4; r++) sb[w0 + CT<T>::row(lane, r)][i] = csub(b[r], chain_elem<T>(re, im, r));
-  __syncthreads();
-  const int c4 = w0 / 4;                 // this wave's four columns
-  if (tile * NC + c4 < p.nrhs) {
-    T y[4];
+  for (int u = 0; u < 3; u++)
+    if (u < me) fload(u, x);
+  auto rest = [&]() {      // what is left of this wave's rows
 #pragma unroll
-    for (int c = 0; c < 4; c++) y[c] = sb[lane][c4 + c];
-    auto steps = [&](int u, const T (&d)[16]) __attribute__((always_inline)) {
+    for (int r = 0; r < 4; r++) sb[w0 + CT<T>::row(lane, r)][i] = csub(b[r], chain_elem<T>(re, im, r));
+  };
 #pragma unroll
-      for (int s = 0; s < 16; s++) {
-        const int k = FWD ? 16 * u + s : TB - 1 - 16 * u - s;
-        if (k < bs) {
-          const T rk = readlane_t(rd, k);
-#pragma unroll
-          for (int c = 0; c < 4; c++) {
-            T v = readlane_t(y[c], k);
-            if (!UNIT) {
-              v = cmul(v, rk);
-              if (lane == k) y[c] = v;
-            }
-            if (FWD ? lane > k : lane < k) y[c] = fnma_t(y[c], d[s], v);
-          }
-        }
-      }
-    };
-    steps(0, m);
-    dload(3, m);
-    steps(1, x);
-    steps(2, a);
-    steps(3, m);
-#pragma unroll
-    for (int c = 0; c < 4; c++) sb[lane][c4 + c] = lane < bs ? y[c] : zero_v<T>();
+  for (int r = 0; r < 4; r++) {
+    const int br = w0 + CT<T>::row(lane, r);
+    b[r] = br < bs ? csub(b[r], chain_elem<T>(re, im, r)) : zero_v<T>();
   }
-  __syncthreads();
+  re = CT<T>::zero();
+  im = CT<T>::zero();
+  auto solve = [&](auto uc, T (&d)[16]) __attribute__((always_inline)) {
+    constexpr int u = decltype(uc)::value;
+    if (me == u) rest();
+    __syncthreads();
+    T y = sub(u) + i < bs ? sb[sub(u) + i][c4 + kq] : zero_v<T>();
+    static_for<0, 15>([&](auto sc) __attribute__((always_inline)) {
+      constexpr int s = decltype(sc)::value, k = FWD ? s : 15 - s;
+      const T v = row_bcast<k>(UNIT ? y : cmul(y, rd[u]));
+      if (FWD ? i > k : i < k) y = fnma_t(y, d[s], v);
+    });
+    if (!UNIT) y = cmul(y, rd[u]);
+    sb[sub(u) + i][c4 + kq] = y;
+    __syncthreads();
+    if (u < me) {
+#pragma unroll
+      for (int s = 0; s < 4; s++) chain_mac1<T>(x[4 * u + s], sb[sub(u) + 4 * s + kq][i], re, im);
+    }
+  };
+  solve(std::integral_constant<int, 0>{}, m);
+  dload(2, m);
+  solve(std::integral_constant<int, 1>{}, a);
+  dload(3, a);
+  solve(std::integral_constant<int, 2>{}, m);
+  solve(std::integral_constant<int, 3>{}, a);
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int br = w0 + kq + 4 * r;

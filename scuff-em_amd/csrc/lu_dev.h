@@ -178,6 +178,17 @@ __device__ inline unsigned wave_max_key(unsigned k)
   return max(max(a, b), max(c, d));
 }
 
+// f(0), f(1), .. f(N - 1) with compile-time indices (a loop of this size is
+// past the compiler's limit for unrolling, and a rolled one would index the
+// row's registers, i.e. keep it in scratch memory)
+template <int J, int N, typename F> __device__ __attribute__((always_inline)) inline void static_for(F &&f)
+{
+  if constexpr (J < N) {
+    f(std::integral_constant<int, J>{});
+    static_for<J + 1, N>(f);
+  }
+}
+
 // slots of the exact panel's exchange area (lu_panel.hip): one per column
 // and workgroup, 64-bit words {key, position, the candidate row}
 template <typename T> struct XW;          // 64-bit words of one entry
