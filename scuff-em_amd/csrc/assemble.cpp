@@ -960,8 +960,19 @@ int Assembler::assemble_block(int sa, int sb, cdouble omega, double2 *B, long ld
     std::memset(&GS, 0, sizeof(GS));
     GS.n = ntorque;
     for (int i = 0; i < 9 * ntorque; i++) GS.g[i] = gamma[i];
-    HIPCHK(launch_grad(stream, DA.nE, DA.EI, DA.EL, DA.V, DA.PVI, DA.PC, DB.nE, DB.EI, DB.EL, DB.V, DB.PVI, DB.PC,
-                       SA.IsPEC, SB.IsPEC, ng, d_regs_ + 2, GB, ldg, gstride, GS, TB));
+    // (the block's column bands are those of its orientation lo, hi)
+    if (SA.IsPEC && SB.IsPEC && ntorque == 0 && sa < sb) {
+      const FarBands &F = NB.bands;
+      if (ensure(&d_HP_, &cap_HP_, (size_t)std::max(F.maxSlots, 1) * F.rowsCap * std::max(ng, 1) * 54)) return -2;
+      for (int k = 0; k < F.count(); k++) {
+        const int c0 = F.colStart[k], s0 = F.slotStart[k];
+        HIPCHK(launch_grad_band(stream, DA.nE, DA.EI, DA.EL, DA.V, DA.PVI, DA.PC, DA.nP, DB.EI, DB.EL, DB.V, DB.PVI,
+                                DB.PC, F.d_slots + s0, F.slotStart[k + 1] - s0, F.d_cols + c0, F.d_colSlots + 2 * c0,
+                                F.colStart[k + 1] - c0, ng, d_regs_ + 2, d_HP_, F.rowsCap, GB, ldg, gstride));
+      }
+    } else
+      HIPCHK(launch_grad(stream, DA.nE, DA.EI, DA.EL, DA.V, DA.PVI, DA.PC, DB.nE, DB.EI, DB.EL, DB.V, DB.PVI, DB.PC,
+                         SA.IsPEC, SB.IsPEC, ng, d_regs_ + 2, GB, ldg, gstride, GS, TB));
     prof_end(stream, tok, 0.0);
   }
   HIPCHK(hipStreamSynchronize(stream));

@@ -114,6 +114,13 @@ struct GammaSet {
   int n;
   double g[27];
 };
+// the same for perfectly conducting surfaces, one column band of the block
+// (no axes): HB holds nslots x rowsCap records of 54 doubles per region
+hipError_t launch_grad_band(hipStream_t stream, int nEa, const int *EIa, const double *ELa, const double *Va,
+                            const int *PVIa, const double *PCa, int nPa, const int *EIb, const double *ELb,
+                            const double *Vb, const int *PVIb, const double *PCb, const int *slotPanels, int nslots,
+                            const int *bandCols, const int *colSlots, int ncols, int nreg, const RegionK *regs,
+                            double *HB, long rowsCap, double2 *GB, long ldg, long gstride);
 hipError_t launch_grad(hipStream_t stream, int nEa, const int *EIa, const double *ELa, const double *Va,
                        const int *PVIa, const double *PCa, int nEb, const int *EIb, const double *ELb,
                        const double *Vb, const int *PVIb, const double *PCb, int pecA, int pecB, int nreg,

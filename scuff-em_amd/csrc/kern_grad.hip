@@ -67,8 +67,11 @@ __device__ void ppi_grad(const double *Va0, const double *Va1, const double *Va2
         R[c] = X[c] - XP;
       }
       double r2 = R[0] * R[0] + R[1] * R[1] + R[2] * R[2], r = sqrt(r2), ir = 1.0 / r;
-      double e = exp(-k.i * r), sn, cs;
-      sincos(k.r * r, &sn, &cs);
+      // (real and imaginary wavenumbers skip the exponential or the sine and
+      // cosine: exact there)
+      double e = 1.0, sn = 0.0, cs = 1.0;
+      if (k.i != 0) e = exp(-k.i * r);
+      if (k.r != 0) sincos(k.r * r, &sn, &cs);
       cplx Phi = mk(e * cs, e * sn) * (SCUFFX_INV4PI_G * ir * wp);
       cplx Psi = Phi * (ik - mk(ir, 0)) * ir;
       cplx Zeta = Phi * (ik2 - 3.0 * ir * ik + mk(3.0 * ir * ir, 0)) * (ir * ir);
@@ -162,13 +165,133 @@ k_grad_stamp(int nEa, const int *EIa, const double *ELa, const double *Va, const
   }
 }
 
+// Between perfectly conducting surfaces only dH0 is wanted, and a panel pair's
+// integrals serve the nine edge pairs that meet it.  With x, y from the
+// panels' centroids, R = D + x - y,
+//   dH0/dx_m (Qa, Qb) = A_m - Qb.B_m - Qa.C_m + (Qa.Qb + 4/(ik)^2) E_m,
+//   A_m = sum R_m (x.y) Psi, B_m = sum R_m x Psi, C_m = sum R_m y Psi,
+//   E_m = sum R_m Psi,
+// and the sums over y for one x need sum {1, y, y y} Psi only (ten words).
+// One thread per (row panel, slot) writes the 9 x 3 values of each region; the
+// band's column edges are then combined from them, as the matrix is.  Bound:
+// FP64 vector rate.  Two N=1920 spheres: under 0.9 ms, where each edge pair
+// integrated its four panel pairs by itself in 8.7.
+__global__ void __launch_bounds__(128)
+k_grad_pair(const double *Va, const int *PVIa, const double *PCa, int nPa, const double *Vb, const int *PVIb,
+            const double *PCb, const int *slotPanels, int nreg, const RegionK *regs, double *HB, long rowsCap)
+{
+#pragma clang fp contract(fast)
+  const int pa = blockIdx.x * blockDim.x + threadIdx.x, slot = blockIdx.y;
+  if (pa >= nPa) return;
+  const int pb = slotPanels[slot];
+  double Pa[9], Pb[9], D[3];            // vertices from the centroids
+  for (int c = 0; c < 3; c++) {
+    for (int v = 0; v < 3; v++) {
+      Pa[3 * v + c] = Va[3 * PVIa[3 * pa + v] + c] - PCa[4 * pa + c];
+      Pb[3 * v + c] = Vb[3 * PVIb[3 * pb + v] + c] - PCb[4 * pb + c];
+    }
+    D[c] = PCa[4 * pa + c] - PCb[4 * pb + c];
+  }
+  // relative centroid distance (AssessPanelPair.cc:161-166)
+  const double rRel = sqrt(D[0] * D[0] + D[1] * D[1] + D[2] * D[2]) / fmax(PCa[4 * pa + 3], PCb[4 * pb + 3]);
+  const double *rule = rRel > 4.0 ? c_gtcr4 : c_gtcr20;
+  const int np = rRel > 4.0 ? 6 : 78;
+  for (int r = 0; r < nreg; r++) {
+    const cplx k = regs[r].k;
+    cplx A[3], B[3][3], C[3][3], E[3];
+    for (int m = 0; m < 3; m++) {
+      A[m] = mk(0, 0); E[m] = mk(0, 0);
+      for (int c = 0; c < 3; c++) { B[m][c] = mk(0, 0); C[m][c] = mk(0, 0); }
+    }
+#pragma unroll 1
+    for (int i = 0; i < np; i++) {
+      const double u = rule[3 * i], v = rule[3 * i + 1], w = rule[3 * i + 2] * SCUFFX_INV4PI_G;
+      double x[3], Dx[3];
+      for (int c = 0; c < 3; c++) {
+        x[c] = Pa[c] + u * (Pa[3 + c] - Pa[c]) + v * (Pa[6 + c] - Pa[c]);
+        Dx[c] = D[c] + x[c];
+      }
+      cplx q0 = mk(0, 0), q[3], Q[6];     // Q: xx, yy, zz, xy, xz, yz
+      for (int c = 0; c < 3; c++) q[c] = mk(0, 0);
+      for (int c = 0; c < 6; c++) Q[c] = mk(0, 0);
+#pragma unroll 1
+      for (int j = 0; j < np; j++) {
+        const double up = rule[3 * j], vp = rule[3 * j + 1];
+        double y[3], R[3];
+        for (int c = 0; c < 3; c++) {
+          y[c] = Pb[c] + up * (Pb[3 + c] - Pb[c]) + vp * (Pb[6 + c] - Pb[c]);
+          R[c] = Dx[c] - y[c];
+        }
+        const double rr = sqrt(R[0] * R[0] + R[1] * R[1] + R[2] * R[2]), ir = 1.0 / rr;
+        double e = rule[3 * j + 2] * ir, sn = 0.0, cs = 1.0;
+        if (k.i != 0) e *= exp(-k.i * rr);
+        if (k.r != 0) sincos(k.r * rr, &sn, &cs);
+        // Psi = Phi (ik - 1/r) / r
+        const double a = -(k.i + ir) * ir, b = k.r * ir, fr = e * cs, fi = e * sn;
+        const cplx g = mk(fr * a - fi * b, fr * b + fi * a);
+        q0 += g;
+        for (int c = 0; c < 3; c++) q[c] += y[c] * g;
+        Q[0] += (y[0] * y[0]) * g; Q[1] += (y[1] * y[1]) * g; Q[2] += (y[2] * y[2]) * g;
+        Q[3] += (y[0] * y[1]) * g; Q[4] += (y[0] * y[2]) * g; Q[5] += (y[1] * y[2]) * g;
+      }
+      for (int m = 0; m < 3; m++) {
+        const cplx N = w * (Dx[m] * q0 - q[m]);
+        E[m] += N;
+        for (int c = 0; c < 3; c++) {
+          const cplx M = w * (Dx[m] * q[c] - Q[c == m ? c : c + m + 2]);
+          A[m] += x[c] * M;
+          B[m][c] += x[c] * N;
+          C[m][c] += M;
+        }
+      }
+    }
+    const cplx ik = IMUL(k), c4 = 4.0 / (ik * ik);
+    double *out = HB + (((long)slot * rowsCap + pa) * nreg + r) * 54;
+    for (int a = 0; a < 3; a++)
+      for (int b = 0; b < 3; b++) {
+        const double *qa = Pa + 3 * a, *qb = Pb + 3 * b;
+        const cplx qq = mk(dot3(qa, qb), 0) + c4;
+        for (int m = 0; m < 3; m++) {
+          cplx h = A[m] + qq * E[m];
+          for (int c = 0; c < 3; c++) h = h - qb[c] * B[m][c] - qa[c] * C[m][c];
+          double *o = out + (3 * (3 * a + b) + m) * 2;
+          o[0] = h.r; o[1] = h.i;
+        }
+      }
+  }
+}
+
+// the band's column edges from its records: grid.y = column edge
+__global__ void __launch_bounds__(256)
+k_grad_comb(int nEa, const int *EIa, const double *ELa, const int *bandCols, const int *colSlots, const int *EIb,
+            const double *ELb, int nreg, const RegionK *regs, const double *HB, long rowsCap, double2 *GB, long ldg,
+            long gstride)
+{
+  const int ea = blockIdx.x * blockDim.x + threadIdx.x, j = blockIdx.y;
+  if (ea >= nEa) return;
+  const int eb = bandCols[j];
+  const double LL = ELa[ea] * ELb[eb];
+  cplx m00[3] = {mk(0, 0), mk(0, 0), mk(0, 0)};
+  for (int r = 0; r < nreg; r++) {
+    cplx S[3] = {mk(0, 0), mk(0, 0), mk(0, 0)};
+#pragma unroll
+    for (int st = 0; st < 4; st++) {
+      const int s = st >> 1, t = st & 1;
+      const int pa = EIa[4 * ea + s], pb = EIb[4 * eb + t];
+      if (pa < 0 || pb < 0) continue;
+      const int q = 3 * EIa[4 * ea + 2 + s] + EIb[4 * eb + 2 + t];
+      const double *h = HB + (((long)colSlots[2 * j + t] * rowsCap + pa) * nreg + r) * 54 + 6 * q;
+      const double sg = s == t ? 1.0 : -1.0;
+      for (int m = 0; m < 3; m++) S[m] += sg * mk(h[2 * m], h[2 * m + 1]);
+    }
+    for (int m = 0; m < 3; m++) m00[m] += regs[r].pf1 * (LL * S[m]);
+  }
+  for (int m = 0; m < 3; m++) GB[(long)m * gstride + ea + (long)eb * ldg] = make_double2(m00[m].r, m00[m].i);
+}
+
 static bool g_gtcr20_ready[64] = {false};
 
-hipError_t launch_grad(hipStream_t stream, int nEa, const int *EIa, const double *ELa, const double *Va,
-                       const int *PVIa, const double *PCa, int nEb, const int *EIb, const double *ELb,
-                       const double *Vb, const int *PVIb, const double *PCb, int pecA, int pecB, int nreg,
-                       const RegionK *regs, double2 *GB, long ldg, long gstride, const GammaSet &GS,
-                       double2 *TB)
+static hipError_t grad_tables()
 {
   int dev = 0;
   hipGetDevice(&dev);
@@ -177,6 +300,34 @@ hipError_t launch_grad(hipStream_t stream, int nEa, const int *EIa, const double
     if (e != hipSuccess) return e;
     g_gtcr20_ready[dev & 63] = true;
   }
+  return hipSuccess;
+}
+
+hipError_t launch_grad_band(hipStream_t stream, int nEa, const int *EIa, const double *ELa, const double *Va,
+                            const int *PVIa, const double *PCa, int nPa, const int *EIb, const double *ELb,
+                            const double *Vb, const int *PVIb, const double *PCb, const int *slotPanels, int nslots,
+                            const int *bandCols, const int *colSlots, int ncols, int nreg, const RegionK *regs,
+                            double *HB, long rowsCap, double2 *GB, long ldg, long gstride)
+{
+  if (nPa <= 0 || nslots <= 0 || ncols <= 0 || nEa <= 0) return hipSuccess;
+  hipError_t e = grad_tables();
+  if (e != hipSuccess) return e;
+  if (nreg > 0)
+    hipLaunchKernelGGL(k_grad_pair, dim3((nPa + 127) / 128, nslots), dim3(128), 0, stream, Va, PVIa, PCa, nPa, Vb, PVIb,
+                       PCb, slotPanels, nreg, regs, HB, rowsCap);
+  hipLaunchKernelGGL(k_grad_comb, dim3((nEa + 255) / 256, ncols), dim3(256), 0, stream, nEa, EIa, ELa, bandCols,
+                     colSlots, EIb, ELb, nreg, regs, HB, rowsCap, GB, ldg, gstride);
+  return hipGetLastError();
+}
+
+hipError_t launch_grad(hipStream_t stream, int nEa, const int *EIa, const double *ELa, const double *Va,
+                       const int *PVIa, const double *PCa, int nEb, const int *EIb, const double *ELb,
+                       const double *Vb, const int *PVIb, const double *PCb, int pecA, int pecB, int nreg,
+                       const RegionK *regs, double2 *GB, long ldg, long gstride, const GammaSet &GS,
+                       double2 *TB)
+{
+  hipError_t e = grad_tables();
+  if (e != hipSuccess) return e;
   if (nEa <= 0 || nEb <= 0) return hipSuccess;
   dim3 grid((nEa + 127) / 128, nEb);
   hipLaunchKernelGGL(k_grad_stamp, grid, dim3(128), 0, stream, nEa, EIa, ELa, Va, PVIa, PCa, nEb, EIb, ELb, Vb,

@@ -163,7 +163,8 @@ struct RowSums {
 // vector products 27 operations more.  sy: the points of the second panel
 // (one panel for the whole workgroup); sp: per thread the first panel as {V0 -
 // centroid, V1 - V0, V2 - V0} and D, in LDS, so that the point loop, rolled,
-// keeps to 256 registers (two waves per SIMD).  Bound: FP64 vector rate; FARNUM
+// keeps to 256 registers (two waves per SIMD).  Bound: FP64 vector rate.
+// N=3840 dielectric, 1.8 million pairs and two regions: 425 us (617 before)
 __device__ inline void pair_moments_far(const double (*sp)[256], const double (*sy)[3], cplx k, int needH1, Moments &m)
 {
 #pragma clang fp contract(fast)

