@@ -1218,11 +1218,111 @@ k_trsm_blk(const T *A, long lda, long r0, int jb, const T *linv, T *B, long ldb,
   if (row < jb) B[row + c * ldb] = b;
 }
 
+// The same solve where columns are many (complex64, jb = 16 NT): a wave
+// holds 16 columns of all jb rows in the matrix unit's result layout, lane (j,
+// q) rows 4 q + r of column j in word r, which is also the layout of a right
+// operand whose k-step r takes rows 4 q + r: products feed products without
+// leaving the registers, and no wave waits for another.  Bound: the matrix
+// units, 32 cycles an instruction (576 for 128 rows).  A wave per 64 rows of
+// one column by lane reads (k_trsm_blk, still better for a single
+// factorization's next 256 columns, where only 16 waves would run) took 358 us
+// a launch in the batch of 32 at N=3840, this one 73.
+template <int NT>
+__global__ void __launch_bounds__(256)
+k_trsm_mm(const float2 *A, long lda, long r0, const float2 *linv, float2 *B, long ldb, long ncol, BStride bs)
+{
+  typedef CT<float2> M;
+  {
+    const long bi = blockIdx.y;   // instance of a batch
+    A += bi * bs.a;
+    B += bi * bs.a;
+    linv = bshift(linv, bi * bs.s);
+  }
+  const int lane = threadIdx.x & 63, j = lane & 15, q = lane >> 4;
+  const long c0 = ((long)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
+  if (c0 >= ncol) return;
+  float2 *Bc = B + 4 * q + min(c0 + j, ncol - 1) * ldb;
+  f4 br[NT], bi[NT];
+#pragma unroll
+  for (int t = 0; t < NT; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const float2 v = Bc[16 * t + r];
+      br[t][r] = v.x;
+      bi[t][r] = v.y;
+    }
+  // acc += s a x
+  auto mac = [&](float2 a, float xr, float xi, f4 &re, f4 &im) __attribute__((always_inline)) {
+    re = M::mfma(a.x, xr, re);
+    im = M::mfma(a.x, xi, im);
+    re = M::mfma(-a.y, xi, re);
+    im = M::mfma(a.y, xr, im);
+  };
+  const float2 *Ap = A + (r0 + j) + (r0 + 4 * q) * lda;
+#pragma unroll
+  for (int i = 0; i < NT / 2; i++) {
+    // X = Linv_i B_i (its upper right 16 x 16 part is zero)
+    const float2 *Li = linv + (long)i * PW * PW + j + 4 * q * PW;
+    f4 xr[2], xi[2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      xr[u] = M::zero();
+      xi[u] = M::zero();
+#pragma unroll
+      for (int t = 0; t <= u; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+          mac(Li[16 * u + (16 * t + r) * PW], br[2 * i + t][r], bi[2 * i + t][r], xr[u], xi[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+      br[2 * i + u] = xr[u];
+      bi[2 * i + u] = xi[u];
+    }
+    // the rows below: B_k -= L_ki X
+#pragma unroll
+    for (int k = 2 * i + 2; k < NT; k++)
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          float2 a = Ap[16 * k + (PW * i + 16 * t + r) * lda];
+          a.x = -a.x;
+          a.y = -a.y;
+          mac(a, xr[t][r], xi[t][r], br[k], bi[k]);
+        }
+  }
+  if (c0 + j < ncol) {
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) Bc[16 * t + r] = make_float2(br[t][r], bi[t][r]);
+  }
+}
+
+// whether it takes a solve: its block widths, and 4096 columns, i.e. a wave for
+// a quarter of the SIMDs.  The N=15360 mixed solve takes 136.9 ms with this
+// line, 138.9 with 16384, 138.5 without the kernel and 143.8 with it for every
+// solve; the batch 149.2, 150.0 and 161.0
+static bool trsm_mm(const float2 *A, long lda, long r0, int jb, const float2 *linv, float2 *B, long ldb, long ncol,
+                    hipStream_t s, int nbat = 1, BStride bs = BStride())
+{
+  if ((jb != 128 && jb != 256) || ncol * nbat < 4096) return false;
+  int tok = prof_begin(s, PK_TRSM_C64);
+  const dim3 grid((unsigned)((ncol + 63) / 64), (unsigned)nbat);
+  if (jb == 128) hipLaunchKernelGGL(k_trsm_mm<8>, grid, dim3(256), 0, s, A, lda, r0, linv, B, ldb, ncol, bs);
+  else hipLaunchKernelGGL(k_trsm_mm<16>, grid, dim3(256), 0, s, A, lda, r0, linv, B, ldb, ncol, bs);
+  prof_end(s, tok, 4.0 * (double)jb * (double)jb * (double)ncol * nbat);
+  return true;
+}
+
 template <typename T>
 static void trsm_blk(const T *A, long lda, long r0, int jb, const T *linv, T *B, long ldb, long ncol, hipStream_t s,
                      int nbat = 1, BStride bs = BStride())
 {
   if (ncol <= 0 || jb <= 0) return;
+  if constexpr (std::is_same<T, float2>::value)
+    if (trsm_mm(A, lda, r0, jb, linv, B, ldb, ncol, s, nbat, bs)) return;
   int tok = prof_begin(s, std::is_same<T, double2>::value ? PK_TRSM_C128 : PK_TRSM_C64);
   // one wave per 64 rows of the block: two for a 128-column block
   const unsigned nthr = jb <= 128 ? 128u : 256u;
@@ -1397,7 +1497,13 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
       laswp_plans(A, lda, c2, n, 0, 0, plans + p0 * PLAN_LEN, bplans, side);
       if (fast) {
         if constexpr (!IsReal<T>::v)
-          trsm_block_inv(A, lda, K, (int)jb, (const T *)S.linv + p0 * PW * PW, A + K + c2 * lda, lda, n - c2, side);
+          {
+            const T *li = (const T *)S.linv + p0 * PW * PW;
+            bool done = false;
+            if constexpr (std::is_same<T, float2>::value)
+              done = trsm_mm(A, lda, K, (int)jb, li, A + K + c2 * lda, lda, n - c2, side);
+            if (!done) trsm_block_inv(A, lda, K, (int)jb, li, A + K + c2 * lda, lda, n - c2, side);
+          }
       } else
         trsm_block(A, lda, K, (int)jb, A + K + c2 * lda, lda, n - c2, side);
       // beside tournament panels: at most three trailing-GEMM workgroups

@@ -126,3 +126,29 @@ def test_block_inverses_low_frequency(sx, O):
     _, rel, info = sx.SweepBatched(Gs, np.array([0.049, 0.058, 0.067, 0.079]), pw)
     assert info[0] == 0
     assert np.max(rel) <= 2e-12, rel
+
+
+# the mixed factorization's block rows on the matrix units: past 4096 columns
+# right of the next block, a number of columns that is no multiple of 16 and an
+# odd leading dimension
+def test_mixed_wide_block_rows(sx):
+    import torch
+    n = 4699
+    print(f"mixed block rows n={n}", flush=True)
+    A = matrix(n, "complex64", 11)
+    M = sx.HMatrix.from_numpy(A.astype("complex128"))
+    LU32 = torch.zeros((n, n), dtype=torch.complex64, device="cuda")
+    ipiv = torch.zeros(n, dtype=torch.int32, device="cuda")
+    assert sx.lib().scuffx_lu32_from_c128(sx._ptr(M.t), n, n, sx._ptr(LU32), n, sx._ptr(ipiv)) == 0
+    F, piv = LU32.cpu().numpy().T, ipiv.cpu().numpy()
+    perm = np.arange(n)
+    for i in range(n):
+        perm[[i, piv[i] - 1]] = perm[[piv[i] - 1, i]]
+    # P A v = L (U v) for a few vectors, against |L| |U| of a random matrix
+    # (2e-5 sqrt(n / 40) relative to |A|, as for the smaller orders)
+    v = matrix(8, "complex128", 3)[0][:4]
+    V = np.outer(np.ones(n), v) * np.random.default_rng(4).standard_normal((n, 4))
+    UV = np.triu(F).astype("complex128") @ V
+    LUV = np.tril(F, -1).astype("complex128") @ UV + UV
+    res = np.linalg.norm(A.astype("complex128")[perm] @ V - LUV) / (np.linalg.norm(A) * np.linalg.norm(V) / np.sqrt(n))
+    assert res <= 2e-5 * np.sqrt(n / 40), res
