@@ -20,6 +20,7 @@
 #include <algorithm>
 
 #include "bem.h"
+#include "exprel.h"
 
 namespace scuffx {
 
@@ -49,59 +50,6 @@ struct Moments {
   cplx s, u[3], v[3], w[3];
 };
 
-template <int DESING>
-__device__ inline void pair_moments(const double *xi, const double *eta, const double *D,
-                                    cplx k, int needH1, Moments &m)
-{
-#pragma clang fp contract(fast)
-  m.S1 = mk(0, 0); m.Sxy = mk(0, 0); m.s = mk(0, 0);
-  for (int c = 0; c < 3; c++) { m.Sx[c] = mk(0, 0); m.Sy[c] = mk(0, 0); m.u[c] = mk(0, 0); m.v[c] = mk(0, 0); m.w[c] = mk(0, 0); }
-  cplx ik = IMUL(k);
-  for (int i = 0; i < 6; i++) {
-    const double wi = c_tcr4[3 * i + 2];
-    const double *x = xi + 3 * i;
-    for (int j = 0; j < 6; j++) {
-      const double wj = c_tcr4[3 * j + 2];
-      const double *y = eta + 3 * j;
-      double R[3] = {D[0] + x[0] - y[0], D[1] + x[1] - y[1], D[2] + x[2] - y[2]};
-      double r2 = R[0] * R[0] + R[1] * R[1] + R[2] * R[2];
-      double r = sqrt(r2);
-      double ir = 1.0 / r;
-      cplx Phi;
-      if (DESING) {
-        // ExpRel(ikr,4) = sum_{m>=4} (ikr)^m/m!, stopped at |term|<1e-8|sum|
-        // (PanelPanelInteractions.cc:84-103)
-        cplx z = ik * r, term = mk(1, 0), sum = mk(0, 0);
-        int q;
-        for (q = 1; q < 4; q++) term = term * (z / (double)q);
-        for (; q < 100; q++) {
-          term = term * (z / (double)q);
-          sum += term;
-          if (norm2(term) < 1.0e-16 * norm2(sum)) break;
-        }
-        Phi = sum * (SCUFFX_INV4PI * ir);
-      } else {
-        double e = exp(-k.i * r), sn, cs;
-        sincos(k.r * r, &sn, &cs);
-        Phi = mk(e * cs, e * sn) * (SCUFFX_INV4PI * ir);
-      }
-      Phi = Phi * (wi * wj);
-      m.S1 += Phi;
-      for (int c = 0; c < 3; c++) { m.Sx[c] += x[c] * Phi; m.Sy[c] += y[c] * Phi; }
-      m.Sxy += (x[0] * y[0] + x[1] * y[1] + x[2] * y[2]) * Phi;
-      if (needH1) {
-        cplx Psi = Phi * (ik - mk(ir, 0)) * ir;
-        double xy[3], Rx[3], yR[3];
-        cross3(x, y, xy);
-        cross3(R, x, Rx);
-        cross3(y, R, yR);
-        m.s += (xy[0] * R[0] + xy[1] * R[1] + xy[2] * R[2]) * Psi;
-        for (int c = 0; c < 3; c++) { m.u[c] += Rx[c] * Psi; m.v[c] += yR[c] * Psi; m.w[c] += R[c] * Psi; }
-      }
-    }
-  }
-}
-
 // one (Qa, Qb) source-vertex combination of a pair's moments
 __device__ inline void combo_ab(const Moments &m, const double *qa, const double *qb, cplx c4, int needH1, cplx *h0,
                                 cplx *h1)
@@ -117,15 +65,6 @@ __device__ inline void combo_ab(const Moments &m, const double *qa, const double
     for (int c = 0; c < 3; c++) t = t - qb[c] * m.u[c] - qa[c] * m.v[c] + qq[c] * m.w[c];
     *h1 = t;
   }
-}
-
-__device__ inline void combos_from_moments(const Moments &m, const double *Qa, const double *Qb,
-                                           cplx k, int needH1, cplx *H0, cplx *H1)
-{
-  cplx ik = IMUL(k);
-  cplx c4 = 4.0 / (ik * ik);
-  for (int a = 0; a < 3; a++)
-    for (int b = 0; b < 3; b++) combo_ab(m, Qa + 3 * a, Qb + 3 * b, c4, needH1, H0 + 3 * a + b, H1 + 3 * a + b);
 }
 
 // TCR4 point i of a panel given as p = {V0 - centroid, V1 - V0, V2 - V0}
@@ -156,16 +95,19 @@ struct RowSums {
   cplx p0, p[3], q0, q[3];
 };
 
-// The moments of pair_moments<0>, from the row sums: with R = D + x - y
+// The moments of a pair from the row sums: with R = D + x - y
 // every moment is linear in them, e.g. u = sum (R x x) Psi = (D x x) q0 +
 // x x q and s = sum ((x x y).R) Psi = (x x q).D, so a point pair costs its
 // kernel and 16 multiply-adds where the moments themselves took 40 and the
 // vector products 27 operations more.  sy: the points of the second panel
-// (one panel for the whole workgroup); sp: per thread the first panel as {V0 -
-// centroid, V1 - V0, V2 - V0} and D, in LDS, so that the point loop, rolled,
-// keeps to 256 registers (two waves per SIMD).  Bound: FP64 vector rate.
-// N=3840 dielectric, 1.8 million pairs and two regions: 425 us (617 before)
-__device__ inline void pair_moments_far(const double (*sp)[256], const double (*sy)[3], cplx k, int needH1, Moments &m)
+// (far: one panel for the whole workgroup; near: two edges per thread); sp: per
+// thread the first panel as {V0 - origin, V1 - V0, V2 - V0} and D, in LDS, so
+// that the point loop, rolled, keeps to 256 registers (two waves per SIMD).  Bound: FP64 vector rate.
+// N=3840 dielectric, two regions: 430 us (617 before)
+// NEAR: Phi with ExpRel(ikr, 4) = sum_{m>=4} (ikr)^m/m!, stopped at |term| <
+// 1e-8 |sum|, in the exponential's place (PanelPanelInteractions.cc:84-103)
+template <bool NEAR, int NT>
+__device__ inline void pair_moments_rows(const double (*sp)[NT], const double *sy, cplx k, int needH1, Moments &m)
 {
 #pragma clang fp contract(fast)
   m.S1 = mk(0, 0); m.Sxy = mk(0, 0); m.s = mk(0, 0);
@@ -185,17 +127,33 @@ __device__ inline void pair_moments_far(const double (*sp)[256], const double (*
     for (int c = 0; c < 3; c++) { t.p[c] = mk(0, 0); t.q[c] = mk(0, 0); }
 #pragma unroll 1
     for (int j = 0; j < 6; j++) {
-      const double y[3] = {sy[j][0], sy[j][1], sy[j][2]};
+      double y[3];
+      for (int c = 0; c < 3; c++)
+        y[c] = NEAR ? c_tcr4[3 * j] * sy[c * NT + tid] + c_tcr4[3 * j + 1] * sy[(3 + c) * NT + tid] : sy[3 * j + c];
       const double R[3] = {Dx[0] - y[0], Dx[1] - y[1], Dx[2] - y[2]};
-      double r, ir, sn = 0.0, cs = 1.0;
+      double r, ir;
       rsqrt_sqrt(R[0] * R[0] + R[1] * R[1] + R[2] * R[2], &ir, &r);
-      // (a real wavenumber, as in a lossless region at real frequency,
-      // skips the exponential, an imaginary one, as at imaginary frequency,
-      // the sine and cosine: both are exact there)
-      double e = c_tcr4[3 * j + 2] * ir;
-      if (k.i != 0) e *= exp(-k.i * r);
-      if (k.r != 0) sincos(k.r * r, &sn, &cs);
-      const double fr = e * cs, fi = e * sn;
+      double e = c_tcr4[3 * j + 2] * ir, fr, fi;
+      if constexpr (NEAR) {
+        const cplx z = mk(-k.i * r, k.r * r);
+        cplx term = cmulf(cmulf(z, z), (1.0 / 6.0) * z), sum = mk(0, 0);
+        for (int q = 4; q < 100; q++) {
+          term = cmulf(term, c_inv.v[q] * z);
+          sum += term;
+          if (norm2(term) < 1.0e-16 * norm2(sum)) break;
+        }
+        fr = e * sum.r;
+        fi = e * sum.i;
+      } else {
+        // (a real wavenumber, as in a lossless region at real frequency,
+        // skips the exponential, an imaginary one, as at imaginary frequency,
+        // the sine and cosine: both are exact there)
+        double sn = 0.0, cs = 1.0;
+        if (k.i != 0) e *= exp(-k.i * r);
+        if (k.r != 0) sincos(k.r * r, &sn, &cs);
+        fr = e * cs;
+        fi = e * sn;
+      }
       t.p0.r += fr; t.p0.i += fi;
       for (int c = 0; c < 3; c++) { t.p[c].r += y[c] * fr; t.p[c].i += y[c] * fi; }
       if (needH1) {
@@ -288,7 +246,7 @@ k_far(const double *Va, const int *PVIa, const double *PCa, int rowLimit,
   for (int r = 0; r < nreg; r++) {
     Moments m;
     cplx k = regs[r].k;
-    pair_moments_far(sp, sy, k, needH1, m);
+    pair_moments_rows<false, 256>(sp, &sy[0][0], k, needH1, m);
     // source vertices relative to the centroids
     double Qa[9], Qb[9];
     for (int c = 0; c < 3; c++) {
@@ -455,26 +413,38 @@ hipError_t launch_far(hipStream_t stream, const double *Va, const int *PVIa, con
 // singular terms rebuilt from the cached frequency-independent integrals
 // (PanelPanelInteractions.cc:504-559, QDFIPPI.cc:67-260).
 // ---------------------------------------------------------------------
-__global__ void __launch_bounds__(128)
+// One thread per (pair, region = blockIdx.y): the moments first, then each
+// (Qa, Qb) with its singular terms, so that neither holds the other's
+// registers.  Bound: latency (36 points in sequence, few waves).  N=3840
+// dielectric: 127 us in the batched sweep, where both regions in one thread, 20
+// moments a point and the nine pairs' terms kept in scratch memory took 195
+__global__ void __launch_bounds__(64, 2)
 k_near(const NearPair *nps, int nnear, const double *records, int nreg, const RegionK *regs,
        int needH1, double *HN)
 {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
+  constexpr int NT = 64;
+  __shared__ double sp[12][NT], sq[6][NT];
+  const int t = blockIdx.x * NT + threadIdx.x, r = blockIdx.y, tid = threadIdx.x;
   if (t >= nnear) return;
   const NearPair &P = nps[t];
   const double *Q = records + (long long)P.rec * SCUFFX_QIF_LEN;
   // reordered vertices: x = Va0 + u(Va1-Va0) + v(Va2-Va0); local origin Va0
-  double xi[18], eta[18], Qal[9], Qbl[9], D[3];
+  // (each thread reads only what it wrote: no barrier)
   for (int c = 0; c < 3; c++) {
-    double aA = P.Va[3 + c] - P.Va[c], aB = P.Va[6 + c] - P.Va[c];
-    double bA = P.Vb[3 + c] - P.Vb[c], bB = P.Vb[6 + c] - P.Vb[c];
-    for (int i = 0; i < 6; i++) {
-      xi[3 * i + c] = c_tcr4[3 * i] * aA + c_tcr4[3 * i + 1] * aB;
-      eta[3 * i + c] = c_tcr4[3 * i] * bA + c_tcr4[3 * i + 1] * bB;
-    }
-    for (int q = 0; q < 3; q++) { Qal[3 * q + c] = P.Qa[3 * q + c] - P.Va[c]; Qbl[3 * q + c] = P.Qb[3 * q + c] - P.Vb[c]; }
-    D[c] = P.Va[c] - P.Vb[c];
+    sp[c][tid] = 0.0;
+    sp[3 + c][tid] = P.Va[3 + c] - P.Va[c];
+    sp[6 + c][tid] = P.Va[6 + c] - P.Va[c];
+    sp[9 + c][tid] = P.Va[c] - P.Vb[c];
+    sq[c][tid] = P.Vb[3 + c] - P.Vb[c];
+    sq[3 + c][tid] = P.Vb[6 + c] - P.Vb[c];
   }
+  const cplx k = regs[r].k;
+  Moments m;
+  pair_moments_rows<true, NT>(sp, &sq[0][0], k, needH1, m);
+  const cplx ik = IMUL(k), c4 = 4.0 / (ik * ik), OOIK2 = 1.0 / (ik * ik);
+  cplx PF[5];
+  PF[0] = mk(SCUFFX_INV4PI, 0);
+  for (int q = 1; q < 5; q++) PF[q] = ik * PF[q - 1];
   // Q-dependent FIPPI recombination, shared pieces
   const double *OVa[3] = {P.OVa0, P.OVa1, P.OVa2}, *OVb[3] = {P.OVb0, P.OVb1, P.OVb2};
   double A[3], B[3], AP[3], BP[3];
@@ -487,18 +457,38 @@ k_near(const NearPair *nps, int nnear, const double *records, int nreg, const Re
   double Lc[3];
   const double *Vc = P.flipped ? P.Vb : P.Va;
   for (int c = 0; c < 3; c++) Lc[c] = x0[c] - (Vc[c] + Vc[3 + c] + Vc[6 + c]) / 3.0;
-  bool applyL = sqrt(dot3(Lc, Lc)) > 1.0e-8 * sqrt(dot3(A, A));
-  double hDot[9][4], hNab[4], hTim[9][4], hTimRM3[9];
+  const bool applyL = sqrt(dot3(Lc, Lc)) > 1.0e-8 * sqrt(dot3(A, A));
+  const double hNab[4] = {4.0 * RM1[0], 1.0, 4.0 * R1[0], 4.0 * R2[0]};
+  const int stride = needH1 ? 4 : 2;
+  double *out = HN + ((long long)t * nreg + r) * 9 * stride;
   // hDot/hTimes for moments RM1, R0, R1, R2 (QDFIPPI.cc:163-251)
-  for (int a = 0; a < 3; a++)
-    for (int b = 0; b < 3; b++) {
-      const double *Qa = P.Qa + 3 * a, *Qb = P.Qb + 3 * b;
-      const double *OQa = P.flipped ? Qb : Qa, *OQb = P.flipped ? Qa : Qb;
-      double V0mQ[3], V0PmQP[3];
-      sub3(OVa[0], OQa, V0mQ); sub3(OVb[0], OQb, V0PmQP);
-      double VdVP = dot3(V0mQ, V0PmQP), VdAP = dot3(V0mQ, AP), VdBP = dot3(V0mQ, BP);
-      double AdVP = dot3(A, V0PmQP), AdAP = dot3(A, AP), AdBP = dot3(A, BP);
-      double BdVP = dot3(B, V0PmQP), BdAP = dot3(B, AP), BdBP = dot3(B, BP);
+#pragma unroll 1
+  for (int ab = 0; ab < 9; ab++) {
+    const int a = ab / 3, b = ab - 3 * a;
+    const double *Qa = P.Qa + 3 * a, *Qb = P.Qb + 3 * b;
+    const double *OQa = P.flipped ? Qb : Qa, *OQb = P.flipped ? Qa : Qb;
+    cplx h0, h1;
+    {
+      double qa[3], qb[3];
+      sub3(Qa, P.Va, qa); sub3(Qb, P.Vb, qb);
+      combo_ab(m, qa, qb, c4, needH1, &h0, &h1);
+    }
+    double V0mQ[3], V0PmQP[3];
+    sub3(OVa[0], OQa, V0mQ); sub3(OVb[0], OQb, V0PmQP);
+    double VdVP = dot3(V0mQ, V0PmQP), VdAP = dot3(V0mQ, AP), VdBP = dot3(V0mQ, BP);
+    double AdVP = dot3(A, V0PmQP), AdAP = dot3(A, AP), AdBP = dot3(A, BP);
+    double BdVP = dot3(B, V0PmQP), BdAP = dot3(B, AP), BdBP = dot3(B, BP);
+    auto hDot = [&](const double *M) {
+      return M[0] * VdVP + M[1] * VdAP + M[2] * VdBP + M[3] * AdVP + M[4] * AdAP
+             + M[5] * AdBP + M[6] * BdVP + M[7] * BdAP + M[8] * BdBP;
+    };
+    h0 += PF[0] * (mk(hDot(RM1), 0) + OOIK2 * hNab[0])
+          + PF[1] * (mk(hDot(r0m), 0) + OOIK2 * hNab[1])
+          + PF[2] * 0.5 * (mk(hDot(R1), 0) + OOIK2 * hNab[2])
+          + PF[3] * (1.0 / 6.0) * (mk(hDot(R2), 0) + OOIK2 * hNab[3]);
+    double *o = out + ab * stride;
+    o[0] = h0.r; o[1] = h0.i;
+    if (needH1) {
       double QamQb[3], QaxQb[3], V0mV0P[3], S[3];
       sub3(OVa[0], OVb[0], V0mV0P);
       sub3(Qa, Qb, QamQb);
@@ -514,47 +504,15 @@ k_near(const NearPair *nps, int nnear, const double *records, int nreg, const Re
       cross3(B, BP, S);          double ht0101 = dot3(QamQb, S);
       double rm3 = dot3(QaxQb, xMxp) + dot3(QamQb, xXxp);
       if (applyL) { cross3(Lc, QamQb, S); rm3 -= dot3(S, xMxp); }
-      const double *Ms[4] = {RM1, r0m, R1, R2};
-      for (int q = 0; q < 4; q++) {
-        const double *M = Ms[q];
-        hDot[3 * a + b][q] = M[0] * VdVP + M[1] * VdAP + M[2] * VdBP + M[3] * AdVP + M[4] * AdAP
-                             + M[5] * AdBP + M[6] * BdVP + M[7] * BdAP + M[8] * BdBP;
-        hTim[3 * a + b][q] = M[0] * ht0000 + M[3] * ht1000 + M[6] * ht0100 + M[1] * ht0010
-                             + M[2] * ht0001 + M[4] * ht1010 + M[5] * ht1001 + M[7] * ht0110
-                             + M[8] * ht0101;
-      }
-      hTimRM3[3 * a + b] = rm3;
-      if (P.flipped) {
-        hTimRM3[3 * a + b] *= -1.0;
-        for (int q = 0; q < 3; q++) hTim[3 * a + b][q] *= -1.0;
-      }
-    }
-  hNab[0] = 4.0 * RM1[0]; hNab[1] = 1.0; hNab[2] = 4.0 * R1[0]; hNab[3] = 4.0 * R2[0];
-  int stride = needH1 ? 4 : 2;
-  double *out = HN + (long long)t * (nreg * 9 * stride);
-  for (int r = 0; r < nreg; r++) {
-    cplx k = regs[r].k;
-    Moments m;
-    pair_moments<1>(xi, eta, D, k, needH1, m);
-    cplx H0[9], H1[9];
-    combos_from_moments(m, Qal, Qbl, k, needH1, H0, H1);
-    cplx ik = IMUL(k), OOIK2 = 1.0 / (ik * ik), PF[5];
-    PF[0] = mk(SCUFFX_INV4PI, 0);
-    for (int q = 1; q < 5; q++) PF[q] = ik * PF[q - 1];
-    for (int q = 0; q < 9; q++) {
-      cplx h0 = H0[q];
-      h0 += PF[0] * (mk(hDot[q][0], 0) + OOIK2 * hNab[0])
-            + PF[1] * (mk(hDot[q][1], 0) + OOIK2 * hNab[1])
-            + PF[2] * 0.5 * (mk(hDot[q][2], 0) + OOIK2 * hNab[2])
-            + PF[3] * (1.0 / 6.0) * (mk(hDot[q][3], 0) + OOIK2 * hNab[3]);
-      double *o = out + (r * 9 + q) * stride;
-      o[0] = h0.r; o[1] = h0.i;
-      if (needH1) {
-        cplx h1 = H1[q];
-        h1 += PF[0] * (-1.0 * hTimRM3[q]) + PF[2] * (0.5 * hTim[q][0])
-              + PF[3] * ((1.0 / 3.0) * hTim[q][1]) + PF[4] * ((1.0 / 6.0) * hTim[q][2]);
-        o[2] = h1.r; o[3] = h1.i;
-      }
+      const double sg = P.flipped ? -1.0 : 1.0;
+      auto hTim = [&](const double *M) {
+        return sg * (M[0] * ht0000 + M[3] * ht1000 + M[6] * ht0100 + M[1] * ht0010
+                     + M[2] * ht0001 + M[4] * ht1010 + M[5] * ht1001 + M[7] * ht0110
+                     + M[8] * ht0101);
+      };
+      h1 += PF[0] * (-1.0 * (sg * rm3)) + PF[2] * (0.5 * hTim(RM1))
+            + PF[3] * ((1.0 / 3.0) * hTim(r0m)) + PF[4] * ((1.0 / 6.0) * hTim(R1));
+      o[2] = h1.r; o[3] = h1.i;
     }
   }
 }
@@ -563,8 +521,8 @@ hipError_t launch_near(hipStream_t stream, const NearPair *np, int nnear, const 
                        int nreg, const RegionK *regs, int needH1, double *HN)
 {
   if (nnear <= 0 || nreg <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_near, dim3((nnear + 127) / 128), dim3(128), 0, stream, np, nnear, records,
-                     nreg, regs, needH1, HN);
+  hipLaunchKernelGGL(k_near, dim3((nnear + 63) / 64, nreg), dim3(64), 0, stream, np, nnear, records, nreg, regs, needH1,
+                     HN);
   return hipGetLastError();
 }
 
