@@ -287,7 +287,7 @@ struct Moments32 {
   fcx s, u[3], v[3], w[3];
 };
 
-// the far-pair moments in FP32 from panels given as in pair_moments_far:
+// the far-pair moments in FP32 from panels as tcr4_point takes them:
 // each point formed in FP64, as before the cast, inside a rolled 6 x 6
 // point loop
 template <bool REALK>

@@ -189,7 +189,7 @@ template <int J, int N, typename F> __device__ __attribute__((always_inline)) in
   }
 }
 
-// slots of the exact panel's exchange area (lu_panel.hip): one per column
+// slots of the exact panel's exchange area (lu_panel.inc): one per column
 // and workgroup, 64-bit words {key, position, the candidate row}
 template <typename T> struct XW;          // 64-bit words of one entry
 template <> struct XW<double2> { static const int n = 2; };
