@@ -25,6 +25,9 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
 // the intermediate vector W (n), the inverses of the 64x64 diagonal blocks
 // of L and U (nblk * 64 * 64 each, nblk = ceil(n / 64)), the composed row
 // permutation (n ints) and the one-launch solve's words (2 nblk + 8).
+// refined (complex64): the caller corrects the solution by residuals in
+// higher precision, so that products with the diagonal blocks' inverses do;
+// otherwise they are substituted through and invL, invU are not used.
 // inv_ready: invL / invU and perm already hold the inverses and the
 // composed row permutation for these factors (set by the first solve;
 // clear it for new factors).
@@ -33,7 +36,7 @@ struct SolveWs {
   T *W = nullptr, *invL = nullptr, *invU = nullptr;
   int *perm = nullptr;
   unsigned long long *chain = nullptr;
-  bool inv_ready = false;
+  bool inv_ready = false, refined = false;
 };
 // bytes of the buffers above for n rows, each part rounded to 256 bytes
 template <typename T>

@@ -1549,7 +1549,7 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
 
 // ---------------------------------------------------------------------
 // triangular solves, in one launch per triangle: one right-hand side down
-// the 64-row blocks with the inverses of the diagonal blocks (k_trsv_chain),
+// the 64-row blocks (k_trsv_chain),
 // several right-hand sides and transposed systems as a chain of block
 // products on the matrix cores with substitution (k_trsm_chain).
 // ---------------------------------------------------------------------
@@ -1623,7 +1623,7 @@ static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, b
 
 // Inverses of the diagonal 64x64 blocks of L (unit lower, blockIdx.y = 0)
 // and U (blockIdx.y = 1), identity past row n: every block step of a
-// one-right-hand-side solve is then a product.  Columns of the inverse by
+// refined complex64 solve is then a product.  Columns of the inverse by
 // substitution, so that L X and U X, not X L and X U, are the identity to
 // rounding (the transpose of U^T's inverse converged ten times slower in the
 // refinement).  One workgroup a block, a wave for 16 columns of the inverse, a
@@ -1767,7 +1767,7 @@ k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin
 // Workgroup g owns the 64 rows of block g: it subtracts the off-diagonal
 // blocks' products with every earlier solution block as that block is
 // published (forward: blocks k < g of L; backward: k > g of U), then
-// applies the inverse diagonal block and publishes its own 64 values.  The
+// solves with the diagonal block and publishes its own 64 values.  The
 // output starts filled with a sentinel (a NaN bit pattern in every 64-bit
 // word that no solve produces), and every entry is written once, by an
 // agent-scope relaxed atomic store: a reader that sees a word other than
@@ -1778,6 +1778,13 @@ k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin
 // block's 16 values per thread are loaded before the wait.  The forward
 // solve, which reads its right-hand side b once per row, leaves the
 // sentinel in b (mark), where the backward solve writes its output.
+// SUB: the diagonal block by substitution, one wave, x_k by lane reads.  Not
+// SUB: by its explicit inverse, for callers that refine the solution in higher
+// precision.  Products with the inverse of a badly scaled block (dielectric
+// surfaces near the low-frequency limit, whose electric and magnetic rows differ by
+// 1e6) lose digits that no residual of their own brings back further down:
+// eps = 10 sphere of 960 functions at frequency 0.001i in complex128: forward
+// error 2e-4 with the inverses, 9e-9 by substitution.
 #define SCUFFX_CHAIN_SENT 0x7FF4DEADBEEF0003ULL
 
 // a loaded value is final once none of its 64-bit words is the sentinel
@@ -1811,12 +1818,13 @@ __global__ void k_chain_fill(T *x, long n)
   }
 }
 
-template <typename T, bool LOWER>
+template <typename T, bool LOWER, bool SUB>
 __global__ void __launch_bounds__(256)
 k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int mark, unsigned *err)
 {
   __shared__ T part[4][TB];
   __shared__ T bx[TB];
+  __shared__ T sD[SUB ? TB : 1][TB];       // [column][row] of the diagonal block
   const int t = threadIdx.x, r = t & (TB - 1), q = t >> 6;
   const long nblk = (n + TB - 1) / TB;
   const long g = blockIdx.x;
@@ -1844,9 +1852,22 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
 #pragma unroll
     for (int u = 0; u < 16; u++) m[u] = ib[r + (long)(q * 16 + u) * TB];
   };
+  // SUB: the diagonal block into LDS and its diagonal's reciprocals, ahead of
+  // the waits (zero past row n, where nothing uses the results)
+  T rd = unit_v<T>();
+  if constexpr (SUB) {
+#pragma unroll
+    for (int u = 0; u < 16; u++) {
+      const int c = q * 16 + u;
+      const T v = LU[g * TB + min(r, bs - 1) + (g * TB + min(c, bs - 1)) * lda];
+      sD[c][r] = r < bs && c < bs ? v : zero_v<T>();
+    }
+    if (!LOWER && q == 0 && r < bs) rd = crecip(LU[row + row * lda]);
+    __syncthreads();
+  }
   T a[16];
   if (nk > 0) load(blk(0), a);
-  else load_inv(a);
+  else if (!SUB) load_inv(a);
   for (long i = 0; i < nk; i++) {
     const long k = blk(i);
     // this thread's 16 values of block k, once published (bounded)
@@ -1874,7 +1895,7 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
       mac(acc, a[u], x[u]);
     }
     if (i + 1 < nk) load(blk(i + 1), a);
-    else load_inv(a);
+    else if (!SUB) load_inv(a);
     part[q][r] = acc;
     __syncthreads();
     if (q == 0) {
@@ -1883,6 +1904,23 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
       b = csub(b, s4);
     }
     __syncthreads();
+  }
+  if constexpr (SUB) {
+    // own block: a lane a row, its products summed by themselves
+    if (q != 0) return;
+    T z = zero_v<T>();
+#pragma unroll
+    for (int j = 0; j < TB; j++) {
+      const int k = LOWER ? j : TB - 1 - j;
+      T v = cadd(b, z);
+      if (!LOWER) v = cmul(v, rd);
+      v = readlane_t(v, k);
+      if (LOWER ? r > k : r < k) z = fnma_t(z, sD[k][r], v);
+    }
+    T xg = cadd(b, z);
+    if (!LOWER) xg = cmul(xg, rd);
+    if (r < bs) st_coh(xout + row, xg);
+    return;
   }
   // own block: x_g = inv(D_g) b_g
   if (q == 0) bx[r] = b;
@@ -2139,7 +2177,7 @@ template <typename T> static bool chain_resident(long n)
   if (ncu < 0) {
     int dev = 0, c = 0;
     hipGetDevice(&dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_trsv_chain<T, true>, 256, 0);
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_trsv_chain<T, true, true>, 256, 0);
     hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
     ncu = c;
   }
@@ -2147,8 +2185,8 @@ template <typename T> static bool chain_resident(long n)
 }
 
 // lower (forward) then upper (backward) solve of one right-hand side in
-// two cooperative launches (chain_resident(n)); returns -2 without a
-// workspace, -6 on a time-out
+// two cooperative launches (chain_resident(n)), by substitution if the block
+// inverses are null; returns -2 without a workspace, -6 on a time-out
 template <typename T>
 static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *invU, T *B, T *W, hipStream_t s,
                       unsigned long long *words)
@@ -2164,14 +2202,16 @@ static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *inv
   int mark = 1, nomark = 0;
   void *al[] = {(void *)&LU, (void *)&lda, (void *)&n, (void *)&invL, (void *)&B, (void *)&W, (void *)&mark,
                 (void *)&err};
-  if (hipLaunchCooperativeKernel((const void *)k_trsv_chain<T, true>, dim3((unsigned)nblk), dim3(256), al, 0, s) !=
-      hipSuccess)
-    return -3;
+  const void *kl = (const void *)k_trsv_chain<T, true, true>, *ku = (const void *)k_trsv_chain<T, false, true>;
+  if constexpr (std::is_same<T, float2>::value)
+    if (invL) {
+      kl = (const void *)k_trsv_chain<T, true, false>;
+      ku = (const void *)k_trsv_chain<T, false, false>;
+    }
+  if (hipLaunchCooperativeKernel(kl, dim3((unsigned)nblk), dim3(256), al, 0, s) != hipSuccess) return -3;
   void *au[] = {(void *)&LU, (void *)&lda, (void *)&n, (void *)&invU, (void *)&W, (void *)&B, (void *)&nomark,
                 (void *)&err};
-  if (hipLaunchCooperativeKernel((const void *)k_trsv_chain<T, false>, dim3((unsigned)nblk), dim3(256), au, 0, s) !=
-      hipSuccess)
-    return -3;
+  if (hipLaunchCooperativeKernel(ku, dim3((unsigned)nblk), dim3(256), au, 0, s) != hipSuccess) return -3;
   unsigned tmo = 0;
   hipMemcpyAsync(&tmo, err, sizeof(unsigned), hipMemcpyDeviceToHost, s);
   hipStreamSynchronize(s);
@@ -2289,18 +2329,19 @@ int lu_solve(const T *LU, long n, long lda, const int *d_ipiv, char trans, long 
   const bool tr = trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', cj = trans == 'C' || trans == 'c';
   if (!tr && trans != 'N' && trans != 'n') return -1;
   if (!tr && nrhs == 1 && chain_resident<T>(n)) {
-    const long nblk = (n + TB - 1) / TB;
     T *W = ws ? ws->W : (T *)ws_get(WS_SOLVE_W, sizeof(T) * n);
-    T *invL = ws ? ws->invL : (T *)ws_get(WS_SOLVE_INVL, sizeof(T) * nblk * TB * TB);
-    T *invU = ws ? ws->invU : (T *)ws_get(WS_SOLVE_INVU, sizeof(T) * nblk * TB * TB);
-    if (!W || !invL || !invU) return -2;
+    if (!W) return -2;
     // a solve after the first with the same factors reuses the block
     // inverses and the composed permutation
     const bool cached = ws && ws->inv_ready;
-    if (!cached) {
-      tri_inv(LU, lda, n, invL, invU, stream);
-      if (ws) ws->inv_ready = true;
-    }
+    T *invL = nullptr, *invU = nullptr;
+    if constexpr (std::is_same<T, float2>::value)
+      if (ws && ws->refined) {
+        invL = ws->invL;
+        invU = ws->invU;
+        if (!cached) tri_inv(LU, lda, n, invL, invU, stream);
+      }
+    if (ws) ws->inv_ready = true;
     apply_row_perm(B, ldb, n, nrhs, d_ipiv, true, W, stream, ws ? ws->perm : nullptr, cached);
     return trsv_chain(LU, lda, n, invL, invU, B, W, stream, ws ? ws->chain : nullptr);
   }

@@ -47,6 +47,7 @@ RefineWs refine_ws_carve(char *base, long n, int m)
   w.V = (double2 *)base; base += r256(sizeof(double2) * n * ((long)m + 1));
   w.Z = (double2 *)base; base += r256(sizeof(double2) * n * (long)m);
   w.sws = solve_ws_carve<float2>(base, n);
+  w.sws.refined = true;
   return w;
 }
 

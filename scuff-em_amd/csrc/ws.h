@@ -12,8 +12,6 @@ namespace scuffx {
 enum WsSlot {
   WS_PANEL = 0,    // LU panel scratch (barrier words, candidates, plan)
   WS_SOLVE_W,      // triangular solve: intermediate vector(s)
-  WS_SOLVE_INVL,   // triangular solve: inverses of the diagonal blocks of L
-  WS_SOLVE_INVU,   // ... and of U
   WS_REFINE,       // refinement: residual, partial sums, complex64 residual, scalar
   WS_PERM,         // triangular solve: composed row permutation of ipiv
   WS_PERM_TMP,     // ... and the permuted right-hand sides (many-column solves)

@@ -152,3 +152,45 @@ def test_mixed_wide_block_rows(sx):
     LUV = np.tril(F, -1).astype("complex128") @ UV + UV
     res = np.linalg.norm(A.astype("complex128")[perm] @ V - LUV) / (np.linalg.norm(A) * np.linalg.norm(V) / np.sqrt(n))
     assert res <= 2e-5 * np.sqrt(n / 40), res
+
+
+# solves with one right-hand side near the low-frequency limit, where a
+# dielectric's electric and magnetic rows differ by 1e6: products with the
+# inverses of the 64x64 diagonal blocks lost seven digits.  Substitution solves
+# (T + dT) x = b with |dT| <= gamma_n |T| for each triangle (Higham, Accuracy
+# and Stability, theorem 8.5), so |P b - L U x| <= 2 gamma_n |L| |U| |x| entry by
+# entry; a complex product rounds 2 sqrt(2) times as much as a real one
+@pytest.mark.parametrize("dtype,noalloc", [("complex128", False), ("float64", False), ("complex128", True),
+                                           ("complex64", False), ("complex64", True)])
+def test_badly_scaled_blocks(sx, O, dtype, noalloc):
+    V, T = O.icosphere(2)
+    G = sx.RWGGeometry()
+    G.AddMesh(V, T, "CONST_EPS_10")
+    print(f"badly scaled blocks {dtype} noalloc={noalloc}", flush=True)
+    A = G.AssembleBEMMatrix(0.001j).numpy()
+    if dtype == "float64":
+        A = A.real.copy()
+    A = A.astype(dtype)
+    n = A.shape[0]
+    M = sx.HMatrix.from_numpy(A, dtype=dtype)
+    assert M.LUFactorize() == 0
+    F, piv = M.numpy(), M.ipiv.cpu().numpy()
+    wide = np.longdouble if dtype == "float64" else np.clongdouble
+    L, U = np.tril(F, -1).astype(wide) + np.eye(n), np.triu(F).astype(wide)
+    perm = np.arange(n)
+    for i in range(n):
+        perm[[i, piv[i] - 1]] = perm[[piv[i] - 1, i]]
+    for rows in (np.arange(n) % 2, np.ones(n)):
+        b = (matrix(n, dtype, 17)[0] * rows).astype(dtype)
+        X = sx.HMatrix.from_numpy(b.reshape(n, 1), dtype=dtype)
+        if noalloc:
+            rc = sx.lib().scuffx_lu_solve_noalloc(sx._ptr(M.t), n, n, sx._ptr(M.ipiv), sx._ptr(X.t), M.prec)
+            assert rc == 0
+        else:
+            M.LUSolve(X)
+        x = X.numpy()[:, 0].astype(wide)
+        res = np.abs(b[perm].astype(wide) - L @ (U @ x))
+        bound = np.abs(L) @ (np.abs(U) @ np.abs(x))
+        c = 1.0 if dtype == "float64" else 2.0 * np.sqrt(2.0)
+        print(f"  {float(np.max(res / bound)):.2e}", flush=True)
+        assert np.max(res / bound) <= 2 * c * n * EPS[dtype]
