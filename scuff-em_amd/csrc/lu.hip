@@ -853,7 +853,16 @@ template <typename T> __device__ inline T readlane_t(T v, int k)
   return r;
 }
 
-// r - l x with fused multiply-adds
+// l x, and r - l x, with fused multiply-adds
+__device__ inline double fmul_t(double l, double x) { return l * x; }
+__device__ inline double2 fmul_t(double2 l, double2 x)
+{
+  return make_double2(fma(l.x, x.x, -(l.y * x.y)), fma(l.x, x.y, l.y * x.x));
+}
+__device__ inline float2 fmul_t(float2 l, float2 x)
+{
+  return make_float2(fmaf(l.x, x.x, -(l.y * x.y)), fmaf(l.x, x.y, l.y * x.x));
+}
 __device__ inline double fnma_t(double r, double l, double x) { return fma(-l, x, r); }
 __device__ inline double2 fnma_t(double2 r, double2 l, double2 x)
 {
@@ -1960,16 +1969,27 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
 // lane for each of the 64 rows, x_k by lane reads, took 10 us a block in
 // complex128; products with the explicit inverse 2 us, but where the block is
 // badly scaled, eps = 10 spheres at imaginary frequency 0.001, they lose every
-// digit.)  The entries of the first sub-block are loaded before the wait.
+// digit.)  The entries of the first sub-block wait in LDS.
+// Rounding: a block's 64 products and a sub-block's own are summed by
+// themselves and subtracted once, not term by term from the right-hand side.
+// Transposed systems (EXACT) sum two k-steps at a time, keep what the
+// subtractions lose (two-sums, added back before each use) and correct the
+// quotients: their error then is that of a dot product of 256 partial sums and
+// one division a row, i.e. 0.85 to 1.07 of it over orders 100 to 1500 and the
+// three types, where sums over four blocks, products subtracted term by term
+// and rounded reciprocals had 1.7 to 3.8 times as much (up to 1.7 times as much
+// as products with the blocks' inverses in the untransposed form, now 0.7 to
+// 0.98).  One transposed system, order 3840, complex128: 1.69 -> 2.13 ms; the
+// untransposed forms take the same time.
 // bin: column-major right-hand sides, row r taken from pin[r] if given, or
 // null: packed in win.  bout: column-major results or null, row r to pout[r]
 // if given.  cj: 1 conjugates the right-hand sides, 2 the results in bout.
 // Bound: the chain of block steps up to a few hundred columns (a round trip,
 // 16 complex 16x16x4 products and 64 substitution steps per wave), the
-// matrix units past that.  N=3840 complex128: 12 us a step; 181 columns 2.1
-// ms, where substitution in 256-row blocks by one workgroup a column and GEMM
-// updates took 6.0; one transposed system 1.7 ms, where a single workgroup
-// with a reduction per row took 24; 1920 columns 6.4 ms (35 TFLOP/s).
+// matrix units past that.  N=3840 complex128: 12 us a step (17 transposed);
+// 181 columns 2.1 ms, where substitution in 256-row blocks by one workgroup a
+// column and GEMM updates took 6.0; one transposed system 2.1 ms, where a single
+// workgroup with a reduction per row took 24.
 template <typename T> struct ChainArgs {
   const T *A; long lda; long n;
   const T *bin; long ldb; const int *pin; const T *win;
@@ -1977,9 +1997,9 @@ template <typename T> struct ChainArgs {
   long nrhs; int cj; unsigned *err, *ticket;
 };
 
-// acc += a x for one and for 16 k-steps of the matrix instruction
+// acc += a x for one k-step of the matrix instruction
 template <typename T>
-__device__ inline void chain_mac1(T a, T x, typename CT<T>::V4 &re, typename CT<T>::V4 &im)
+__device__ inline void chain_mac(T a, T x, typename CT<T>::V4 &re, typename CT<T>::V4 &im)
 {
   if constexpr (IsReal<T>::v) re = CT<T>::mfma(a, x, re);
   else {
@@ -1989,11 +2009,26 @@ __device__ inline void chain_mac1(T a, T x, typename CT<T>::V4 &re, typename CT<
     im = CT<T>::mfma(a.y, x.x, im);
   }
 }
-template <typename T>
-__device__ inline void chain_mac(const T (&a)[16], const T (&x)[16], typename CT<T>::V4 &re, typename CT<T>::V4 &im)
+// h - v, what its rounding lost added to l (Knuth's two-sum)
+template <typename R> __device__ inline void two_diff(R &h, R &l, R v)
 {
-#pragma unroll
-  for (int s = 0; s < 16; s++) chain_mac1<T>(a[s], x[s], re, im);
+  const R z = h - v, w = z - h;
+  l += (h - (z - w)) - (v + w);
+  h = z;
+}
+__device__ inline void sub2(double &h, double &l, double v) { two_diff(h, l, v); }
+template <typename T> __device__ inline void sub2(T &h, T &l, T v)
+{
+  two_diff(h.x, l.x, v.x);
+  two_diff(h.y, l.y, v.y);
+}
+__device__ inline bool is_finite(double v) { return isfinite(v); }
+template <typename T> __device__ inline bool is_finite(T v) { return isfinite(v.x) && isfinite(v.y); }
+// v / d from d's reciprocal, corrected by the residual where that is finite
+template <typename T> __device__ inline T quot(T v, T d, T rd)
+{
+  const T q = cmul(v, rd), c = cmul(fnma_t(v, d, q), rd);
+  return is_finite(c) ? cadd(q, c) : q;
 }
 // v of lane k of this lane's row of 16
 template <int K> __device__ inline float row_bcast(float v)
@@ -2025,8 +2060,10 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
 {
   typedef typename CT<T>::V4 V4;
   constexpr int NC = 16;
-  constexpr bool UNIT = FWD != TRANS;
-  __shared__ T sb[TB][NC + 1];
+  constexpr bool UNIT = FWD != TRANS, EXACT = TRANS;
+  __shared__ T sb[TB][NC + 1];                     // right-hand sides, then solutions
+  __shared__ T sl[EXACT ? TB : 1][NC + 1];         // what their roundings lost
+  __shared__ T sm[16][17], sd[TB], sr[TB];         // first diagonal sub-block; the diagonal and its reciprocals
   __shared__ unsigned s_tk;
   const int t = threadIdx.x, lane = t & 63, i = lane & 15, kq = lane >> 4, w0 = (t >> 6) * 16;
   if (t == 0) s_tk = __hip_atomic_fetch_add(p.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2066,26 +2103,52 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
 #pragma unroll
     for (int s = 0; s < 16; s++) d[s] = at(sub(u) + i, sub(u) + (FWD ? s : 15 - s));
   };
-  auto fload = [&](int u, T (&f)[16]) {       // f[4 u ..]
+  auto fload = [&](int u, T (&f)[12]) {       // f[4 u ..]
 #pragma unroll
     for (int s = 0; s < 4; s++) f[4 * u + s] = at(w0 + i, sub(u) + 4 * s + kq);
   };
   // the first sub-block, the diagonal's reciprocals and the right-hand side,
   // loaded ahead
-  T m[16], b[4], rd[4];
-  dload(0, m);
-#pragma unroll
-  for (int u = 0; u < 4; u++) rd[u] = UNIT ? unit_v<T>() : sub(u) + i < bs ? crecip(at(sub(u) + i, sub(u) + i)) : unit_v<T>();
+  {
+    const int s = t >> 4;
+    sm[s][i] = at(sub(0) + i, sub(0) + (FWD ? s : 15 - s));
+    if (!UNIT && t < TB) {
+      const T d = at(t, t);
+      sd[t] = d;
+      sr[t] = t < bs ? crecip(d) : unit_v<T>();
+    }
+  }
+  // b: the right-hand side less the products so far; bl (EXACT): the sum of
+  // what its roundings lost
+  T b[4], bl[4];
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int br = w0 + CT<T>::row(lane, r);
     const long row = g * TB + br, c = tile * NC + i;
-    b[r] = zero_v<T>();
+    b[r] = bl[r] = zero_v<T>();
     if (p.bin) {
       if (br < bs && c < p.nrhs) b[r] = conj_if(p.bin[(p.pin ? p.pin[row] : row) + c * p.ldb], p.cj & 1);
     } else if (br < bs) b[r] = p.win[(tile * nblk * TB + row) * NC + i];
   }
-  V4 re = CT<T>::zero(), im = CT<T>::zero();
+  __syncthreads();
+  // the sum of ns k-steps' products (EXACT: of two each, added up), taken from b
+  auto take = [&](const T *a, const T *x, int ns) __attribute__((always_inline)) {
+    V4 re = CT<T>::zero(), im = CT<T>::zero();
+#pragma unroll
+    for (int s = 0; s < ns; s += 2) {
+      V4 tr = EXACT ? CT<T>::zero() : re, ti = EXACT ? CT<T>::zero() : im;
+      chain_mac<T>(a[s], x[s], tr, ti);
+      chain_mac<T>(a[s + 1], x[s + 1], tr, ti);
+      if (EXACT) { re += tr; im += ti; }
+      else { re = tr; im = ti; }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+      const T v = chain_elem<T>(re, im, r);
+      if (EXACT) sub2(b[r], bl[r], v);
+      else b[r] = csub(b[r], v);
+    }
+  };
   T a[16], x[16];
   if (nk > 0) load(blk(0), a);
   for (long q = 0; q < nk; q++) {
@@ -2102,57 +2165,60 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
       if (++spins > GBAR_SPIN) { __hip_atomic_store(p.err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); break; }
       __builtin_amdgcn_s_sleep(1);
     }
-    chain_mac<T>(a, x, re, im);
+    take(a, x, 16);
     if (q + 1 < nk) load(blk(q + 1), a);
-    if ((q & 3) == 3) {
-      // sums of 256 products each, subtracted one by one: a sum over the
-      // whole row would round against its own size (error 1.6 times as large)
-#pragma unroll
-      for (int r = 0; r < 4; r++) b[r] = csub(b[r], chain_elem<T>(re, im, r));
-      re = CT<T>::zero();
-      im = CT<T>::zero();
-    }
   }
   // this wave's place in the block's solve order, its columns
   const int me = FWD ? w0 / 16 : 3 - w0 / 16, c4 = w0 / 4;
+  T f[12];
+#pragma unroll
+  for (int s = 0; s < 16; s++) x[s] = sm[s][i];
   dload(1, a);
 #pragma unroll
   for (int u = 0; u < 3; u++)
-    if (u < me) fload(u, x);
-  auto rest = [&]() {      // what is left of this wave's rows
-#pragma unroll
-    for (int r = 0; r < 4; r++) sb[w0 + CT<T>::row(lane, r)][i] = csub(b[r], chain_elem<T>(re, im, r));
-  };
-#pragma unroll
-  for (int r = 0; r < 4; r++) {
-    const int br = w0 + CT<T>::row(lane, r);
-    b[r] = br < bs ? csub(b[r], chain_elem<T>(re, im, r)) : zero_v<T>();
-  }
-  re = CT<T>::zero();
-  im = CT<T>::zero();
+    if (u < me) fload(u, f);
   auto solve = [&](auto uc, T (&d)[16]) __attribute__((always_inline)) {
     constexpr int u = decltype(uc)::value;
-    if (me == u) rest();
+    if (me == u) {
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int br = w0 + CT<T>::row(lane, r);
+        sb[br][i] = br < bs ? b[r] : zero_v<T>();
+        if (EXACT) sl[br][i] = br < bs ? bl[r] : zero_v<T>();
+      }
+    }
     __syncthreads();
-    T y = sub(u) + i < bs ? sb[sub(u) + i][c4 + kq] : zero_v<T>();
+    const int row = sub(u) + i;
+    // y + yl: what is left (EXACT: yl as bl, else the products' own sum)
+    T y = sb[row][c4 + kq], yl = EXACT ? sl[EXACT ? row : 0][c4 + kq] : zero_v<T>();
+    const T dd = UNIT ? unit_v<T>() : sd[row], rd = UNIT ? unit_v<T>() : sr[row];
+    auto value = [&]() __attribute__((always_inline)) {
+      const T z = cadd(y, yl);
+      return UNIT ? z : EXACT ? quot(z, dd, rd) : cmul(z, rd);
+    };
     static_for<0, 15>([&](auto sc) __attribute__((always_inline)) {
       constexpr int s = decltype(sc)::value, k = FWD ? s : 15 - s;
-      const T v = row_bcast<k>(UNIT ? y : cmul(y, rd[u]));
-      if (FWD ? i > k : i < k) y = fnma_t(y, d[s], v);
+      const T v = row_bcast<k>(value());
+      if (FWD ? i > k : i < k) {
+        if (EXACT) sub2(y, yl, fmul_t(d[s], v));
+        else yl = fnma_t(yl, d[s], v);
+      }
     });
-    if (!UNIT) y = cmul(y, rd[u]);
-    sb[sub(u) + i][c4 + kq] = y;
+    sb[row][c4 + kq] = value();
     __syncthreads();
-    if (u < me) {
+    if constexpr (u < 3)
+      if (u < me) {
+        T z[4];
 #pragma unroll
-      for (int s = 0; s < 4; s++) chain_mac1<T>(x[4 * u + s], sb[sub(u) + 4 * s + kq][i], re, im);
-    }
+        for (int s = 0; s < 4; s++) z[s] = sb[sub(u) + 4 * s + kq][i];
+        take(f + 4 * u, z, 4);
+      }
   };
-  solve(std::integral_constant<int, 0>{}, m);
-  dload(2, m);
+  solve(std::integral_constant<int, 0>{}, x);
+  dload(2, x);
   solve(std::integral_constant<int, 1>{}, a);
   dload(3, a);
-  solve(std::integral_constant<int, 2>{}, m);
+  solve(std::integral_constant<int, 2>{}, x);
   solve(std::integral_constant<int, 3>{}, a);
 #pragma unroll
   for (int r = 0; r < 4; r++) {

@@ -194,3 +194,71 @@ def test_badly_scaled_blocks(sx, O, dtype, noalloc):
         c = 1.0 if dtype == "float64" else 2.0 * np.sqrt(2.0)
         print(f"  {float(np.max(res / bound)):.2e}", flush=True)
         assert np.max(res / bound) <= 2 * c * n * EPS[dtype]
+
+
+def triangular(F, piv, B, trans, dtype, partial):
+    """op(P^T L U) X = B row by row in dtype; a row's products in `partial`
+    strided partial sums (0: one sum)"""
+    n = F.shape[0]
+    F, X = F.astype(dtype), B.astype(dtype)
+    pad = np.zeros((max(1, partial) * (-(-n // max(1, partial))), X.shape[1]), dtype=dtype)
+
+    def dot(a, lo, hi):
+        if not partial:
+            return a @ X[lo:hi]
+        v = pad[:partial * (-(-(hi - lo) // partial))]
+        v[:hi - lo] = a[:, None] * X[lo:hi]
+        v[hi - lo:] = 0
+        s = np.zeros((partial, X.shape[1]), dtype=dtype)
+        for part in v.reshape(-1, partial, X.shape[1]):
+            s = s + part
+        while len(s) > 1:
+            s = s[:len(s) // 2] + s[len(s) // 2:]
+        return s[0]
+
+    if trans == "N":
+        for i in range(n):
+            X[[i, piv[i] - 1]] = X[[piv[i] - 1, i]]
+        for i in range(1, n):
+            X[i] = X[i] - dot(F[i, :i], 0, i)
+        for i in range(n - 1, -1, -1):
+            X[i] = (X[i] - dot(F[i, i + 1:], i + 1, n)) / F[i, i]
+    else:
+        for i in range(n):
+            X[i] = (X[i] - dot(F[:i, i], 0, i)) / F[i, i]
+        for i in range(n - 2, -1, -1):
+            X[i] = X[i] - dot(F[i + 1:, i], i + 1, n)
+        for i in range(n - 1, -1, -1):
+            X[[i, piv[i] - 1]] = X[[piv[i] - 1, i]]
+    return X
+
+
+# rounding of the solves against the same factors in wider arithmetic.  The
+# yardstick is substitution in the same type with a row's products in 256
+# partial sums, as one workgroup a row would take them: transposed systems
+# are to be no further off (they were 2.1 to 3.7 times as far), untransposed ones
+# within the 2.2 times that products with the diagonal blocks' inverses had (they
+# were 3.5 times as far in complex types).  Both are averages over eight
+# columns; a quarter more allows for their scatter
+@pytest.mark.parametrize("dtype", ["complex128", "float64", "complex64"])
+@pytest.mark.parametrize("n,nrhs", [(100, 8), (300, 8), (970, 8)])
+def test_solve_rounding(sx, n, nrhs, dtype):
+    print(f"solve rounding n={n} {dtype}", flush=True)
+    scale = 1.0 if dtype == "float64" else np.sqrt(0.5)
+    A = (matrix(n, "complex128" if dtype != "float64" else dtype, 5 * n) * scale + 1.2 * np.sqrt(n) * np.eye(n))
+    M = sx.HMatrix.from_numpy(A.astype(dtype), dtype=dtype)
+    assert M.LUFactorize() == 0
+    F, piv = M.numpy(), M.ipiv.cpu().numpy()
+    B = matrix(max(n, nrhs), dtype, n)[:n, :nrhs].copy()
+    wide = {"complex128": np.clongdouble, "float64": np.longdouble, "complex64": np.complex128}[dtype]
+    for trans, allowed in (("N", 2.2), ("T", 1.0)):
+        exact = triangular(F, piv, B, trans, wide, 0)
+
+        def err(X):
+            return float(np.linalg.norm(np.abs(X - exact)) / np.linalg.norm(np.abs(exact)))
+
+        X = sx.HMatrix.from_numpy(B, dtype=dtype)
+        M.LUSolve(X, Trans=trans)
+        e, e0 = err(X.numpy()), err(triangular(F, piv, B, trans, dtype, 256))
+        print(f"  {trans} {e:.2e}, yardstick {e0:.2e}", flush=True)
+        assert e <= 1.25 * allowed * e0, (trans, e, e0)
