@@ -1772,8 +1772,10 @@ k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin
   }
 }
 
-// One right-hand side, all block steps in one cooperative launch.
-// Workgroup g owns the 64 rows of block g: it subtracts the off-diagonal
+// One right-hand side, all block steps in one launch.  A workgroup owns the
+// 64 rows of a block, which it takes in solve order from a ticket, so that it
+// only ever waits for workgroups that have started (no residency is needed, and
+// an ordinary launch stays on the stream's own queue): it subtracts the off-diagonal
 // blocks' products with every earlier solution block as that block is
 // published (forward: blocks k < g of L; backward: k > g of U), then
 // solves with the diagonal block and publishes its own 64 values.  The
@@ -1829,14 +1831,19 @@ __global__ void k_chain_fill(T *x, long n)
 
 template <typename T, bool LOWER, bool SUB>
 __global__ void __launch_bounds__(256)
-k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int mark, unsigned *err)
+k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int mark, unsigned *err, unsigned *ticket)
 {
+  __shared__ unsigned s_tk;
   __shared__ T part[4][TB];
   __shared__ T bx[TB];
   __shared__ T sD[SUB ? TB : 1][TB];       // [column][row] of the diagonal block
   const int t = threadIdx.x, r = t & (TB - 1), q = t >> 6;
   const long nblk = (n + TB - 1) / TB;
-  const long g = blockIdx.x;
+  if (t == 0) s_tk = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const long nk = s_tk;                      // blocks before this one in solve order
+  if (nk >= nblk) return;
+  const long g = LOWER ? nk : nblk - 1 - nk;
   const long row = g * TB + r;
   const int bs = (int)std::min<long>(TB, n - g * TB);
   T b = zero_v<T>();
@@ -1844,8 +1851,6 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
     b = bin[row];
     if (mark) chain_mark(bin + row);
   }
-  // blocks k in solve order before g
-  const long nk = LOWER ? g : nblk - 1 - g;
   auto blk = [&](long i) { return LOWER ? i : nblk - 1 - i; };
   auto load = [&](long k, T (&a)[16]) {
 #pragma unroll
@@ -2236,23 +2241,9 @@ __global__ void k_zero_u64(unsigned long long *w, long n)
   if (i < n) w[i] = 0ull;
 }
 
-// whether a grid of one workgroup per 64 rows is resident (cooperative launch)
-template <typename T> static bool chain_resident(long n)
-{
-  static int ncu = -1, perCU = 0;
-  if (ncu < 0) {
-    int dev = 0, c = 0;
-    hipGetDevice(&dev);
-    hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_trsv_chain<T, true, true>, 256, 0);
-    hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, dev);
-    ncu = c;
-  }
-  return (long)ncu * perCU >= (n + TB - 1) / TB;
-}
-
 // lower (forward) then upper (backward) solve of one right-hand side in
-// two cooperative launches (chain_resident(n)), by substitution if the block
-// inverses are null; returns -2 without a workspace, -6 on a time-out
+// two launches, by substitution if the block inverses are null; returns -2
+// without a workspace, -6 on a time-out
 template <typename T>
 static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *invU, T *B, T *W, hipStream_t s,
                       unsigned long long *words)
@@ -2260,24 +2251,23 @@ static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *inv
   const long nblk = (n + TB - 1) / TB;
   char *w = words ? (char *)words : (char *)ws_get(WS_CHAIN, sizeof(unsigned long long) * (2 * nblk + 8));
   if (!w) return -2;
-  unsigned *err = (unsigned *)w;
+  unsigned *err = (unsigned *)w, *ticket = (unsigned *)(w + sizeof(unsigned long long));
   // cleared and filled by kernels (not memset nodes, so that a captured
   // sequence does the same on every replay)
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, s, (unsigned long long *)w, 8L);
   hipLaunchKernelGGL(k_chain_fill<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, W, n);
-  int mark = 1, nomark = 0;
-  void *al[] = {(void *)&LU, (void *)&lda, (void *)&n, (void *)&invL, (void *)&B, (void *)&W, (void *)&mark,
-                (void *)&err};
-  const void *kl = (const void *)k_trsv_chain<T, true, true>, *ku = (const void *)k_trsv_chain<T, false, true>;
-  if constexpr (std::is_same<T, float2>::value)
-    if (invL) {
-      kl = (const void *)k_trsv_chain<T, true, false>;
-      ku = (const void *)k_trsv_chain<T, false, false>;
-    }
-  if (hipLaunchCooperativeKernel(kl, dim3((unsigned)nblk), dim3(256), al, 0, s) != hipSuccess) return -3;
-  void *au[] = {(void *)&LU, (void *)&lda, (void *)&n, (void *)&invU, (void *)&W, (void *)&B, (void *)&nomark,
-                (void *)&err};
-  if (hipLaunchCooperativeKernel(ku, dim3((unsigned)nblk), dim3(256), au, 0, s) != hipSuccess) return -3;
+  auto both = [&](auto sub) {
+    hipLaunchKernelGGL((k_trsv_chain<T, true, decltype(sub)::value>), dim3((unsigned)nblk), dim3(256), 0, s, LU, lda, n,
+                       invL, B, W, 1, err, ticket);
+    hipLaunchKernelGGL((k_trsv_chain<T, false, decltype(sub)::value>), dim3((unsigned)nblk), dim3(256), 0, s, LU, lda, n,
+                       invU, W, B, 0, err, ticket + 2);
+  };
+  if constexpr (std::is_same<T, float2>::value) {
+    if (invL) both(std::false_type{});
+    else both(std::true_type{});
+  } else
+    both(std::true_type{});
+  if (hipGetLastError() != hipSuccess) return -3;
   unsigned tmo = 0;
   hipMemcpyAsync(&tmo, err, sizeof(unsigned), hipMemcpyDeviceToHost, s);
   hipStreamSynchronize(s);
@@ -2394,7 +2384,7 @@ int lu_solve(const T *LU, long n, long lda, const int *d_ipiv, char trans, long 
   if (ws && !((trans == 'N' || trans == 'n') && nrhs == 1)) return -1;
   const bool tr = trans == 'T' || trans == 't' || trans == 'C' || trans == 'c', cj = trans == 'C' || trans == 'c';
   if (!tr && trans != 'N' && trans != 'n') return -1;
-  if (!tr && nrhs == 1 && chain_resident<T>(n)) {
+  if (!tr && nrhs == 1) {
     T *W = ws ? ws->W : (T *)ws_get(WS_SOLVE_W, sizeof(T) * n);
     if (!W) return -2;
     // a solve after the first with the same factors reuses the block
