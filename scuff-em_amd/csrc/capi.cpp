@@ -1160,6 +1160,7 @@ int tune_nb(long n, int nbat, SweepBuf &B, hipStream_t s)
   if (const char *e = getenv("SCUFFX_SWEEP_NB")) return std::max(32, std::min(256, atoi(e) / 32 * 32));
   int best = 256;
   float best_ms = 1e30f;
+  PanelPass pass(lu_batch_workgroups(n, nbat), lu_batch_slots());
   hipEvent_t e0, e1;
   hipEventCreate(&e0);
   hipEventCreate(&e1);
@@ -1356,8 +1357,15 @@ int scuffx_sweep_batched(scuffx_geom **Gs, int ngeom, const double *omegas, int 
     t[2] = now_ms();
   }
   t[3] = now_ms();
-  hipError_t le = hipGraphLaunch(exec, cs);
-  hipError_t se = hipStreamSynchronize(cs);
+  hipError_t le, se;
+  {
+    // the graph's batches run one after another
+    long wgs = 0;
+    for (int g = 0; g < ngeom; g++) wgs = std::max(wgs, lu_batch_workgroups(bufs[g].n, bufs[g].nbmax));
+    PanelPass pass(wgs, lu_batch_slots());
+    le = hipGraphLaunch(exec, cs);
+    se = hipStreamSynchronize(cs);
+  }
   t[4] = now_ms();
   if (le != hipSuccess || se != hipSuccess) {
     state.graph.release();

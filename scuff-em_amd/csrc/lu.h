@@ -11,6 +11,20 @@
 
 namespace scuffx {
 
+// the share of the current GPU's workgroup slots that panels of `workgroups`
+// take, held until destruction (gate.h); factorizations take it themselves
+class PanelPass {
+ public:
+  PanelPass(long workgroups, long slots);
+  ~PanelPass();
+  PanelPass(const PanelPass &) = delete;
+  PanelPass &operator=(const PanelPass &) = delete;
+
+ private:
+  int dev_ = 0;
+  double share_ = 0.0;
+};
+
 // T = double2 (complex128), float2 (complex64) or double (real, the LHM_REAL
 // matrices of imaginary frequencies: dgetrf/dgetrs semantics).  fast = 1 solves the
 // block rows with the explicit inverses of the 32x32 unit-lower panel
@@ -67,6 +81,10 @@ long noalloc_scratch_bytes();
 // panel workgroups cannot all be resident (nbat > lu_batch_max(n)).
 size_t lu_batch_scratch_bytes(long n);
 int lu_batch_max(long n);
+// panel workgroups of such a batch and the slots there are for them: whoever
+// runs one, directly or as a graph, holds a PanelPass until it has completed
+long lu_batch_workgroups(long n, int nbat);
+long lu_batch_slots();
 // nb: columns per block (a multiple of 32, at most 256)
 int lu_factor_batch(float2 *A, long n, long lda, int nbat, long sa, int *ipiv, long sp, void *scratch, int *status,
                     hipStream_t s, int nb = 256);

@@ -19,6 +19,7 @@
 #include <type_traits>
 #include <vector>
 
+#include "gate.h"
 #include "lu.h"
 #include "lu_dev.h"
 #include "prof.h"
@@ -1340,8 +1341,21 @@ static void trsm_blk(const T *A, long lda, long r0, int jb, const T *linv, T *B,
   prof_end(s, tok, 4.0 * (double)jb * (double)jb * (double)ncol);
 }
 
-// second stream of the lookahead (default priority, non-blocking), one per
-// device, created on first use
+static Gate g_gates[64];
+
+PanelPass::PanelPass(long workgroups, long slots)
+{
+  hipGetDevice(&dev_);
+  dev_ &= 63;
+  share_ = (double)workgroups / (double)std::max(1L, slots);
+  if (share_ > 0) g_gates[dev_].enter(share_);
+}
+
+PanelPass::~PanelPass()
+{
+  if (share_ > 0) g_gates[dev_].leave(share_);
+}
+
 // second stream of the lookahead (default priority, non-blocking), one per
 // device, created on first use.  (Keeping its kernels off a share of the
 // CUs with a CU-masked stream was measured 1.7x slower on gfx950.)
@@ -1389,8 +1403,14 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   hipGetDevice(&dev);
   hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, panel_fn, NR, 0);
+  if (!tourn && Gmax > PX_ONE) {           // (its last panels are of the other kernel)
+    int one = 0;
+    hipOccupancyMaxActiveBlocksPerMultiprocessor(&one, panel_one, NR, 0);
+    perCU = std::min(perCU, one);
+  }
   // the tournament launches one more workgroup (it inverts the diagonal block)
-  if ((long)std::max(1, ncu) * std::max(1, perCU) < Gmax + (tourn ? 1 : 0)) return -5;   // not co-resident
+  const long slots = (long)std::max(1, ncu) * std::max(1, perCU), grid = Gmax + (tourn ? 1 : 0);
+  if (slots < grid) return -5;                                        // not co-resident
   if (Gmax > 64 * KEYS_PER_LANE) return -5;                           // more workgroups than polled keys
   const long npanels = (n + PW - 1) / PW;
   // panel scratch, carved from one workspace: time-out word (its own cache
@@ -1411,13 +1431,16 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
   S.bar = (unsigned *)wsb;
   int *dinfo = (int *)(wsb + off_info);
   int *plans = (int *)(wsb + off_plan);
+  // panels of one workgroup wait for nobody
+  PanelPass pass(!tourn && n <= lrows ? 0 : perCU < 2 ? slots : grid, slots);
   // The trailing update runs beside the next panels on a second stream,
   // unless the panel needs more than half of the resident workgroup slots
   // of its kernel: then the GEMM's workgroups, dispatched without pause
   // on the other stream, could keep part of the panel's grid waiting until
-  // its bounded waits expire (seen at n = 61440 complex128: 480 panel
-  // workgroups of 2 per CU).  Everything then runs on the caller's stream.
-  const bool overlap = 2 * (Gmax + (tourn ? 1 : 0)) <= (long)std::max(1, ncu) * std::max(1, perCU);
+  // its bounded waits expire (seen with 480 panel workgroups in 512 slots; 240
+  // in 512, complex128 of order 61440, run beside it).  Everything then runs
+  // on the caller's stream.
+  const bool overlap = 2 * grid <= slots;
   hipStream_t side = overlap ? side_stream() : stream;
   hipEvent_t evP = nullptr, evR = nullptr;
   hipEventCreateWithFlags(&evP, hipEventDisableTiming);
@@ -2776,15 +2799,18 @@ __global__ void k_batch_status(const char *scratch, long sS, long off_info, int 
   status[2 * b + 1] = (int)((const unsigned *)base)[64];
 }
 
-int lu_batch_max(long n)
+long lu_batch_slots()
 {
   int dev = 0, ncu = 0, perCU = 0;
   hipGetDevice(&dev);
   hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
   hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCU, (const void *)k_panel_ts, 256, 0);
-  const long per = (n + 255) / 256 + 1;
-  return (int)((long)std::max(1, ncu) * std::max(1, perCU) / per);
+  return (long)std::max(1, ncu) * std::max(1, perCU);
 }
+
+long lu_batch_workgroups(long n, int nbat) { return nbat * ((n + 255) / 256 + 1); }
+
+int lu_batch_max(long n) { return (int)(lu_batch_slots() / lu_batch_workgroups(n, 1)); }
 
 int lu_factor_batch(float2 *A, long n, long lda, int nbat, long sa, int *ipiv, long sp, void *scratch, int *status,
                     hipStream_t s, int nb)

@@ -262,3 +262,44 @@ def test_solve_rounding(sx, n, nrhs, dtype):
         e, e0 = err(X.numpy()), err(triangular(F, piv, B, trans, dtype, 256))
         print(f"  {trans} {e:.2e}, yardstick {e0:.2e}", flush=True)
         assert e <= 1.25 * allowed * e0, (trans, e, e0)
+
+
+def test_factorizations_side_by_side(sx):
+    """Threads that factor at once, each on a stream of its own (both panel
+    exchanges, a panel in one workgroup, tournament pivoting): the same bits as
+    one after another."""
+    import threading
+    import torch
+    work = [(4100, "complex128"), (1500, "float64"), (2600, "complex64"), (4000, "mixed"), (400, "complex128")]
+    A = [matrix(n, "complex128" if d == "mixed" else d, n) for n, d in work]
+
+    def factor(i):
+        n, d = work[i]
+        if d != "mixed":
+            M = sx.HMatrix.from_numpy(A[i], dtype=d)
+            assert M.LUFactorize() == 0
+            return M.t, M.ipiv
+        M = sx.HMatrix.from_numpy(A[i])
+        LU32 = torch.zeros((n, n), dtype=torch.complex64, device="cuda")
+        ipiv = torch.zeros(n, dtype=torch.int32, device="cuda")
+        sx._sync_stream()
+        assert sx.lib().scuffx_lu32_from_c128(sx._ptr(M.t), n, n, sx._ptr(LU32), n, sx._ptr(ipiv)) == 0
+        return LU32, ipiv
+
+    print("factorizations side by side", flush=True)
+    alone = [[t.cpu() for t in factor(i)] for i in range(len(work))]
+    together = [None] * len(work)
+
+    def thread(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            out = factor(i)
+            torch.cuda.current_stream().synchronize()
+            together[i] = [t.cpu() for t in out]
+
+    ts = [threading.Thread(target=thread, args=(i,)) for i in range(len(work))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for a, b in zip(alone, together):
+        assert b is not None and all(torch.equal(x, y) for x, y in zip(a, b))
