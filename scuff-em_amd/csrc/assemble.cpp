@@ -12,6 +12,7 @@
 // pairs (Taylor-Duffy); a final kernel combines them per edge pair.
 #include "assemble.h"
 #include "fippi_cache.h"
+#include "fippi_heap.h"
 #include "prof.h"
 #include "ws.h"
 
@@ -528,21 +529,25 @@ int Assembler::build_fippi(hipStream_t stream)
     // separated pairs first: some of them split regions thousands of times,
     // and whatever starts last ends last
     std::stable_partition(todo.begin(), todo.end(), [&](int j) { return jobs_[j].ncv == 0; });
-    // heaps large enough for the whole evaluation budget (1e6 points, 66 per
-    // split), one per resident workgroup (four per CU, 9.5 MB each), fewer if
-    // there is no memory for them
-    const int cap = 15360;
-    int slots = std::min(1024, nt);
+    // a heap per workgroup (records, keys and slot numbers in one allocation:
+    // one that fits leaves nothing to fail after it).  The kernel's own private
+    // memory comes on top, up to 4.5 GB: a launch that cannot have it aborts the
+    // queue, so that much and 1 GB stay free
     Scratch sc;
     int *d_counter = sc.alloc<int>(1), *d_ovf = sc.alloc<int>(nj), *d_todo = sc.put(todo);
-    double *hd = nullptr;
-    while (!(hd = sc.alloc<double>((size_t)cap * 76 * slots)) && slots > 1) {
+    size_t mfree = 0, mtotal = 0, priv = 0;
+    HIPCHK(hipMemGetInfo(&mfree, &mtotal));
+    HIPCHK(fippi_private_bytes(&priv));
+    int slots = fippi_slots(nt, mfree, priv + ((size_t)1 << 30));
+    char *heap = nullptr;
+    while (!(heap = sc.alloc<char>(kFippiHeapBytes * slots)) && slots > 1) {
       hipGetLastError();
       slots = (slots + 1) / 2;
     }
-    double *hk = sc.alloc<double>((size_t)cap * slots);
-    int *hs = sc.alloc<int>((size_t)cap * slots);
-    if (!d_counter || !d_ovf || !d_todo || !hd || !hk || !hs) { err_ = "device allocation failed"; return -2; }
+    if (!d_counter || !d_ovf || !d_todo || !heap) { err_ = "device allocation failed"; return -2; }
+    const int cap = kFippiCap;
+    double *hd = (double *)heap, *hk = hd + (size_t)cap * 76 * slots;
+    int *hs = (int *)(hk + (size_t)cap * slots);
     HIPCHK(hipMemsetAsync(d_ovf, 0, sizeof(int) * nj, stream));
     HIPCHK(hipMemsetAsync(d_counter, 0, sizeof(int), stream));
     int tok = prof_begin(stream, PK_FIPPI);

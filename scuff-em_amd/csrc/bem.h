@@ -85,6 +85,8 @@ hipError_t launch_self(hipStream_t stream, const double *V, const int *PVI, int 
 // its waves (ten on a CU)
 #define SCUFFX_SELF_SLAB (960 * 20)
 #define SCUFFX_SELF_SLABS 2560
+// device memory that the runtime may want for that kernel's private arrays
+hipError_t fippi_private_bytes(size_t *bytes);
 hipError_t launch_fippi(hipStream_t stream, const FippiJob *jobs, int njobs, double *records,
                         double *heapData, int *heapSlot, double *heapKey, int cap, int nslots,
                         int *counter, int *overflow, const int *jobList);

@@ -846,6 +846,18 @@ k_fippi(const FippiJob *jobs, int njobs, const int *jobList, double *records,
   }
 }
 
+hipError_t fippi_private_bytes(size_t *bytes)
+{
+  int dev = 0, ncu = 0, threads = 0;
+  hipFuncAttributes a;
+  hipError_t e = hipGetDevice(&dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess) e = hipDeviceGetAttribute(&threads, hipDeviceAttributeMaxThreadsPerMultiProcessor, dev);
+  if (e == hipSuccess) e = hipFuncGetAttributes(&a, (const void *)k_fippi);
+  if (e == hipSuccess) *bytes = a.localSizeBytes * (size_t)ncu * (size_t)threads;
+  return e;
+}
+
 hipError_t launch_fippi(hipStream_t stream, const FippiJob *jobs, int njobs, double *records,
                         double *heapData, int *heapSlot, double *heapKey, int cap, int nslots,
                         int *counter, int *overflow, const int *jobList)
