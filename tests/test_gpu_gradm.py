@@ -92,3 +92,22 @@ def test_torque_derivatives_match_oracle(sx, O, mats):
         e = rel_fro(TB[t].numpy(), TBo[t])
         print(f"  torque axis {axes[t]}: {e:.2e}", flush=True)
         assert e <= 1e-12
+
+
+def test_gradm_in_bands(sx, O, monkeypatch):
+    """Conducting pairs combine their derivatives from panel-pair records band
+    by band of the column panels (SCUFFX_FAR_BAND_MB; here three bands of 32, 32
+    and 16 panels): the same bits as in one."""
+    print("gradm in bands", flush=True)
+
+    def block():
+        G, _ = pair(sx, O, 1, (PEC, PEC), (0.2, 0.1, 2.6))
+        return G.AssembleBEMMatrixBlock(0, 1, 0.7 + 0.2j, GradM=True)
+
+    B, GB = block()
+    monkeypatch.setenv("SCUFFX_FAR_BAND_MB", "1")
+    B3, GB3 = block()
+    assert np.array_equal(B.numpy(), B3.numpy())
+    for m in range(3):
+        assert np.array_equal(GB[m].numpy(), GB3[m].numpy())
+        assert np.abs(GB[m].numpy()).max() > 0

@@ -83,6 +83,31 @@ def test_panel_both_exchanges(sx):
     assert np.max(np.abs(M.numpy() - LU)) <= 4 * n * EPS["float64"] * np.max(np.abs(LU)) * 10
 
 
+# the same with the complex slots (66 and 34 words).  complex128: LAPACK's
+# pivots; complex64, where roundings decide near-ties: P A v = L (U v) for
+# vectors v, and multipliers of at most sqrt(2)
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_panel_both_exchanges_complex(sx, dtype):
+    import scipy.linalg as sl
+    n = 4100
+    print(f"both panel exchanges n={n} {dtype}", flush=True)
+    A = matrix(n, dtype, 5)
+    M = sx.HMatrix.from_numpy(A, dtype=dtype)
+    assert M.LUFactorize() == 0
+    F, piv = M.numpy(), M.ipiv.cpu().numpy()
+    if dtype == "complex128":
+        assert np.array_equal(piv, sl.lu_factor(A)[1] + 1)
+    assert np.abs(np.tril(F, -1)).max() <= np.sqrt(2.0) * (1 + 8 * EPS[dtype])
+    perm = np.arange(n)
+    for i in range(n):
+        perm[[i, piv[i] - 1]] = perm[[piv[i] - 1, i]]
+    V = matrix(n, "complex128", 8)[:, :4]
+    UV = np.triu(F).astype("complex128") @ V
+    LUV = np.tril(F, -1).astype("complex128") @ UV + UV
+    res = np.linalg.norm(A.astype("complex128")[perm] @ V - LUV) / (np.linalg.norm(A) * np.linalg.norm(V) / np.sqrt(n))
+    assert res <= 4 * n * EPS[dtype], res        # (as for the smaller orders)
+
+
 # solves by blocks of 64 rows and tiles of 16 columns: one row, the edges of
 # a block and of a tile, one and several blocks, a ragged last block; 1100
 # columns take two sets
