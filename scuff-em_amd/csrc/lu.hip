@@ -1998,17 +1998,18 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
 // complex128; products with the explicit inverse 2 us, but where the block is
 // badly scaled, eps = 10 spheres at imaginary frequency 0.001, they lose every
 // digit.)  The entries of the first sub-block wait in LDS.
-// Rounding: a block's 64 products and a sub-block's own are summed by
-// themselves and subtracted once, not term by term from the right-hand side.
-// Transposed systems (EXACT) sum two k-steps at a time, keep what the
+// Rounding: a block's 64 products are summed two k-steps at a time, a
+// sub-block's own by themselves, and subtracted once, not term by term from the
+// right-hand side.  Transposed systems (EXACT) also keep what the
 // subtractions lose (two-sums, added back before each use) and correct the
-// quotients: their error then is that of a dot product of 256 partial sums and
-// one division a row, i.e. 0.85 to 1.07 of it over orders 100 to 1500 and the
-// three types, where sums over four blocks, products subtracted term by term
-// and rounded reciprocals had 1.7 to 3.8 times as much (up to 1.7 times as much
-// as products with the blocks' inverses in the untransposed form, now 0.7 to
-// 0.98).  One transposed system, order 3840, complex128: 1.69 -> 2.13 ms; the
-// untransposed forms take the same time.
+// quotients.  Their error then is that of a dot product of 256 partial sums and
+// one division a row: 0.85 to 1.07 of it over orders 100 to 1500 and the
+// three types, where one sum over four blocks, products subtracted term by term
+// and rounded reciprocals had 1.7 to 3.8 times as much.  Untransposed it is 0.4 to
+// 0.9 of what products with the blocks' inverses had (2 to 16 columns; up to
+// 1.7 before), inverses of order 64 and up at most that of substitution in
+// 256-row blocks (1.02; up to 1.28 before).  One transposed system, order 3840,
+// complex128: 1.69 -> 2.13 ms; two untransposed columns 1.43 -> 1.46 ms.
 // bin: column-major right-hand sides, row r taken from pin[r] if given, or
 // null: packed in win.  bout: column-major results or null, row r to pout[r]
 // if given.  cj: 1 conjugates the right-hand sides, 2 the results in bout.
@@ -2159,16 +2160,16 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
     } else if (br < bs) b[r] = p.win[(tile * nblk * TB + row) * NC + i];
   }
   __syncthreads();
-  // the sum of ns k-steps' products (EXACT: of two each, added up), taken from b
+  // ns k-steps' products, summed by two each and added up, taken from b
   auto take = [&](const T *a, const T *x, int ns) __attribute__((always_inline)) {
     V4 re = CT<T>::zero(), im = CT<T>::zero();
 #pragma unroll
     for (int s = 0; s < ns; s += 2) {
-      V4 tr = EXACT ? CT<T>::zero() : re, ti = EXACT ? CT<T>::zero() : im;
+      V4 tr = CT<T>::zero(), ti = CT<T>::zero();
       chain_mac<T>(a[s], x[s], tr, ti);
       chain_mac<T>(a[s + 1], x[s + 1], tr, ti);
-      if (EXACT) { re += tr; im += ti; }
-      else { re = tr; im = ti; }
+      re += tr;
+      im += ti;
     }
 #pragma unroll
     for (int r = 0; r < 4; r++) {

@@ -261,12 +261,12 @@ def triangular(F, piv, B, trans, dtype, partial):
 # rounding of the solves against the same factors in wider arithmetic.  The
 # yardstick is substitution in the same type with a row's products in 256
 # partial sums, as one workgroup a row would take them: transposed systems
-# are to be no further off (they were 2.1 to 3.7 times as far), untransposed ones
-# within the 2.2 times that products with the diagonal blocks' inverses had (they
-# were 3.5 times as far in complex types).  Both are averages over eight
-# columns; a quarter more allows for their scatter
+# are to be no further off (they were 1.7 to 3.7 times as far), untransposed ones,
+# which do not keep what their subtractions lose, within 1.5 times (they were 1.7
+# to 3.5; seen 1.2 to 1.5).  A quarter more allows for the scatter of eight
+# columns; 0 columns: the inverse
 @pytest.mark.parametrize("dtype", ["complex128", "float64", "complex64"])
-@pytest.mark.parametrize("n,nrhs", [(100, 8), (300, 8), (970, 8)])
+@pytest.mark.parametrize("n,nrhs", [(100, 8), (300, 8), (970, 8), (64, 0), (200, 0)])
 def test_solve_rounding(sx, n, nrhs, dtype):
     print(f"solve rounding n={n} {dtype}", flush=True)
     scale = 1.0 if dtype == "float64" else np.sqrt(0.5)
@@ -274,9 +274,9 @@ def test_solve_rounding(sx, n, nrhs, dtype):
     M = sx.HMatrix.from_numpy(A.astype(dtype), dtype=dtype)
     assert M.LUFactorize() == 0
     F, piv = M.numpy(), M.ipiv.cpu().numpy()
-    B = matrix(max(n, nrhs), dtype, n)[:n, :nrhs].copy()
+    B = matrix(max(n, nrhs), dtype, n)[:n, :nrhs].copy() if nrhs else np.eye(n, dtype=dtype)
     wide = {"complex128": np.clongdouble, "float64": np.longdouble, "complex64": np.complex128}[dtype]
-    for trans, allowed in (("N", 2.2), ("T", 1.0)):
+    for trans, allowed in (("N", 1.5), ("T", 1.0)):
         exact = triangular(F, piv, B, trans, wide, 0)
 
         def err(X):
