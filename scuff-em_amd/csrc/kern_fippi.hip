@@ -640,7 +640,8 @@ __device__ inline double wave_max(double v)
 // panels), 5.4 us each: a 960-function sphere's table 82 ms, N=3840 169 ms.  One
 // wave a job, 66 points on 64 lanes in two rounds, the heap in HBM and jobs
 // past 4096 regions started again: 35 us a split, 512 and 433 ms.
-// LDS: 40 KB, four workgroups on a CU, as many as the registers allow.
+// LDS: 40 KB, four workgroups on a CU, as many as the registers allow.  8.6 KB of
+// scratch memory a lane hold the common-vertex integrands' tables.
 __global__ void __launch_bounds__(128, 2)
 k_fippi(const FippiJob *jobs, int njobs, const int *jobList, double *records,
         double *heapData, int *heapSlot, double *heapKey, int cap, int *counter, int *overflow)

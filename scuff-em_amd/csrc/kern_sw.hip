@@ -740,7 +740,8 @@ template <int CASE> struct TDFun {
 // every gridDim-th job (a launch per 4096 jobs waited 240 times for its last
 // one).  KIND SW_SEP: no-common-vertex near pairs (all 9 combinations),
 // TD_CV, TD_CE, TD_CT: pairs with one, two or three common vertices, one
-// (Qa, Qb) a job; a kernel each, since their registers and tables differ.  A
+// (Qa, Qb) a job; a kernel each, since their registers and tables differ (SW_SEP
+// spills 64 registers, the others none).  A
 // Taylor-Duffy job keeps its Upsilon tables and cache entries in LDS and
 // its cached integrand values in a slab of scratch memory.
 template <int KIND>

@@ -1628,30 +1628,35 @@ __global__ void __launch_bounds__(64) k_perm_build(const int *ipiv, long n, int 
   for (long i = lane; i < n; i += 64) perm[i] = P[i];
 }
 
-// forward: out[s] = in[perm[s]]; reverse: out[perm[s]] = in[s]
-template <typename T, bool FWD>
-__global__ void __launch_bounds__(256) k_perm_apply(const T *in, long ldi, T *out, long ldo, const int *perm, long n,
-                                                    long sin, long sout, long sperm)
+// out[s] = in[perm[s]]
+template <typename T>
+__global__ void __launch_bounds__(256) k_perm_apply(const T *in, T *out, const int *perm, long n, long sin, long sout,
+                                                    long sperm)
 {
   {
     const long z = blockIdx.z;   // instance of a batch
     in += z * sin; out += z * sout; perm += z * sperm;
   }
   const long s = (long)blockIdx.x * 256 + threadIdx.x;
-  if (s >= n) return;
-  const long c = blockIdx.y;
-  const long p = perm[s];
-  if (FWD) out[s + c * ldo] = in[p + c * ldi];
-  else out[p + c * ldo] = in[s + c * ldi];
+  if (s < n) out[s] = in[perm[s]];
 }
 
-// applies the interchanges of ipiv to the nrhs columns of B (forward, as
-// laswp with increment 1) or their inverse (reverse order); tmp holds n x
-// nrhs elements; perm_ready: perm_buf already holds the composed
+// applies the interchanges of ipiv to b (as laswp with increment 1); tmp
+// holds n elements; perm_ready: perm_buf already holds the composed
 // permutation of ipiv
 template <typename T>
-static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, bool fwd, T *tmp, hipStream_t s,
-                           int *perm_buf = nullptr, bool perm_ready = false);
+static void apply_row_perm(T *b, long n, const int *ipiv, T *tmp, hipStream_t s, int *perm_buf, bool perm_ready)
+{
+  int *perm = n > PERM_LDS_MAX ? nullptr : perm_buf ? perm_buf : (int *)ws_get(WS_PERM, sizeof(int) * n);
+  if (!perm) {
+    // beyond the LDS copy: the interchanges one after another
+    laswp(b, n, 0, 1, 0, n, ipiv, s);
+    return;
+  }
+  if (!(perm_ready && perm == perm_buf)) hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(64), 0, s, ipiv, n, perm, 0L, 0L);
+  hipLaunchKernelGGL(k_perm_apply<T>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, b, tmp, perm, n, 0L, 0L, 0L);
+  hipMemcpyAsync(b, tmp, sizeof(T) * n, hipMemcpyDeviceToDevice, s);
+}
 
 // Inverses of the diagonal 64x64 blocks of L (unit lower, blockIdx.y = 0)
 // and U (blockIdx.y = 1), identity past row n: every block step of a
@@ -1661,9 +1666,9 @@ static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, b
 // refinement).  One workgroup a block, a wave for 16 columns of the inverse, a
 // lane for a row; a step passes one row's values of every column by lane
 // reads.  Bound: issue of the lane reads and updates.  A column per thread of
-// one wave, its sums from LDS, took 100 us for each triangle, this takes 59 us
-// for both in complex128 (order 2501; the first 16 (q + 1) columns only in
-// steps 16 q ..: 78 us with every column in every step).
+// one wave, its sums from LDS, took 100 us for each triangle, this 59 us for
+// both (order 2501, in complex128, which substitutes by now; the first 16 (q + 1)
+// columns only in steps 16 q ..: 78 us with every column in every step).
 #define TB 64
 template <typename T>
 __global__ void __launch_bounds__(256)
@@ -1731,11 +1736,11 @@ static void tri_inv(const T *LU, long lda, long n, T *invL, T *invU, hipStream_t
 
 // one block step: x_b = inv(D_b) r_b (every workgroup, from L2), the
 // solution written to Xout by workgroup 0, and the rows outside the block
-// updated with x_b (LOWER: rows below, else rows above); blockIdx.y = rhs
+// updated with x_b (LOWER: rows below, else rows above)
 template <typename T, bool LOWER>
 __global__ void __launch_bounds__(256)
-k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin, long ldb, T *Xout, long ldx,
-           long sa, long sinv, long sb, long sx)
+k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin, T *Xout, long sa, long sinv, long sb,
+           long sx)
 {
   {
     const long z = blockIdx.z;   // instance of a batch
@@ -1743,8 +1748,7 @@ k_trsv_inv(const T *LU, long lda, long n, long kb, int bs, const T *invb, T *Bin
   }
   __shared__ T rs[TB], xs[TB];
   const int t = threadIdx.x;
-  T *b = Bin + (long)blockIdx.y * ldb;
-  T *xo = Xout + (long)blockIdx.y * ldx;
+  T *b = Bin, *xo = Xout;
   if (t < TB) {
     if (t < bs) rs[t] = b[kb + t]; else { rs[t] = zero_v<T>(); }
   }
@@ -2298,24 +2302,6 @@ static int trsv_chain(const T *LU, long lda, long n, const T *invL, const T *inv
   return tmo ? -6 : 0;
 }
 
-template <typename T>
-static void apply_row_perm(T *B, long ldb, long n, long nrhs, const int *ipiv, bool fwd, T *tmp, hipStream_t s,
-                           int *perm_buf, bool perm_ready)
-{
-  int *perm = n > PERM_LDS_MAX ? nullptr : perm_buf ? perm_buf : (int *)ws_get(WS_PERM, sizeof(int) * n);
-  if (!perm || !tmp) {
-    // beyond the LDS copy: the interchanges one after another, per column
-    if (fwd) laswp(B, ldb, 0, nrhs, 0, n, ipiv, s);
-    else hipLaunchKernelGGL(k_laswp_rev<T>, dim3((unsigned)((nrhs + 63) / 64)), dim3(64), 0, s, B, ldb, n, nrhs, ipiv);
-    return;
-  }
-  if (!(perm_ready && perm == perm_buf)) hipLaunchKernelGGL(k_perm_build, dim3(1), dim3(64), 0, s, ipiv, n, perm, 0L, 0L);
-  dim3 grid((unsigned)((n + 255) / 256), (unsigned)nrhs);
-  if (fwd) hipLaunchKernelGGL((k_perm_apply<T, true>), grid, dim3(256), 0, s, B, ldb, tmp, n, perm, n, 0L, 0L, 0L);
-  else hipLaunchKernelGGL((k_perm_apply<T, false>), grid, dim3(256), 0, s, B, ldb, tmp, n, perm, n, 0L, 0L, 0L);
-  hipMemcpy2DAsync(B, sizeof(T) * ldb, tmp, sizeof(T) * n, sizeof(T) * n, nrhs, hipMemcpyDeviceToDevice, s);
-}
-
 // one triangle of k_trsm_chain
 template <typename T>
 static void trsm_launch(bool fwd, bool trans, const ChainArgs<T> &p, hipStream_t s)
@@ -2422,7 +2408,7 @@ int lu_solve(const T *LU, long n, long lda, const int *d_ipiv, char trans, long 
         if (!cached) tri_inv(LU, lda, n, invL, invU, stream);
       }
     if (ws) ws->inv_ready = true;
-    apply_row_perm(B, ldb, n, nrhs, d_ipiv, true, W, stream, ws ? ws->perm : nullptr, cached);
+    apply_row_perm(B, n, d_ipiv, W, stream, ws ? ws->perm : nullptr, cached);
     return trsv_chain(LU, lda, n, invL, invU, B, W, stream, ws ? ws->chain : nullptr);
   }
   return trsm_chain(LU, lda, n, d_ipiv, tr, cj, nrhs, B, ldb, stream);
@@ -2927,15 +2913,15 @@ int lu_solve_batch(const float2 *LU, long n, long lda, int nbat, long sa, float2
   float2 *W = (float2 *)(base + L.off_W);
   const long swp = sw / 4, swe = sw / 8;   // the stride in ints and in complex64 elements
   // W = P B
-  hipLaunchKernelGGL((k_perm_apply<float2, true>), dim3((unsigned)((n + 255) / 256), 1, (unsigned)nbat), dim3(256), 0,
-                     s, (const float2 *)B, n, W, n, perm, n, sb, swe, swp);
+  hipLaunchKernelGGL(k_perm_apply<float2>, dim3((unsigned)((n + 255) / 256), 1, (unsigned)nbat), dim3(256), 0, s,
+                     (const float2 *)B, W, perm, n, sb, swe, swp);
   // L y = W: W is the running right-hand side, y lands in B
   for (long kb = 0; kb < n; kb += TB) {
     const int bs = (int)std::min<long>(TB, n - kb);
     const long rows = n - kb - bs;
     dim3 grid((unsigned)std::max<long>(1, (rows + 255) / 256), 1, (unsigned)nbat);
     hipLaunchKernelGGL((k_trsv_inv<float2, true>), grid, dim3(256), 0, s, LU, lda, n, kb, bs,
-                       invL + (kb / TB) * TB * TB, W, n, B, n, sa, swe, swe, sb);
+                       invL + (kb / TB) * TB * TB, W, B, sa, swe, swe, sb);
   }
   // U x = y: B is the running right-hand side, x lands in W
   const long last = ((n - 1) / TB) * TB;
@@ -2943,7 +2929,7 @@ int lu_solve_batch(const float2 *LU, long n, long lda, int nbat, long sa, float2
     const int bs = (int)std::min<long>(TB, n - kb);
     dim3 grid((unsigned)std::max<long>(1, (kb + 255) / 256), 1, (unsigned)nbat);
     hipLaunchKernelGGL((k_trsv_inv<float2, false>), grid, dim3(256), 0, s, LU, lda, n, kb, bs,
-                       invU + (kb / TB) * TB * TB, B, n, W, n, sa, swe, sb, swe);
+                       invU + (kb / TB) * TB * TB, B, W, sa, swe, sb, swe);
   }
   // B = x
   hipLaunchKernelGGL(k_copy_batch, dim3((unsigned)((n + 255) / 256), 1, (unsigned)nbat), dim3(256), 0, s,

@@ -27,7 +27,6 @@ __device__ inline double cmul(double a, double b) { return a * b; }
 __device__ inline double csub(double a, double b) { return a - b; }
 __device__ inline double cadd(double a, double b) { return a + b; }
 __device__ inline double crecip(double a) { return 1.0 / a; }
-__device__ inline double cdiv(double a, double b) { return a / b; }
 // pivot magnitude |re| + |im| (izamax / idamax)
 __device__ inline double mag1(double a) { return fabs(a); }
 template <typename T> __device__ inline auto mag1(T a) -> decltype(a.x) { return fabs(a.x) + fabs(a.y); }
@@ -44,13 +43,7 @@ template <typename T> __device__ inline void mac(T &acc, T a, T b)
   acc.y += a.x * b.y + a.y * b.x;
 }
 __device__ inline void mac(double &acc, double a, double b) { acc += a * b; }
-// acc += conj(a) b (conj = identity for real)
-template <typename T> __device__ inline void macc(T &acc, T a, T b, bool cj)
-{
-  if (cj) a.y = -a.y;
-  mac(acc, a, b);
-}
-__device__ inline void macc(double &acc, double a, double b, bool) { acc += a * b; }
+// conj(a) if cj (identity for real)
 template <typename T> __device__ inline T conj_if(T a, bool cj) { if (cj) a.y = -a.y; return a; }
 __device__ inline double conj_if(double a, bool) { return a; }
 template <typename T> __device__ inline double re_of(T a) { return a.x; }
@@ -59,15 +52,6 @@ __device__ inline double re_of(double a) { return a; }
 __device__ inline double im_of(double) { return 0; }
 template <typename T> struct IsReal { static const bool v = false; };
 template <> struct IsReal<double> { static const bool v = true; };
-
-template <typename T> __device__ inline T cdiv(T a, T b)
-{
-  typedef decltype(a.x) R;
-  T r;
-  if (fabs(b.x) >= fabs(b.y)) { R t = b.y / b.x, d = b.x + b.y * t; r.x = (a.x + a.y * t) / d; r.y = (a.y - a.x * t) / d; }
-  else { R t = b.x / b.y, d = b.x * t + b.y; r.x = (a.x * t + a.y) / d; r.y = (a.y * t - a.x) / d; }
-  return r;
-}
 
 // Strides between the instances of a batch of equal-size factorizations:
 // matrix elements (a), pivot entries (p) and bytes of each instance's
@@ -85,7 +69,7 @@ template <typename P> __device__ inline P *bshift(P *p, long bytes)
 
 struct PanelScratch {
   unsigned *bar;   // [64]: time-out word of the bounded waits
-  int *plan;       // [2*PW+1]: dst rows, src rows, count of the panel's net row permutation
+  int *plan;       // [4*PW+1]: dst rows [2*PW], src rows [2*PW], count of the panel's net row permutation
   void *linv;      // [npanels][PW][PW] T or null: inverse of each panel's unit-lower block (column-major)
   unsigned long long *ts;   // tournament-pivoting sets and root area (k_panel_ts), or null
   unsigned long long *xch;  // exchange area of k_panel_x: 2 sets of [PW][Gmax] slots, or null
