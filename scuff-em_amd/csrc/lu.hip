@@ -854,6 +854,8 @@ template <typename T> __device__ inline T readlane_t(T v, int k)
   return r;
 }
 
+__device__ inline double fma_r(double a, double b, double c) { return fma(a, b, c); }
+__device__ inline float fma_r(float a, float b, float c) { return fmaf(a, b, c); }
 // l x, and r - l x, with fused multiply-adds
 __device__ inline double fmul_t(double l, double x) { return l * x; }
 __device__ inline double2 fmul_t(double2 l, double2 x)
@@ -2005,23 +2007,23 @@ k_trsv_chain(const T *LU, long lda, long n, const T *inv, T *bin, T *xout, int m
 // Rounding: a block's 64 products are summed two k-steps at a time, a
 // sub-block's own by themselves, and subtracted once, not term by term from the
 // right-hand side.  Transposed systems (EXACT) also keep what the
-// subtractions lose (two-sums, added back before each use) and correct the
-// quotients.  Their error then is that of a dot product of 256 partial sums and
-// one division a row: 0.85 to 1.07 of it over orders 100 to 1500 and the
-// three types, where one sum over four blocks, products subtracted term by term
+// subtractions lose (two-sums, added back before each use) and multiply by
+// reciprocals in two words.  Their error then is that of a dot product of 256
+// partial sums and one division a row: 0.81 to 0.97 of it over orders 100 to 1500
+// and the three types, where one sum over four blocks, products subtracted term by term
 // and rounded reciprocals had 1.7 to 3.8 times as much.  Untransposed it is 0.4 to
 // 0.9 of what products with the blocks' inverses had (2 to 16 columns; up to
 // 1.7 before), inverses of order 64 and up at most that of substitution in
 // 256-row blocks (1.02; up to 1.28 before).  One transposed system, order 3840,
-// complex128: 1.69 -> 2.13 ms; two untransposed columns 1.43 -> 1.46 ms.
+// complex128: 1.69 -> 1.96 ms; two untransposed columns 1.43 -> 1.46 ms.
 // bin: column-major right-hand sides, row r taken from pin[r] if given, or
 // null: packed in win.  bout: column-major results or null, row r to pout[r]
 // if given.  cj: 1 conjugates the right-hand sides, 2 the results in bout.
 // Bound: the chain of block steps up to a few hundred columns (a round trip,
 // 16 complex 16x16x4 products and 64 substitution steps per wave), the
-// matrix units past that.  N=3840 complex128: 12 us a step (17 transposed);
+// matrix units past that.  N=3840 complex128: 12 us a step (16 transposed);
 // 181 columns 2.1 ms, where substitution in 256-row blocks by one workgroup a
-// column and GEMM updates took 6.0; one transposed system 2.1 ms, where a single
+// column and GEMM updates took 6.0; one transposed system 2.0 ms, where a single
 // workgroup with a reduction per row took 24.
 template <typename T> struct ChainArgs {
   const T *A; long lda; long n;
@@ -2055,13 +2057,27 @@ template <typename T> __device__ inline void sub2(T &h, T &l, T v)
   two_diff(h.x, l.x, v.x);
   two_diff(h.y, l.y, v.y);
 }
-__device__ inline bool is_finite(double v) { return isfinite(v); }
-template <typename T> __device__ inline bool is_finite(T v) { return isfinite(v.x) && isfinite(v.y); }
-// v / d from d's reciprocal, corrected by the residual where that is finite
-template <typename T> __device__ inline T quot(T v, T d, T rd)
+// a reciprocal rh of d and what it lacks: 1 / d = rh + rl to twice the
+// precision (0 where the reciprocal is not finite)
+__device__ inline double recip_lo(double d, double rh)
 {
-  const T q = cmul(v, rd), c = cmul(fnma_t(v, d, q), rd);
-  return is_finite(c) ? cadd(q, c) : q;
+  const double rl = fma(-d, rh, 1.0) * rh;
+  return isfinite(rl) ? rl : 0.0;
+}
+template <typename T> __device__ inline T recip_lo(T d, T rh)
+{
+  const T rl = cmul(fnma_t(unit_v<T>(), d, rh), rh);
+  return isfinite(rl.x) && isfinite(rl.y) ? rl : zero_v<T>();
+}
+// v (rh + rl)
+__device__ inline double mul2(double v, double rh, double rl) { return fma(v, rh, v * rl); }
+template <typename T> __device__ inline T mul2(T v, T rh, T rl)
+{
+  const T t = fmul_t(v, rl);
+  T q;
+  q.x = fma_r(v.x, rh.x, fma_r(-v.y, rh.y, t.x));
+  q.y = fma_r(v.x, rh.y, fma_r(v.y, rh.x, t.y));
+  return q;
 }
 // v of lane k of this lane's row of 16
 template <int K> __device__ inline float row_bcast(float v)
@@ -2096,7 +2112,8 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
   constexpr bool UNIT = FWD != TRANS, EXACT = TRANS;
   __shared__ T sb[TB][NC + 1];                     // right-hand sides, then solutions
   __shared__ T sl[EXACT ? TB : 1][NC + 1];         // what their roundings lost
-  __shared__ T sm[16][17], sd[TB], sr[TB];         // first diagonal sub-block; the diagonal and its reciprocals
+  __shared__ T sm[16][17], sr[TB];                 // first diagonal sub-block; the diagonal's reciprocals
+  __shared__ T srl[EXACT ? TB : 1];                // what the reciprocals lack
   __shared__ unsigned s_tk;
   const int t = threadIdx.x, lane = t & 63, i = lane & 15, kq = lane >> 4, w0 = (t >> 6) * 16;
   if (t == 0) s_tk = __hip_atomic_fetch_add(p.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2146,9 +2163,9 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
     const int s = t >> 4;
     sm[s][i] = at(sub(0) + i, sub(0) + (FWD ? s : 15 - s));
     if (!UNIT && t < TB) {
-      const T d = at(t, t);
-      sd[t] = d;
-      sr[t] = t < bs ? crecip(d) : unit_v<T>();
+      const T d = at(t, t), rd = t < bs ? crecip(d) : unit_v<T>();
+      sr[t] = rd;
+      if (EXACT) srl[EXACT ? t : 0] = t < bs ? recip_lo(d, rd) : zero_v<T>();
     }
   }
   // b: the right-hand side less the products so far; bl (EXACT): the sum of
@@ -2224,10 +2241,10 @@ __global__ void __launch_bounds__(256, 2) k_trsm_chain(ChainArgs<T> p)
     const int row = sub(u) + i;
     // y + yl: what is left (EXACT: yl as bl, else the products' own sum)
     T y = sb[row][c4 + kq], yl = EXACT ? sl[EXACT ? row : 0][c4 + kq] : zero_v<T>();
-    const T dd = UNIT ? unit_v<T>() : sd[row], rd = UNIT ? unit_v<T>() : sr[row];
+    const T rd = UNIT ? unit_v<T>() : sr[row], rl = UNIT || !EXACT ? zero_v<T>() : srl[EXACT ? row : 0];
     auto value = [&]() __attribute__((always_inline)) {
       const T z = cadd(y, yl);
-      return UNIT ? z : EXACT ? quot(z, dd, rd) : cmul(z, rd);
+      return UNIT ? z : EXACT ? mul2(z, rd, rl) : cmul(z, rd);
     };
     static_for<0, 15>([&](auto sc) __attribute__((always_inline)) {
       constexpr int s = decltype(sc)::value, k = FWD ? s : 15 - s;
