@@ -174,7 +174,7 @@ k_grad_stamp(int nEa, const int *EIa, const double *ELa, const double *Va, const
 // and the sums over y for one x need sum {1, y, y y} Psi only (ten words).
 // One thread per (row panel, slot) writes the 9 x 3 values of each region; the
 // band's column edges are then combined from them, as the matrix is.  Bound:
-// FP64 vector rate.  Two N=1920 spheres: under 0.9 ms, where each edge pair
+// FP64 vector issue at one wave a SIMD (50 % of the cycles, 16 TFLOP/s).  Two N=1920 spheres: under 0.9 ms, where each edge pair
 // integrated its four panel pairs by itself in 8.7.
 __global__ void __launch_bounds__(128)
 k_grad_pair(const double *Va, const int *PVIa, const double *PCa, int nPa, const double *Vb, const int *PVIb,

@@ -169,7 +169,8 @@ __device__ inline double cc_node(int e)
 // first TD_NPRE nodes, one per lane (orders 0 .. 4), come before the first
 // test, order 5's last one if it is asked for; their sums are taken from LDS,
 // a lane per order and value.  Later orders, if any, keep their nodes in a
-// scratch slab.  Bound: FP64 vector rate of the kernel values.  Bodies of
+// scratch slab.  Bound: latency of a job's kernel values and sums (0.3 to 1.1
+// waves a SIMD; 7 to 30 % of the cycles issue vector instructions).  Bodies of
 // N=7155: 0.61 ms an assembly, where a wave for each (Qa, Qb), with the
 // exponentials of every power and polynomial its own, took 2.9
 __global__ void __launch_bounds__(64)

@@ -41,7 +41,7 @@ int lu_factor(T *A, long n, long lda, int *d_ipiv, int *info, hipStream_t stream
 // permutation (n ints) and the one-launch solve's words (2 nblk + 8).
 // refined (complex64): the caller corrects the solution by residuals in
 // higher precision, so that products with the diagonal blocks' inverses do;
-// otherwise they are substituted through and invL, invU are not used.
+// otherwise they are substituted through and there are no invL, invU.
 // inv_ready: invL / invU and perm already hold the inverses and the
 // composed row permutation for these factors (set by the first solve;
 // clear it for new factors).
@@ -54,10 +54,10 @@ struct SolveWs {
 };
 // bytes of the buffers above for n rows, each part rounded to 256 bytes
 template <typename T>
-size_t solve_ws_bytes(long n);
-// carves the buffers from `base` (solve_ws_bytes(n) bytes)
+size_t solve_ws_bytes(long n, bool refined);
+// carves the buffers from `base` (solve_ws_bytes(n, refined) bytes)
 template <typename T>
-SolveWs<T> solve_ws_carve(char *base, long n);
+SolveWs<T> solve_ws_carve(char *base, long n, bool refined);
 
 // solves op(A) X = B with the factors of lu_factor; trans 'N', 'T', 'C'.
 // With ws (trans 'N', nrhs 1 only) it allocates nothing.

@@ -2380,23 +2380,26 @@ static int trsm_chain(const T *LU, long lda, long n, const int *ipiv, bool tr, b
 }
 
 template <typename T>
-size_t solve_ws_bytes(long n)
+size_t solve_ws_bytes(long n, bool refined)
 {
   auto r256 = [](size_t b) { return 256 * ((b + 255) / 256); };
   const long nblk = (n + TB - 1) / TB;
-  return r256(sizeof(T) * n) + 2 * r256(sizeof(T) * nblk * TB * TB) + r256(sizeof(int) * n) +
+  return r256(sizeof(T) * n) + (refined ? 2 * r256(sizeof(T) * nblk * TB * TB) : 0) + r256(sizeof(int) * n) +
          r256(sizeof(unsigned long long) * (2 * nblk + 8));
 }
 
 template <typename T>
-SolveWs<T> solve_ws_carve(char *base, long n)
+SolveWs<T> solve_ws_carve(char *base, long n, bool refined)
 {
   auto r256 = [](size_t b) { return 256 * ((b + 255) / 256); };
   const long nblk = (n + TB - 1) / TB;
   SolveWs<T> w;
   w.W = (T *)base; base += r256(sizeof(T) * n);
-  w.invL = (T *)base; base += r256(sizeof(T) * nblk * TB * TB);
-  w.invU = (T *)base; base += r256(sizeof(T) * nblk * TB * TB);
+  w.refined = refined;
+  if (refined) {
+    w.invL = (T *)base; base += r256(sizeof(T) * nblk * TB * TB);
+    w.invU = (T *)base; base += r256(sizeof(T) * nblk * TB * TB);
+  }
   w.perm = (int *)base; base += r256(sizeof(int) * n);
   w.chain = (unsigned long long *)base;
   return w;
@@ -2505,22 +2508,20 @@ template int lu_solve<double2>(const double2 *, long, long, const int *, char, l
                                SolveWs<double2> *);
 template int lu_solve<float2>(const float2 *, long, long, const int *, char, long, float2 *, long, hipStream_t,
                               SolveWs<float2> *);
-template size_t solve_ws_bytes<double2>(long);
-template size_t solve_ws_bytes<float2>(long);
-template SolveWs<double2> solve_ws_carve<double2>(char *, long);
-template SolveWs<float2> solve_ws_carve<float2>(char *, long);
+template size_t solve_ws_bytes<double2>(long, bool);
+template size_t solve_ws_bytes<float2>(long, bool);
+template SolveWs<double2> solve_ws_carve<double2>(char *, long, bool);
+template SolveWs<float2> solve_ws_carve<float2>(char *, long, bool);
 
 // ---------------------------------------------------------------------
 // one-right-hand-side solve that allocates nothing: the buffers of a
-// SolveWs (W, inverses of the 64x64 diagonal blocks of L and U, composed
-// permutation, one-launch words) are carved from a fixed device array,
-// one copy per GPU, held until the process ends.  Every call on a GPU
+// SolveWs (W, composed permutation, one-launch words) are carved from a
+// fixed device array, one copy per GPU, held until the process ends.  Every call on a GPU
 // shares that GPU's array, so calls that overlap on one GPU race.
 // ---------------------------------------------------------------------
 constexpr long r256_const(long b) { return 256 * ((b + 255) / 256); }
 constexpr long NOALLOC_NBLK = (NOALLOC_MAX_N + TB - 1) / TB;
 constexpr long NOALLOC_BYTES = r256_const((long)sizeof(double2) * NOALLOC_MAX_N) +
-                               2 * r256_const((long)sizeof(double2) * NOALLOC_NBLK * TB * TB) +
                                r256_const((long)sizeof(int) * NOALLOC_MAX_N) +
                                r256_const((long)sizeof(unsigned long long) * (2 * NOALLOC_NBLK + 8));
 static __device__ __align__(256) unsigned char scratch[NOALLOC_BYTES];
@@ -2549,11 +2550,11 @@ template <typename T>
 int lu_solve_noalloc(const T *LU, long n, long lda, const int *d_ipiv, T *B, hipStream_t stream)
 {
   if (n < 0 || lda < std::max(1L, n)) return -1;
-  if (n > NOALLOC_MAX_N || (long)solve_ws_bytes<T>(n) > NOALLOC_BYTES) return -7;
+  if (n > NOALLOC_MAX_N || (long)solve_ws_bytes<T>(n, false) > NOALLOC_BYTES) return -7;
   if (n == 0) return 0;
   char *base = (char *)noalloc_scratch_ptr();
   if (!base) return -3;
-  SolveWs<T> w = solve_ws_carve<T>(base, n);
+  SolveWs<T> w = solve_ws_carve<T>(base, n, false);
   w.inv_ready = false;   // the array holds whatever the last call left
   return lu_solve<T>(LU, n, lda, d_ipiv, 'N', 1, B, std::max(1L, n), stream, &w);
 }

@@ -30,7 +30,7 @@ size_t refine_ws_bytes(long n, int m)
 {
   return 3 * r256(sizeof(double2) * n) + r256(sizeof(double2) * n * residual_chunks(n)) +
          r256(sizeof(float2) * n) + 256 + r256(sizeof(double2) * REFINE_PARTS * (REFINE_GMRES_MAX + 1)) +
-         r256(sizeof(double2) * n * (2 * (long)m + 1)) + solve_ws_bytes<float2>(n);
+         r256(sizeof(double2) * n * (2 * (long)m + 1)) + solve_ws_bytes<float2>(n, true);
 }
 
 RefineWs refine_ws_carve(char *base, long n, int m)
@@ -46,8 +46,7 @@ RefineWs refine_ws_carve(char *base, long n, int m)
   w.part = (double2 *)base; base += r256(sizeof(double2) * REFINE_PARTS * (REFINE_GMRES_MAX + 1));
   w.V = (double2 *)base; base += r256(sizeof(double2) * n * ((long)m + 1));
   w.Z = (double2 *)base; base += r256(sizeof(double2) * n * (long)m);
-  w.sws = solve_ws_carve<float2>(base, n);
-  w.sws.refined = true;
+  w.sws = solve_ws_carve<float2>(base, n, true);
   return w;
 }
 
